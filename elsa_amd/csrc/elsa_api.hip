@@ -97,21 +97,32 @@ int plan_fwd(const elsa_fwd_args* a, elsa_fwd_plan* pl) {
     // 3% from 1 to 8 partitions
     int64_t p = cdiv(1024, q_tiles);
     p = std::min<int64_t>(p, std::max<int64_t>(1, n / 512));
-    // fp32: its fold spends 16 times longer per key than fp16's, so short partitions cost little
-    // and the grid's fill decides: where the rule above leaves fewer than 256 work-groups,
-    // partitions down to 64 keys until about 512.  Forward ms (Phase 1 + Phase 2, d64): B1 H8 1K
-    // 0.050 -> 0.029 (2 -> 8 partitions), causal 1K 0.051 -> 0.029, B8 H3 N197 0.024 -> 0.015 (1 ->
-    // 3), B1 H8 N512 0.047 -> 0.014 (1 -> 8); B8 H3 N1025 (432 work-groups) keeps 2 partitions
-    // (0.086 against 0.089 ms with 3).  The count is capped at ceil(n / 64), not floor(n / 64): a
-    // short tail partition costs less than a third 32-key stage in every work-group: B8 H3 N197
-    // 0.0154 -> 0.0127 ms (3 -> 4 partitions), B2 H3 N300 0.0149 -> 0.0131, B1 H2 N90 0.0124 ->
-    // 0.0112 (1 -> 2)
-    // Causal grids, whose work-groups above the diagonal return at once, fill below 512 work-groups
-    // too: B2 H8 N1024 causal 0.0515 -> 0.0380 ms (2 -> 4 partitions), B8 H3 N1025 causal 0.0656 ->
-    // 0.0644 (2 -> 3); non-causal ones there went both ways (B2 H8 N1024 0.051 -> 0.047, B8 H3 N1025
-    // 0.0856 -> 0.0890, B3 H8 N1024 0.083 -> 0.086) and keep the 256 bound.
-    if (a->dtype == ELSA_F32 && q_tiles * p < (a->is_causal ? 512 : 256))
-      p = std::max<int64_t>(p, std::min<int64_t>(cdiv(512, q_tiles), cdiv(n, 64)));
+    if (a->dtype == ELSA_F32) {
+      // fp32 from 1024 keys without a causal mask, where the 1024 work-group target leaves the last round of
+      // the chip mostly empty: rounds x (partition keys + 130) over 256-row work-groups, one per CU (the
+      // 8-wave fold), 130 keys for a work-group's fixed cost; the count with the least, if 7% below the
+      // target's.  Forward ms (Phase 1 + Phase 2, d64): B2 H8 N4097 0.499 -> 0.438 (2 -> 5 partitions), B2 H8
+      // 2K 0.105 -> 0.101 (4 -> 2); B1 H8 4K (0.190 against 0.186 with 2) and B8 H3 N1025 keep 4 and 2
+      if (!a->is_causal && n >= 1024) {
+        const int64_t tiles = bh * cdiv(q_rows, 256);
+        auto cost = [&](int64_t c) {
+          const int64_t len = cdiv(cdiv(n, c), kt) * kt;
+          return cdiv(tiles * cdiv(n, len), 256) * (len + 130);
+        };
+        int64_t best = p;
+        for (int64_t c = 1; c <= std::max<int64_t>(1, n / 512); ++c)
+          if (cost(c) < cost(best)) best = c;
+        if (cost(best) * 100 < cost(p) * 93) p = best;
+      }
+      // Where fewer than 256 128-row work-groups are left, partitions down to 64 keys until about 512.
+      // Forward ms, d64: B1 H8 1K 0.0463 -> 0.0286 (2 -> 8 partitions; 4: 0.0258), B1 H8 N512 0.0416 -> 0.0162
+      // (1 -> 8), B8 H3 N197 0.0170 -> 0.0131 (1 -> 4), d128 B1 H4 N1025 0.0788 -> 0.0364 (2 -> 11).  The count is
+      // capped at ceil(n / 64), not floor(n / 64): a short tail partition costs less than another 32-key
+      // stage in every work-group.  Causal grids, whose work-groups above the diagonal return at once, fill
+      // below 512 too: B2 H8 N1024 causal 0.0473 -> 0.0294 ms (2 -> 4), B1 H8 1K causal 0.0451 -> 0.0249 (2 -> 8).
+      if (q_tiles * p < (a->is_causal ? 512 : 256))
+        p = std::max<int64_t>(p, std::min<int64_t>(cdiv(512, q_tiles), cdiv(n, 64)));
+    }
     // fp16/bf16 grids at d <= 64 from 512 keys under 192 work-groups (a few heads of at most 2K rows):
     // partitions down to 128 keys until about 256 work-groups.  Forward ms (fp16 d64): B1 H8 1K 0.012
     // -> 0.010 (2 -> 4 partitions), N512 0.0099 -> 0.0084 (1 -> 4), causal N1025 0.0139 -> 0.0121
@@ -424,13 +435,9 @@ elsa::BwdParams bwd_params(const elsa_bwd_args* a) {
   p.lse_lo = reinterpret_cast<float*>(base + 2 * align256(rows * 4));
   p.dp = elsa::pad_head_dim(a->head_dim);
   p.split = elsa::bwd_splits(a->dtype, p.dp, p.BH, p.N, a->bias.ptr != nullptr, a->is_causal != 0);
-  // rows (dK/dV) or keys (dq) per range: whole stages, 64 rows in the fp16/bf16 kernels and 32 in the
-  // fp32 ones (against 64 for fp32: B1 H8 N1025 causal backward 0.161 -> 0.143 ms with 8 ranges of 160
-  // keys instead of 192, B2 H3 N300 0.063 -> 0.054, B8 H3 N1025 0.335 -> 0.320)
-  {
-    const int64_t st = a->dtype == ELSA_F32 ? 32 : 64;
-    p.split_len = p.split > 1 ? (int)((((int64_t)p.N + p.split - 1) / p.split + st - 1) / st * st) : p.N;
-  }
+  // 16-bit kernels: rows (dK/dV) or keys (dq) per range, whole 64-row stages; the fp32 ones deal their
+  // stages out in turn and every range holds a partial (split_len 1 makes the combine read them all)
+  p.split_len = a->dtype == ELSA_F32 ? 1 : p.split > 1 ? (int)((((int64_t)p.N + p.split - 1) / p.split + 63) / 64 * 64) : p.N;
   p.part = p.split > 1 ? reinterpret_cast<float*>(base + 3 * align256(rows * 4)) : nullptr;
   p.part_stride = (int64_t)(align256((size_t)p.split * rows * p.dp * 4) / 4);
   const int H = a->heads, N = a->seq_len, D = a->head_dim;
@@ -683,8 +690,21 @@ int elsa_bwd_dbias(const elsa_bwd_args* a, float* dbias, int32_t bias_batch, int
   float* ds = direct ? dbias
                      : reinterpret_cast<float*>(static_cast<char*>(a->workspace) + elsa_bwd_workspace_bytes(a));
   hipError_t e = hipSuccess;
+  const bool is_short = elsa::bwd_short_takes(a->dtype, a->seq_len, elsa::pad_head_dim(a->head_dim));
+  if (is_short && !direct && bias_batch == 1 && bias_heads == a->heads) {
+    // dS summed over the batch inside the backward, one partial per range of it (at most batch: they fit the
+    // dS buffer), then over the ranges
+    elsa::BwdParams p = bwd_params(a);
+    const int groups = elsa::bwd_short_groups(a->batch, a->heads);
+    p.ds_out = groups > 1 ? ds : dbias;
+    if ((e = elsa::launch_bwd_short(p, a->dtype, 2, st)) != hipSuccess) return hip_fail(e, "backward launch");
+    if (groups == 1) return ELSA_OK;
+    const int64_t n = (int64_t)a->heads * a->seq_len * a->seq_len;
+    if ((e = elsa::launch_dbias_reduce(ds, dbias, groups, n, st)) != hipSuccess) return hip_fail(e, "dbias sum launch");
+    return ELSA_OK;
+  }
   // causal dk/dv workgroups skip the stages above their keys: those dS entries stay zero
-  if (a->is_causal && (e = elsa::launch_zero_fill(ds, (int64_t)(ds_bytes(a) / sizeof(float)), st)) != hipSuccess)
+  if (a->is_causal && !is_short && (e = elsa::launch_zero_fill(ds, (int64_t)(ds_bytes(a) / sizeof(float)), st)) != hipSuccess)
     return hip_fail(e, "zero fill");
   elsa::BwdParams p = bwd_params(a);
   p.ds_out = ds;

@@ -1,4 +1,5 @@
-// ELSA backward on gfx950: exact recompute of p from the saved base-2 row state.
+// ELSA backward on gfx950: exact recompute of p from the saved base-2 row state.  The dq and dk/dv kernels
+// here are the fp16 / bf16 ones (fp32: elsa_bwd_f32.hip; at most 64 rows: elsa_bwd_short.hip).
 //
 //   preprocess  D = rowsum(O * dO), LSE2 = m + log2(max(z, 1e-30))   (attention_bwd.py:188-224)
 //   dq kernel   per 32-row wave tile, loop over 32-key tiles:         (attention_bwd.py:309-412)
@@ -14,8 +15,7 @@
 // S^T / S directly usable as the B operand of the following MFMA.
 #include <algorithm>
 
-#include "elsa_internal.h"
-#include "elsa_mfma.h"
+#include "elsa_bwd_common.h"
 
 namespace elsa {
 
@@ -34,13 +34,6 @@ struct BwdCfg {
   static constexpr int NJ = 16 / KP;
   static constexpr int CE = 16 / (int)sizeof(T);
 };
-
-__device__ inline float load_bias_b(const BiasView& b, int bi, int hi, int row, int key) {
-  const int64_t off = (int64_t)bi * b.sb + (int64_t)hi * b.sh + (int64_t)row * b.sq + (int64_t)key * b.sk;
-  if (b.dtype == ELSA_F32) return static_cast<const float*>(b.ptr)[off];
-  if (b.dtype == ELSA_F16) return static_cast<float>(static_cast<const f16*>(b.ptr)[off]);
-  return static_cast<float>(static_cast<const bf16*>(b.ptr)[off]);
-}
 
 // Copy rows [row0, row0+TT) x [0, DP) of an [N, D] matrix with row stride rs (elements)
 // into LDS, row-major (stride RS) and/or transposed (stride TS); rows >= row_end and
@@ -85,68 +78,7 @@ __device__ inline typename Mfma<T>::frag a_frag(const T* rm, const T* tr, int c,
   }
 }
 
-// fp32 stage staging, double-buffered: each thread first loads its 16-byte chunks of the
-// next TT rows into registers (f32_stage_load, issued before the current stage's MFMAs),
-// then writes them into the other LDS buffer (f32_stage_store2).  Rows >= row_end and
-// d >= D read as zeros.
-template <int DP, int NT>
-struct F32Stage {
-  static constexpr int CPR = DP / 4;              // 16-byte chunks per row
-  static constexpr int TOTAL = BwdCfg<float, DP>::TT * CPR;
-  static constexpr int NCH = (TOTAL + NT - 1) / NT;  // chunks per thread
-};
-
-template <int DP, int NT, int NR>
-__device__ inline void f32_stage_load(Chunk16 (&reg)[NR], const float* __restrict__ src, int64_t rs, int row0,
-                                      int row_end, int D, int tid) {
-  using S = F32Stage<DP, NT>;
-  static_assert(NR == S::NCH, "one register chunk per staged chunk of this thread");
-  static_for<0, S::NCH>([&](auto I) {
-    constexpr int i = decltype(I)::value;
-    const int ci = tid + i * NT;
-    const int r = ci / S::CPR, d0 = (ci % S::CPR) * 4;
-    Chunk16 v{};
-    if (ci < S::TOTAL && row0 + r < row_end && d0 < D)
-      v = *reinterpret_cast<const Chunk16*>(src + (int64_t)(row0 + r) * rs + d0);
-    reg[i] = v;
-  });
-}
-
-// fp32 dk/dv staging: the register chunks written transposed (row stride TS) and row-major
-// with stride RS4 (four consecutive d of one row in one 16-byte load).
-template <int DP, int NT, int NR, int TS, int RS4>
-__device__ inline void f32_stage_store2(const Chunk16 (&reg)[NR], float* tr, float* rm, int tid) {
-  using S = F32Stage<DP, NT>;
-  static_assert(NR == S::NCH, "one register chunk per staged chunk of this thread");
-  static_for<0, S::NCH>([&](auto I) {
-    constexpr int i = decltype(I)::value;
-    const int ci = tid + i * NT;
-    if (S::TOTAL % NT == 0 || ci < S::TOTAL) {
-      const int r = ci / S::CPR, d0 = (ci % S::CPR) * 4;
-#pragma unroll
-      for (int t = 0; t < 4; ++t) tr[(d0 + t) * TS + r] = __uint_as_float(reg[i][t]);
-      *reinterpret_cast<Chunk16*>(rm + r * RS4 + d0) = reg[i];
-    }
-  });
-}
-
 // ------------------------------------------------------------------ preprocess
-// LSE2 = m + log2(max(z, 1e-30)) (attention_bwd.py:224), formed in double and split into its fp32
-// rounding hi and the remainder lo, so that the fp32 kernels' p = exp2(s*c - LSE2) does not carry
-// the half-ulp of a ~15-magnitude LSE2 (3e-7 relative, the same for a whole row) into every
-// gradient of that row.  A row with no valid key (z == 0) gets +inf instead of -inf, so that p is 0
-// without a test.
-__device__ inline void lse2_split(float m, float z, float& hi, float& lo) {
-  if (z > 0.f) {
-    const double l = (double)m + log2((double)fmaxf(z, 1.0e-30f));
-    hi = (float)l;
-    lo = (float)(l - (double)hi);
-  } else {
-    hi = __builtin_huge_valf();
-    lo = 0.f;
-  }
-}
-
 template <typename T>
 __global__ __launch_bounds__(256) void bwd_pre_kernel(const BwdParams p) {
   // grid: x = block of 32 rows, y = batch * head.  The 8 lanes of a row read its 16-byte
@@ -179,394 +111,6 @@ __global__ __launch_bounds__(256) void bwd_pre_kernel(const BwdParams p) {
   lse2_split(p.row_m[i], p.row_z[i], lhi, llo);
   p.lse_row[i] = lhi;
   p.lse_lo[i] = llo;
-}
-
-// ------------------------------------------------------------------ dq
-// fp32 only (the fp16 / bf16 kernel follows below).  The fp32 MFMA takes one operand
-// element per lane and k-step; over d the contraction order is k-step kk = 4m + u of lane
-// group g at d = 8m + 4g + u, so one 16-byte load of a row-major K or V row gives a lane
-// four k-steps.  The transposed K tile (dQ operand) keeps stride TT + 1 and 4-byte loads.
-template <typename T, int DP, int WAVES, bool HAS_BIAS>
-__global__ __launch_bounds__(64 * WAVES) void bwd_dq_kernel(const BwdParams p) {
-  static_assert(sizeof(T) == 4, "fp32 kernel");
-  using C = BwdCfg<T, DP>;
-  using M = Mfma<T>;
-  constexpr int NT = 64 * WAVES, BM = 32 * WAVES;
-  constexpr int TT = C::TT;       // keys per stage
-  constexpr int TS1 = TT + 1;     // transposed K tile [DP][TS1]: conflict-free transposing writes
-  constexpr int RS4 = DP + 4;     // row-major K and V tiles [TT][RS4]
-  constexpr int NM = DP / 8;
-  // two buffers: stage i + 1 goes from global memory into registers while stage i computes, and
-  // from there into the other buffer
-  __shared__ __attribute__((aligned(16))) float Kr[2][TT * RS4];
-  __shared__ __attribute__((aligned(16))) float Vr[2][TT * RS4];
-  __shared__ __attribute__((aligned(16))) float Kt[2][DP * TS1];
-
-  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 31,
-            g = lane >> 5;
-  WgCoord wg = xcd_order();
-  if (p.causal) wg.x = (int)gridDim.x - 1 - wg.x;  // causal: heaviest row blocks first
-  const int bh = wg.y;
-  const int wg_row0 = wg.x * BM;
-  const int wg_last = min(p.N, wg_row0 + BM) - 1;
-  const int my_row = wg_row0 + wave * 32 + c;
-  const bool row_ok = my_row < p.N;
-  const int bi = bh / p.H, hi = bh % p.H;
-  const T* Q = static_cast<const T*>(p.q) + bi * p.qs[0] + hi * p.qs[1];
-  const T* K = static_cast<const T*>(p.k) + bi * p.ks[0] + hi * p.ks[1];
-  const T* V = static_cast<const T*>(p.v) + bi * p.vs[0] + hi * p.vs[1];
-  const T* dO = static_cast<const T*>(p.dout) + bi * p.gs[0] + hi * p.gs[1];
-
-  // this lane's row of Q and dO at d = 8m + 4g .. + 3 (the B operands of S and dP)
-  f32x4 qf[NM], gf[NM];
-  const int rsafe = row_ok ? my_row : 0;
-#pragma unroll
-  for (int m = 0; m < NM; ++m) {
-    const int d0 = 8 * m + 4 * g;
-    const bool ok = row_ok && d0 < p.D;
-    qf[m] = ok ? *reinterpret_cast<const f32x4*>(Q + (int64_t)rsafe * p.qs[2] + d0) : f32x4{};
-    gf[m] = ok ? *reinterpret_cast<const f32x4*>(dO + (int64_t)rsafe * p.gs[2] + d0) : f32x4{};
-  }
-  float lse, lse_lo, dd;
-  const int64_t ri = (int64_t)bh * p.N + rsafe;
-  if constexpr (DP <= 64) {
-    // the preprocess of these rows, in bwd_pre_kernel's order: that kernel's lane j of a row chains
-    // fmas over the 4-float chunks j, j + 8, ... below D, and the 8 lanes' sums add pairwise,
-    // ((a0 + a1) + (a2 + a3)) + ((a4 + a5) + (a6 + a7)).  Here chunk 2m + g is this lane's m-th
-    // load, so lane group g forms a_{2i+g} over m = i, i + 4, and lanes c and c + 32 add the pairs.
-    // The work-groups of the first key range store D and LSE2 for the dK/dV kernel, so a whole
-    // backward launches no preprocess.
-    const T* O = static_cast<const T*>(p.out) + bi * p.os[0] + hi * p.os[1] + (int64_t)rsafe * p.os[2];
-    float pair[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      float a = 0.f;
-#pragma unroll
-      for (int m = i; m < NM; m += 4) {
-        const int d0 = 8 * m + 4 * g;
-        if (d0 < p.D) {
-          const f32x4 o4 = row_ok ? *reinterpret_cast<const f32x4*>(O + d0) : f32x4{};
-#pragma unroll
-          for (int t = 0; t < 4; ++t) a = fmaf(o4[t], gf[m][t], a);
-        }
-      }
-      pair[i] = a + __shfl_xor(a, 32);
-    }
-    const float dsum = (pair[0] + pair[1]) + (pair[2] + pair[3]);
-    float lhi, llo;
-    lse2_split(p.row_m[ri], p.row_z[ri], lhi, llo);
-    if (row_ok && g == 0 && wg.z == 0) {
-      p.d_row[ri] = dsum;
-      p.lse_row[ri] = lhi;
-      p.lse_lo[ri] = llo;
-    }
-    lse = row_ok ? lhi : 0.f;
-    lse_lo = row_ok ? llo : 0.f;
-    dd = row_ok ? dsum : 0.f;
-  } else {
-    lse = row_ok ? p.lse_row[ri] : 0.f;
-    lse_lo = row_ok ? p.lse_lo[ri] : 0.f;
-    dd = row_ok ? p.d_row[ri] : 0.f;
-  }
-  const bool live = row_ok && lse > kNegInf;
-
-  f32x16 acc[C::NDT];
-#pragma unroll
-  for (int dt = 0; dt < C::NDT; ++dt) acc[dt] = f32x16{};
-  const int k_end = p.causal ? wg_last + 1 : p.N;
-  // split (bwd_splits; 1 range of N keys otherwise): this work-group's keys [k_lo, k_hi) over grid z,
-  // whole 32-key stages, so a stage never straddles a range end short of k_end.  An empty range
-  // writes no partial, and the combine (kind 0 past N, kind 1 past a causal row block) skips it.
-  const int k_lo = min(k_end, (int)wg.z * p.split_len), k_hi = min(k_end, k_lo + p.split_len);
-  if (p.split > 1 && k_lo >= k_hi) return;
-  constexpr int CPR = DP / 4;  // 16-byte chunks per key row
-  constexpr int NCH = TT * CPR / NT;
-  static_assert((TT * CPR) % NT == 0, "staging must divide evenly");
-  // chunk tid + i NT of a stage: key row ci / CPR, head dims (ci % CPR) * 4 .. + 3; keys >= k_hi
-  // and d >= D are zeros
-  f32x4 kreg[NCH], vreg[NCH];
-  auto gload = [&](int t0) {
-#pragma unroll
-    for (int i = 0; i < NCH; ++i) {
-      const int ci = tid + i * NT;
-      const int r = ci / CPR, d0 = (ci % CPR) * 4, key = t0 + r;
-      const bool ok = key < k_hi && d0 < p.D;
-      kreg[i] = ok ? *reinterpret_cast<const f32x4*>(K + (int64_t)key * p.ks[2] + d0) : f32x4{};
-      vreg[i] = ok ? *reinterpret_cast<const f32x4*>(V + (int64_t)key * p.vs[2] + d0) : f32x4{};
-    }
-  };
-  auto sstore = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < NCH; ++i) {
-      const int ci = tid + i * NT;
-      const int r = ci / CPR, d0 = (ci % CPR) * 4;
-      *reinterpret_cast<f32x4*>(&Kr[buf][r * RS4 + d0]) = kreg[i];
-      *reinterpret_cast<f32x4*>(&Vr[buf][r * RS4 + d0]) = vreg[i];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) Kt[buf][(d0 + u) * TS1 + r] = kreg[i][u];
-    }
-  };
-  if (k_lo < k_hi) {
-    gload(k_lo);
-    sstore(0);
-  }
-  __syncthreads();
-
-  for (int t0 = k_lo, buf = 0; t0 < k_hi; t0 += TT, buf ^= 1) {
-    // buffer buf ^ 1 was last read by the previous stage, before the barrier that ended it
-    const bool has_next = t0 + TT < k_hi;
-    if (has_next) gload(t0 + TT);
-    f32x16 s = f32x16{}, dp = f32x16{};
-    {
-      // A operands: stage key swap23(c), d = 8m + 4g .. + 3
-      const float* kr = Kr[buf] + swap23(c) * RS4 + 4 * g;
-      const float* vr = Vr[buf] + swap23(c) * RS4 + 4 * g;
-#pragma unroll
-      for (int m = 0; m < NM; ++m) {
-        const f32x4 ka = *reinterpret_cast<const f32x4*>(kr + 8 * m);
-        const f32x4 va = *reinterpret_cast<const f32x4*>(vr + 8 * m);
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          s = M::mma(ka[u], qf[m][u], s);
-          dp = M::mma(va[u], gf[m][u], dp);
-        }
-      }
-    }
-    const bool full = !HAS_BIAS && (t0 + TT <= k_hi) && (!p.causal || t0 + TT - 1 <= wg_row0 + wave * 32);
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int key = t0 + key_of_reg(r, g);
-      bool ok = live;
-      if (!full) ok = ok && key < k_hi && (!p.causal || key <= my_row);
-      // s*c - LSE2 with one rounding of the (small) difference, then LSE2's low part
-      float x = fmaf(s[r], p.scale_log2, -lse) - lse_lo;
-      if constexpr (HAS_BIAS) x = ok ? fmaf(load_bias_b(p.bias, bi, hi, my_row, key), kLog2e, x) : x;
-      const float pr = ok ? fast_exp2(x) : 0.f;
-      s[r] = pr * (dp[r] - dd);
-    }
-    // this stage's 32 keys into a fresh accumulator, then one add into the running sum: each
-    // dq element is a chain of N/32 adds plus 16 MFMA steps, not N/2 MFMA steps (B8 H3 N1025:
-    // 1.06e-6 from the exact dq against the 1e-6 bar, sequential over 513 steps)
-    f32x16 st[C::NDT];
-#pragma unroll
-    for (int dt = 0; dt < C::NDT; ++dt) st[dt] = f32x16{};
-#pragma unroll
-    for (int jb = 0; jb < 4; ++jb) {
-      const int k0 = 16 * (jb >> 1) + 8 * g + 4 * (jb & 1);  // key_of_reg(4 jb, g)
-#pragma unroll
-      for (int dt = 0; dt < C::NDT; ++dt) {
-        const float* ka = Kt[buf] + (dt * 32 + c) * TS1 + k0;
-#pragma unroll
-        for (int u = 0; u < 4; ++u) st[dt] = M::mma(ka[u], s[4 * jb + u], st[dt]);
-      }
-    }
-#pragma unroll
-    for (int dt = 0; dt < C::NDT; ++dt) acc[dt] += st[dt];
-    if (has_next) sstore(buf ^ 1);
-    __syncthreads();
-  }
-  if (!row_ok) return;
-  if (p.split > 1) {  // this key range's unscaled dQ: the combine sums the ranges and scales
-    float* dst = p.part + (((int64_t)wg.z * p.BH + bh) * p.N + my_row) * p.dp;
-#pragma unroll
-    for (int dt = 0; dt < C::NDT; ++dt)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) dst[dt * 32 + drow(r, g)] = acc[dt][r];
-    return;
-  }
-  T* out = static_cast<T*>(p.dq) + bi * p.dqs[0] + hi * p.dqs[1] + (int64_t)my_row * p.dqs[2];
-#pragma unroll
-  for (int dt = 0; dt < C::NDT; ++dt)
-#pragma unroll
-    for (int q4 = 0; q4 < 4; ++q4) {  // 16-byte stores, as in bwd_dkdv_kernel
-      const int d = dt * 32 + drow(4 * q4, g);
-      if (d < p.D)
-        *reinterpret_cast<f32x4*>(out + d) = f32x4{acc[dt][4 * q4] * p.scale, acc[dt][4 * q4 + 1] * p.scale,
-                                                   acc[dt][4 * q4 + 2] * p.scale, acc[dt][4 * q4 + 3] * p.scale};
-    }
-}
-
-// ------------------------------------------------------------------ dk / dv
-// fp32 only (the fp16 / bf16 kernels follow below).
-// 2 waves per SIMD up to D = 64 (243 VGPRs, no AGPRs, no spills).  With one 16-byte LDS load
-// per four k-steps the waves keep their operand reads ahead of the MFMAs (B1 H8 d64: 16K
-// 10.92 -> 9.23 ms, 4K 0.764 -> 0.703 ms against one 4-byte load per k-step).
-template <typename T, int DP, int WAVES, bool HAS_BIAS>
-__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(DP >= 128 ? 1 : 2, 2)))
-void bwd_dkdv_kernel(const BwdParams p) {
-  static_assert(sizeof(T) == 4, "fp32 kernel");
-  using C = BwdCfg<T, DP>;
-  using M = Mfma<T>;
-  constexpr int NT = 64 * WAVES, BN = 32 * WAVES;
-  constexpr int TT = C::TT;       // stage rows
-  constexpr int TS1 = TT + 1;     // transposed tiles [DP][TS1]: conflict-free transposing writes
-  constexpr int RS4 = DP + 4;     // row-major tiles [TT][RS4]
-  constexpr int NM = DP / 8;      // 16-byte operand loads per lane over the head dim
-  // The fp32 MFMA takes one operand element per lane and k-step, and the contraction order
-  // is free: over d, k-step kk = 4m + u of lane group g takes d = 8m + 4g + u, so one
-  // 16-byte load of a row-major Q or dO row gives a lane four k-steps.  The transposed tiles
-  // (dK / dV operands) keep stride TT + 1 and 4-byte loads: at a 16-byte aligned stride
-  // their transposing writes conflicted 4-way (16K 9.20 against 9.01 ms).
-  __shared__ __attribute__((aligned(16))) float Qt[2][DP * TS1];
-  __shared__ __attribute__((aligned(16))) float Gt[2][DP * TS1];
-  __shared__ __attribute__((aligned(16))) float Qr[2][TT * RS4];
-  __shared__ __attribute__((aligned(16))) float Gr[2][TT * RS4];
-  __shared__ float lse_s[2][TT], lo_s[2][TT], dd_s[2][TT];
-
-  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 31,
-            g = lane >> 5;
-  // causal: the work of a key block shrinks with its index (heaviest first; paired heavy with
-  // light where the grid fits in one round)
-  const WgCoord wg = (p.causal && WAVES == 4) ? xcd_order_paired() : xcd_order();
-  const int bh = wg.y;
-  const int wg_key0 = wg.x * BN;
-  const int key0 = wg_key0 + wave * 32;
-  const int my_key = key0 + c;
-  const bool key_ok = my_key < p.N;
-  const int bi = bh / p.H, hi = bh % p.H;
-  const T* Q = static_cast<const T*>(p.q) + bi * p.qs[0] + hi * p.qs[1];
-  const T* K = static_cast<const T*>(p.k) + bi * p.ks[0] + hi * p.ks[1];
-  const T* V = static_cast<const T*>(p.v) + bi * p.vs[0] + hi * p.vs[1];
-  const T* dO = static_cast<const T*>(p.dout) + bi * p.gs[0] + hi * p.gs[1];
-
-  // this lane's key row of K and V at d = 8m + 4g .. + 3 (the B operands of S and dP)
-  f32x4 kf[NM], vf[NM];
-  const int ksafe = key_ok ? my_key : 0;
-#pragma unroll
-  for (int m = 0; m < NM; ++m) {
-    const int d0 = 8 * m + 4 * g;
-    const bool ok = key_ok && d0 < p.D;
-    kf[m] = ok ? *reinterpret_cast<const f32x4*>(K + (int64_t)ksafe * p.ks[2] + d0) : f32x4{};
-    vf[m] = ok ? *reinterpret_cast<const f32x4*>(V + (int64_t)ksafe * p.vs[2] + d0) : f32x4{};
-  }
-  f32x16 dk[C::NDT], dv[C::NDT];
-#pragma unroll
-  for (int dt = 0; dt < C::NDT; ++dt) {
-    dk[dt] = f32x16{};
-    dv[dt] = f32x16{};
-  }
-  const int r_begin = p.causal ? (wg_key0 / TT) * TT : 0;
-  // split (bwd_splits; 1 range of N rows otherwise): this work-group's rows [r_lo, r_hi) over grid z,
-  // whole 32-row stages.  An empty range writes no partial, and the combine (kind 0 past N, kind 2
-  // before a causal key block) skips it.
-  const int r_lo = max(r_begin, (int)wg.z * p.split_len), r_hi = min(p.N, (int)wg.z * p.split_len + p.split_len);
-  if (p.split > 1 && r_lo >= r_hi) return;
-  const int ntiles = r_hi > r_lo ? (r_hi - r_lo + TT - 1) / TT : 0;
-  Chunk16 qreg[F32Stage<DP, NT>::NCH], greg[F32Stage<DP, NT>::NCH];
-  float lreg = 0.f, loreg = 0.f, dreg = 0.f;
-  auto gload = [&](int t0) {
-    f32_stage_load<DP, NT>(qreg, Q, p.qs[2], t0, p.N, p.D, tid);
-    f32_stage_load<DP, NT>(greg, dO, p.gs[2], t0, p.N, p.D, tid);
-    if (tid < TT) {
-      const int ra = t0 + tid;
-      lreg = ra < p.N ? p.lse_row[(int64_t)bh * p.N + ra] : kNegInf;
-      loreg = ra < p.N ? p.lse_lo[(int64_t)bh * p.N + ra] : 0.f;
-      dreg = ra < p.N ? p.d_row[(int64_t)bh * p.N + ra] : 0.f;
-    }
-  };
-  auto sstore = [&](int buf) {
-    f32_stage_store2<DP, NT, F32Stage<DP, NT>::NCH, TS1, RS4>(qreg, Qt[buf], Qr[buf], tid);
-    f32_stage_store2<DP, NT, F32Stage<DP, NT>::NCH, TS1, RS4>(greg, Gt[buf], Gr[buf], tid);
-    if (tid < TT) {
-      lse_s[buf][tid] = lreg;
-      lo_s[buf][tid] = loreg;
-      dd_s[buf][tid] = dreg;
-    }
-  };
-  if (ntiles > 0) {
-    gload(r_lo);
-    sstore(0);
-  }
-  __syncthreads();
-
-  for (int it = 0; it < ntiles; ++it) {
-    const int t0 = r_lo + it * TT, buf = it & 1;
-    const bool has_next = it + 1 < ntiles;
-    if (has_next) gload(t0 + TT);
-    f32x16 s = f32x16{}, dp = f32x16{};
-    {
-      // A operands: stage row swap23(c), d = 8m + 4g .. + 3
-      const float* qr = Qr[buf] + swap23(c) * RS4 + 4 * g;
-      const float* gr = Gr[buf] + swap23(c) * RS4 + 4 * g;
-#pragma unroll
-      for (int m = 0; m < NM; ++m) {
-        const f32x4 qa = *reinterpret_cast<const f32x4*>(qr + 8 * m);
-        const f32x4 ga = *reinterpret_cast<const f32x4*>(gr + 8 * m);
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          s = M::mma(qa[u], kf[m][u], s);
-          dp = M::mma(ga[u], vf[m][u], dp);
-        }
-      }
-    }
-    f32x16 pv;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int rl = key_of_reg(r, g);
-      const int row = t0 + rl;
-      const float lse = lse_s[buf][rl];
-      bool ok = key_ok && row < p.N && lse > kNegInf;
-      if (p.causal) ok = ok && row >= my_key;
-      // s*c - LSE2 with one rounding of the (small) difference, then LSE2's low part
-      float x = fmaf(s[r], p.scale_log2, -lse) - lo_s[buf][rl];
-      if constexpr (HAS_BIAS) x = ok ? fmaf(load_bias_b(p.bias, bi, hi, row, my_key), kLog2e, x) : x;
-      const float pr = ok ? fast_exp2(x) : 0.f;
-      pv[r] = pr;
-      s[r] = pr * (dp[r] - dd_s[buf][rl]);
-      if constexpr (HAS_BIAS) {
-        if (p.ds_out != nullptr && key_ok && row < p.N) p.ds_out[((int64_t)bh * p.N + row) * p.N + my_key] = s[r];
-      }
-    }
-#pragma unroll
-    for (int jb = 0; jb < 4; ++jb) {
-      const int row0 = 16 * (jb >> 1) + 8 * g + 4 * (jb & 1);  // key_of_reg(4 jb, g)
-#pragma unroll
-      for (int dt = 0; dt < C::NDT; ++dt) {
-        const int off = (dt * 32 + c) * TS1 + row0;
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          dv[dt] = M::mma(Gt[buf][off + u], pv[4 * jb + u], dv[dt]);
-          dk[dt] = M::mma(Qt[buf][off + u], s[4 * jb + u], dk[dt]);
-        }
-      }
-    }
-    if (has_next) sstore(buf ^ 1);
-    __syncthreads();
-  }
-  if (!key_ok) return;
-  // registers 4q .. 4q + 3 hold head dims dt * 32 + drow(4q, g) .. + 3: one 16-byte store each
-  // (pointers are 16-byte aligned and strides multiples of 8 elements; D is a multiple of 8, so a
-  // group starting below D ends below it)
-  if (p.split > 1) {  // this row range's unscaled dK and dV: the combine sums the ranges and scales dK
-    const int64_t o = (((int64_t)wg.z * p.BH + bh) * p.N + my_key) * p.dp;
-    float* dkp = p.part + p.part_stride + o;
-    float* dvp = p.part + 2 * p.part_stride + o;
-#pragma unroll
-    for (int dt = 0; dt < C::NDT; ++dt)
-#pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
-        const int d = dt * 32 + drow(4 * q4, g);
-        *reinterpret_cast<f32x4*>(dkp + d) =
-            f32x4{dk[dt][4 * q4], dk[dt][4 * q4 + 1], dk[dt][4 * q4 + 2], dk[dt][4 * q4 + 3]};
-        *reinterpret_cast<f32x4*>(dvp + d) =
-            f32x4{dv[dt][4 * q4], dv[dt][4 * q4 + 1], dv[dt][4 * q4 + 2], dv[dt][4 * q4 + 3]};
-      }
-    return;
-  }
-  T* okp = static_cast<T*>(p.dk) + bi * p.dks[0] + hi * p.dks[1] + (int64_t)my_key * p.dks[2];
-  T* ovp = static_cast<T*>(p.dv) + bi * p.dvs[0] + hi * p.dvs[1] + (int64_t)my_key * p.dvs[2];
-#pragma unroll
-  for (int dt = 0; dt < C::NDT; ++dt)
-#pragma unroll
-    for (int q4 = 0; q4 < 4; ++q4) {
-      const int d = dt * 32 + drow(4 * q4, g);
-      if (d < p.D) {
-        *reinterpret_cast<f32x4*>(okp + d) = f32x4{dk[dt][4 * q4] * p.scale, dk[dt][4 * q4 + 1] * p.scale,
-                                                   dk[dt][4 * q4 + 2] * p.scale, dk[dt][4 * q4 + 3] * p.scale};
-        *reinterpret_cast<f32x4*>(ovp + d) =
-            f32x4{dv[dt][4 * q4], dv[dt][4 * q4 + 1], dv[dt][4 * q4 + 2], dv[dt][4 * q4 + 3]};
-      }
-    }
 }
 
 // ------------------------------------------------------------------ fp16 / bf16 dq and dk/dv
@@ -1512,13 +1056,28 @@ __global__ __launch_bounds__(64) void dbias_kernel(const BwdParams p, float* dbi
   }
 }
 
-// dbias = sum over split of part[split], in split order (deterministic).
+// dbias[e] = sum over split of part[split][e]: 32 elements per work-group, each summed by 8 threads over
+// the splits of one residue mod 8, whose sums are added in order (the result does not depend on
+// scheduling).  With one thread and one serial chain per element, 7203 elements were 29 work-groups.
 __global__ __launch_bounds__(256) void dbias_reduce_kernel(const float* part, float* dbias, int nsplit, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
+  __shared__ float acc_s[8][32];
+  const int e = threadIdx.x & 31, q = threadIdx.x >> 5;
+  const int64_t i = (int64_t)blockIdx.x * 32 + e;
   float acc = 0.f;
-  for (int sp = 0; sp < nsplit; ++sp) acc += part[sp * n + i];
+  if (i < n) {
+#pragma unroll 8
+    for (int sp = q; sp < nsplit; sp += 8) acc += part[sp * n + i];
+  }
+  acc_s[q][e] = acc;
+  __syncthreads();
+  if (q != 0 || i >= n) return;
+#pragma unroll
+  for (int w = 1; w < 8; ++w) acc += acc_s[w][e];
   dbias[i] = acc;
+}
+hipError_t launch_dbias_reduce(const float* part, float* dbias, int nsplit, int64_t n, hipStream_t st) {
+  hipLaunchKernelGGL(dbias_reduce_kernel, dim3((unsigned)((n + 31) / 32)), dim3(256), 0, st, part, dbias, nsplit, n);
+  return hipGetLastError();
 }
 
 // dbias[bb', hb', i, j] = sum over the (b, h) pairs broadcast onto (bb', hb') of ds[b, h, i, j].
@@ -1570,8 +1129,7 @@ hipError_t launch_dbias_sum(const float* ds, float* dbias, int B, int H, int N, 
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || nsplit == 1) return e;
   const int64_t n = (int64_t)bias_batch * bias_heads * nn;
-  hipLaunchKernelGGL(dbias_reduce_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, part, dbias, nsplit, n);
-  return hipGetLastError();
+  return launch_dbias_reduce(part, dbias, nsplit, n, st);
 }
 
 hipError_t launch_zero_fill(float* dst, int64_t n, hipStream_t st) {
@@ -1591,8 +1149,33 @@ static int64_t causal_live_wgs(int64_t bh, int64_t n, int s) {
   return bh * live;
 }
 
+// fp32 grids whose last round of the chip is mostly empty: the range count 1..8 that minimises rounds x
+// (stage rows of a range + 65) plus the combine's traffic, in units of one key or row of one round of the
+// 8-wave dk/dv kernel (0.12 us at d64; the two kernels' rounds as in bwd_f32_waves_dq / _dkdv; 65 for a
+// work-group's fixed cost, 180 + 0.0032 x work-groups x head dim per range for the combine).  Whole
+// backward ms, d64: B2 H8 N4097 (528 work-groups for 512 slots) 1.90 -> 1.45 (1 -> 5 ranges); head dim 128 (one
+// 4-wave work-group per CU): B1 H8 2K 0.670 -> 0.377 (1 -> 2), B4 H2 N300 0.120 -> 0.056 (1 -> 4), B1 H8 4K stays.
+static int f32_ragged_splits(int dp, int64_t bh, int64_t n) {
+  const int64_t w4 = bh * ((n + 127) / 128), w8 = bh * ((n + 255) / 256);
+  int best = 1;
+  double best_cost = 0;
+  for (int s = 1; s <= 8 && (s == 1 || n / s >= 64); ++s) {
+    const double k4 = (double)((w4 * s + 255) / 256), k8 = (double)((w8 * s + 255) / 256);
+    const double dq4 = (double)((int64_t)k4 / 2) + ((int64_t)k4 % 2 ? 0.645 : 0.0);
+    const double rounds = dp > 64 ? 2.33 * k4 : std::min(0.94 * k8, dq4) + 1.33 * std::min(k8, 0.645 * k4);
+    const double len = (double)(((n + s - 1) / s + 31) / 32 * 32);
+    const double cost = rounds * (len + 65) + (s > 1 ? 180 + 0.0032 * (double)(w4 * dp) * s : 0.0);
+    if (s == 1 || cost < best_cost) {
+      best = s;
+      best_cost = cost;
+    }
+  }
+  return best;
+}
+
 int bwd_splits(int dtype, int dp, int64_t bh, int64_t n, bool bias, bool causal) {
-  if (bias || dp > 64) return 1;
+  if (bias || (dp > 64 && dtype != ELSA_F32)) return 1;
+  if (dp > 64) return f32_ragged_splits(dp, bh, n);
   const int64_t wgs = bh * ((n + 127) / 128);  // the unsplit 4-wave grid
   // double while the doubled grid stays within one round of 512 work-groups (two per CU): whole
   // backward, fp16 d64, against doubling while the grid was short of 512: B8 H3 N1025 0.083 ->
@@ -1607,6 +1190,7 @@ int bwd_splits(int dtype, int dp, int64_t bh, int64_t n, bool bias, bool causal)
   // B2 H8 N2049 0.895 -> 0.571 (1 -> 2), B1 H8 N4097 1.305 -> 1.098, N5000 1.773 -> 1.333, N3000
   // 0.800 -> 0.723 (2 -> 4).  fp16 went both ways (B2 H8 N2049 0.103 -> 0.085 ms, but B1 H12 N2048
   // 0.076 -> 0.083 and B1 H8 N5000 0.169 -> 0.177), so 16-bit calls count every work-group.
+  if (dtype == ELSA_F32 && !causal && dp == 64 && wgs > 256) return f32_ragged_splits(dp, bh, n);
   const int64_t min_range = dtype == ELSA_F32 ? 64 : 256;
   const bool live_only = causal && dtype == ELSA_F32 && wgs <= 512;
   int s = 1;
@@ -1624,13 +1208,6 @@ int bwd_splits(int dtype, int dp, int64_t bh, int64_t n, bool bias, bool causal)
 //   kind 2 (dK, dV of key n): row ranges z with (z + 1) * split_len <= 128 * (n / 128).
 // Every kind skips ranges that start at or past N.  Those ranges would add zeros, so the sums are
 // the same up to the sign of a zero.
-struct CombineOut {
-  const float* part;
-  void* out;
-  int64_t os[3];
-  float scale;
-  int kind;
-};
 template <typename T>
 __global__ __launch_bounds__(256) void bwd_combine_kernel(CombineOut c0, CombineOut c1, CombineOut c2, int split,
                                                           int split_len, int64_t sstride, int H, int N, int D,
@@ -1680,6 +1257,10 @@ static hipError_t combine_launch(const BwdParams& p, const CombineOut* c, int n,
   return hipGetLastError();
 }
 
+hipError_t combine_launch_f32(const BwdParams& p, const CombineOut* c, int n, hipStream_t st) {
+  return combine_launch<float>(p, c, n, st);
+}
+
 // ------------------------------------------------------------------ launchers
 template <typename T>
 static hipError_t pre_launch(const BwdParams& p, hipStream_t st) {
@@ -1702,19 +1283,11 @@ static hipError_t bwd_launch_short(const BwdParams& p, int stage, hipStream_t st
   const dim3 grid((p.N + 32 * W - 1) / (32 * W), p.BH);
   hipError_t e = hipSuccess;
   if (stage < 0 || stage == 1) {
-    if constexpr (sizeof(T) == 2) {
-      hipLaunchKernelGGL((bwd_dq_half_kernel<T, DP, 1, W, B>), grid, dim3(64 * W), 0, st, p);
-    } else {
-      hipLaunchKernelGGL((bwd_dq_kernel<T, DP, W, B>), grid, dim3(64 * W), 0, st, p);
-    }
+    hipLaunchKernelGGL((bwd_dq_half_kernel<T, DP, 1, W, B>), grid, dim3(64 * W), 0, st, p);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
   if (stage < 0 || stage == 2) {
-    if constexpr (sizeof(T) == 2) {
-      hipLaunchKernelGGL((bwd_dkdv_half_kernel<T, DP, 1, W, B>), grid, dim3(64 * W), 0, st, p);
-    } else {
-      hipLaunchKernelGGL((bwd_dkdv_kernel<T, DP, W, B>), grid, dim3(64 * W), 0, st, p);
-    }
+    hipLaunchKernelGGL((bwd_dkdv_half_kernel<T, DP, 1, W, B>), grid, dim3(64 * W), 0, st, p);
     e = hipGetLastError();
   }
   return e;
@@ -1727,180 +1300,153 @@ static hipError_t bwd_launch3(const BwdParams& p, int stage, hipStream_t st) {
   // LDS-direct staging (unbiased fp16/bf16 D = 64 kernels) where the buffer ranges of N rows stay
   // below 2^31 bytes: K/V for dq, Q/dO for dK/dV.  The LDS-direct dq kernels also run the
   // preprocess of their rows, so a whole backward then launches no bwd_pre_kernel.
+  static_assert(sizeof(T) == 2, "fp32: launch_bwd_f32");
   const int64_t lim = int64_t(1) << 31, es = (int64_t)sizeof(T);
-  const bool ld_kv = sizeof(T) == 2 && !B && DP == 64 && p.D == 64 && (int64_t)p.N * p.ks[2] * es < lim &&
+  const bool ld_kv = !B && DP == 64 && p.D == 64 && (int64_t)p.N * p.ks[2] * es < lim &&
                      (int64_t)p.N * p.vs[2] * es < lim;
-  const bool ld_qg = sizeof(T) == 2 && !B && DP == 64 && p.D == 64 && (int64_t)p.N * p.qs[2] * es < lim &&
+  const bool ld_qg = !B && DP == 64 && p.D == 64 && (int64_t)p.N * p.qs[2] * es < lim &&
                      (int64_t)p.N * p.gs[2] * es < lim;
-  // the fp32 dq kernels at D <= 64 run the preprocess of their rows too
-  const bool pre_in_dq = ld_kv || (sizeof(T) == 4 && DP <= 64);
-  if (stage == 0 || (stage < 0 && !pre_in_dq)) {
+  if (stage == 0 || (stage < 0 && !ld_kv)) {
     if ((e = pre_launch<T>(p, st)) != hipSuccess) return e;
   }
   if constexpr (DP == 32) {
     if (p.N <= 64) return stage == 0 ? e : bwd_launch_short<T, DP, B>(p, stage, st);
   }
-  if constexpr (sizeof(T) == 2) {
-    constexpr int R = 1;  // one 32-wide tile per wave: 2 waves per SIMD beat wider tiles at 1
-    const dim3 grid((p.N + 32 * R * W - 1) / (32 * R * W), p.BH);
-    if constexpr (!B && DP <= 64) {
-      if (p.split > 1) {
-        // an under-filled grid (short sequences, few heads): the key (dq) or row (dK/dV) loop cut
-        // into p.split ranges over grid z, fp32 partials summed by a combine launch
-        const dim3 gs(grid.x, grid.y, (unsigned)p.split);
-        const int kq = p.causal ? 1 : 0, kkv = p.causal ? 2 : 0;
-        const CombineOut cq{p.part, p.dq, {p.dqs[0], p.dqs[1], p.dqs[2]}, p.scale, kq};
-        const CombineOut ck{p.part + p.part_stride, p.dk, {p.dks[0], p.dks[1], p.dks[2]}, p.scale, kkv};
-        const CombineOut cv{p.part + 2 * p.part_stride, p.dv, {p.dvs[0], p.dvs[1], p.dvs[2]}, 1.f, kkv};
-        if (stage < 0 || stage == 1) {
-          if (ld_kv) {
-            hipLaunchKernelGGL((bwd_dq_half_kernel<T, DP, R, W, false, DP == 64>), gs, dim3(64 * W), 0, st, p);
-          } else {
-            hipLaunchKernelGGL((bwd_dq_half_kernel<T, DP, R, W, false>), gs, dim3(64 * W), 0, st, p);
-          }
-          if ((e = hipGetLastError()) != hipSuccess) return e;
-          if (stage == 1 && (e = combine_launch<T>(p, &cq, 1, st)) != hipSuccess) return e;
-        }
-        if (stage < 0 || stage == 2) {
-          if (ld_qg) {
-            hipLaunchKernelGGL((bwd_dkdv_half_kernel<T, DP, R, W, false, DP == 64>), gs, dim3(64 * W), 0, st, p);
-          } else {
-            hipLaunchKernelGGL((bwd_dkdv_half_kernel<T, DP, R, W, false>), gs, dim3(64 * W), 0, st, p);
-          }
-          if ((e = hipGetLastError()) != hipSuccess) return e;
-        }
-        // the whole backward sums the three gradients' partials in one launch
-        if (stage < 0) {
-          const CombineOut all[3] = {cq, ck, cv};
-          e = combine_launch<T>(p, all, 3, st);
-        } else if (stage == 2) {
-          const CombineOut kv[2] = {ck, cv};
-          e = combine_launch<T>(p, kv, 2, st);
-        }
-        return e;
-      }
-    }
-    if (stage < 0 || stage == 1) {
-      // dq with two 32-row tiles per wave: each K/V fragment read from LDS feeds both tiles,
-      // halving the LDS reads per MFMA.  Unbiased, D <= 64 (causal: below), and only where the grid
-      // still puts two 256-row work-groups on every CU.  B1 H8 d64 16K: fp16 0.875 -> 0.814 ms, bf16
-      // 0.841 -> 0.768 ms; causal 16K 0.479 against 0.510 ms and 4K (128 work-groups) 0.074 against
-      // 0.111 ms stay on the 32-row kernel.  At D = 64, 8-wave work-groups of 512 rows (one per CU,
-      // 246 VGPRs), so each K/V stage staged once serves twice the rows: 16K 0.794 -> 0.766 ms (fp16),
-      // 0.750 -> 0.720 ms (bf16), B2 H8 8K 0.404 -> 0.388 ms, 64K 12.13 -> 11.86 ms.
-      const dim3 grid2((p.N + 255) / 256, p.BH);
-      bool wide = false;
-      if constexpr (DP <= 64 && !B) {
-        // causal calls take the two-tile kernel where its 512-row work-groups come in whole pairs of
-        // rounds (a multiple of 512) over heads of at least 32 row blocks, so that the heaviest-first
-        // order balances: dq causal 32K 1.616 -> 1.514 ms, 64K 6.35 -> 5.89 ms, B1 H16 16K 0.829 ->
-        // 0.787 ms, B2 H8 16K bf16 0.778 -> 0.738 ms; one round (B1 H8 16K, 256 work-groups) took
-        // 0.427 -> 0.605 ms, B4 H8 8K 0.457 -> 0.555 ms and B8 H3 N16385 (792) 1.25 -> 1.37 ms
-        const dim3 grid8((p.N + 511) / 512, p.BH);
-        const int64_t n8 = (int64_t)grid8.x * grid8.y;
-        // non-causal D = 64 also where the 512-row work-groups take fewer rounds of the chip (256 at
-        // one per CU) than the 128-row ones (512 at two per CU): B8 H3 N4097 dq 0.190 -> 0.170 ms
-        // (792 work-groups, 2 rounds, against 216, 1); with the rounds level, B1 H8 8K 0.206 -> 0.282 ms
-        const int64_t g1 = (int64_t)((p.N + 127) / 128) * p.BH;
-        const bool fewer_rounds = DP == 64 && !p.causal && (g1 + 511) / 512 > (n8 + 255) / 256;
-        wide = ((int64_t)grid2.x * grid2.y >= 512 && (!p.causal || (DP == 64 && p.N >= 16384 && n8 % 512 == 0))) ||
-               fewer_rounds;
-        bool w8 = false;
-        if constexpr (DP == 64) {
-          if (wide && (n8 >= 256 || fewer_rounds)) {
-            // LDS-direct staging where every head dim chunk is data (D = 64) and the buffer ranges of
-            // N rows of K and V stay below 2^31 bytes
-            if (ld_kv) {
-              hipLaunchKernelGGL((bwd_dq_half_kernel<T, DP, 2, 8, false, true>), grid8, dim3(512), 0, st, p);
-            } else {
-              hipLaunchKernelGGL((bwd_dq_half_kernel<T, DP, 2, 8, false>), grid8, dim3(512), 0, st, p);
-            }
-            w8 = true;
-          }
-        }
-        if (wide && !w8) hipLaunchKernelGGL((bwd_dq_half_kernel<T, DP, 2, W, false>), grid2, dim3(64 * W), 0, st, p);
-      }
-      // otherwise, at D = 64 with the same grid condition, 8-wave work-groups of 32-row tiles
-      // (256 rows): the K/V stage staged once for twice the rows.  Causal 16K dq 0.466 -> 0.412 ms,
-      // 32K 1.675 -> 1.589 ms.
-      if (!wide) {
-        if constexpr (DP == 64) {
-          if ((int64_t)grid2.x * grid2.y >= 512) {
-            if (ld_kv) {
-              hipLaunchKernelGGL((bwd_dq_half_kernel<T, DP, R, 8, false, !B>), grid2, dim3(512), 0, st, p);
-            } else {
-              hipLaunchKernelGGL((bwd_dq_half_kernel<T, DP, R, 8, B>), grid2, dim3(512), 0, st, p);
-            }
-            wide = true;
-          }
-        }
-      }
-      if (!wide) {
+  constexpr int R = 1;  // one 32-wide tile per wave: 2 waves per SIMD beat wider tiles at 1
+  const dim3 grid((p.N + 32 * R * W - 1) / (32 * R * W), p.BH);
+  if constexpr (!B && DP <= 64) {
+    if (p.split > 1) {
+      // an under-filled grid (short sequences, few heads): the key (dq) or row (dK/dV) loop cut
+      // into p.split ranges over grid z, fp32 partials summed by a combine launch
+      const dim3 gs(grid.x, grid.y, (unsigned)p.split);
+      const int kq = p.causal ? 1 : 0, kkv = p.causal ? 2 : 0;
+      const CombineOut cq{p.part, p.dq, {p.dqs[0], p.dqs[1], p.dqs[2]}, p.scale, kq};
+      const CombineOut ck{p.part + p.part_stride, p.dk, {p.dks[0], p.dks[1], p.dks[2]}, p.scale, kkv};
+      const CombineOut cv{p.part + 2 * p.part_stride, p.dv, {p.dvs[0], p.dvs[1], p.dvs[2]}, 1.f, kkv};
+      if (stage < 0 || stage == 1) {
         if (ld_kv) {
-          hipLaunchKernelGGL((bwd_dq_half_kernel<T, DP, R, W, false, !B && DP == 64>), grid, dim3(64 * W), 0, st, p);
+          hipLaunchKernelGGL((bwd_dq_half_kernel<T, DP, R, W, false, DP == 64>), gs, dim3(64 * W), 0, st, p);
         } else {
-          hipLaunchKernelGGL((bwd_dq_half_kernel<T, DP, R, W, B>), grid, dim3(64 * W), 0, st, p);
+          hipLaunchKernelGGL((bwd_dq_half_kernel<T, DP, R, W, false>), gs, dim3(64 * W), 0, st, p);
         }
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+        if (stage == 1 && (e = combine_launch<T>(p, &cq, 1, st)) != hipSuccess) return e;
       }
-      if ((e = hipGetLastError()) != hipSuccess) return e;
+      if (stage < 0 || stage == 2) {
+        if (ld_qg) {
+          hipLaunchKernelGGL((bwd_dkdv_half_kernel<T, DP, R, W, false, DP == 64>), gs, dim3(64 * W), 0, st, p);
+        } else {
+          hipLaunchKernelGGL((bwd_dkdv_half_kernel<T, DP, R, W, false>), gs, dim3(64 * W), 0, st, p);
+        }
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+      }
+      // the whole backward sums the three gradients' partials in one launch
+      if (stage < 0) {
+        const CombineOut all[3] = {cq, ck, cv};
+        e = combine_launch<T>(p, all, 3, st);
+      } else if (stage == 2) {
+        const CombineOut kv[2] = {ck, cv};
+        e = combine_launch<T>(p, kv, 2, st);
+      }
+      return e;
     }
-    if (stage < 0 || stage == 2) {
-      // dK/dV in 8-wave work-groups (256 keys) at D = 64 where that grid still puts two
-      // work-groups on every CU: 16K 1.109 -> 1.078 ms, causal 16K 0.602 -> 0.569 ms, bf16 16K
-      // 1.053 -> 1.028 ms; at 4K (128 work-groups) 0.101 against 0.130 ms, so smaller grids keep 4.
-      // Non-causal grids of 256-511 work-groups (one round at one per CU) take 8 too: dK/dV B8 H3
-      // N4097 0.290 -> 0.278 ms, B1 H8 8K 0.267 -> 0.261 ms, B2 H8 4K 0.138 -> 0.136 ms
+  }
+  if (stage < 0 || stage == 1) {
+    // dq with two 32-row tiles per wave: each K/V fragment read from LDS feeds both tiles,
+    // halving the LDS reads per MFMA.  Unbiased, D <= 64 (causal: below), and only where the grid
+    // still puts two 256-row work-groups on every CU.  B1 H8 d64 16K: fp16 0.875 -> 0.814 ms, bf16
+    // 0.841 -> 0.768 ms; causal 16K 0.479 against 0.510 ms and 4K (128 work-groups) 0.074 against
+    // 0.111 ms stay on the 32-row kernel.  At D = 64, 8-wave work-groups of 512 rows (one per CU,
+    // 246 VGPRs), so each K/V stage staged once serves twice the rows: 16K 0.794 -> 0.766 ms (fp16),
+    // 0.750 -> 0.720 ms (bf16), B2 H8 8K 0.404 -> 0.388 ms, 64K 12.13 -> 11.86 ms.
+    const dim3 grid2((p.N + 255) / 256, p.BH);
+    bool wide = false;
+    if constexpr (DP <= 64 && !B) {
+      // causal calls take the two-tile kernel where its 512-row work-groups come in whole pairs of
+      // rounds (a multiple of 512) over heads of at least 32 row blocks, so that the heaviest-first
+      // order balances: dq causal 32K 1.616 -> 1.514 ms, 64K 6.35 -> 5.89 ms, B1 H16 16K 0.829 ->
+      // 0.787 ms, B2 H8 16K bf16 0.778 -> 0.738 ms; one round (B1 H8 16K, 256 work-groups) took
+      // 0.427 -> 0.605 ms, B4 H8 8K 0.457 -> 0.555 ms and B8 H3 N16385 (792) 1.25 -> 1.37 ms
+      const dim3 grid8((p.N + 511) / 512, p.BH);
+      const int64_t n8 = (int64_t)grid8.x * grid8.y;
+      // non-causal D = 64 also where the 512-row work-groups take fewer rounds of the chip (256 at
+      // one per CU) than the 128-row ones (512 at two per CU): B8 H3 N4097 dq 0.190 -> 0.170 ms
+      // (792 work-groups, 2 rounds, against 216, 1); with the rounds level, B1 H8 8K 0.206 -> 0.282 ms
+      const int64_t g1 = (int64_t)((p.N + 127) / 128) * p.BH;
+      const bool fewer_rounds = DP == 64 && !p.causal && (g1 + 511) / 512 > (n8 + 255) / 256;
+      wide = ((int64_t)grid2.x * grid2.y >= 512 && (!p.causal || (DP == 64 && p.N >= 16384 && n8 % 512 == 0))) ||
+             fewer_rounds;
       bool w8 = false;
       if constexpr (DP == 64) {
-        const dim3 g8((p.N + 255) / 256, p.BH);
-        if ((int64_t)g8.x * g8.y >= (p.causal ? 512 : 256)) {
+        if (wide && (n8 >= 256 || fewer_rounds)) {
           // LDS-direct staging where every head dim chunk is data (D = 64) and the buffer ranges of
-          // N rows of Q and dO stay below 2^31 bytes
-          if constexpr (!B) {
-            if (ld_qg) {
-              hipLaunchKernelGGL((bwd_dkdv_half_kernel<T, DP, R, 8, false, true>), g8, dim3(512), 0, st, p);
-            } else {
-              hipLaunchKernelGGL((bwd_dkdv_half_kernel<T, DP, R, 8, B>), g8, dim3(512), 0, st, p);
-            }
+          // N rows of K and V stay below 2^31 bytes
+          if (ld_kv) {
+            hipLaunchKernelGGL((bwd_dq_half_kernel<T, DP, 2, 8, false, true>), grid8, dim3(512), 0, st, p);
           } else {
-            hipLaunchKernelGGL((bwd_dkdv_half_kernel<T, DP, R, 8, B>), g8, dim3(512), 0, st, p);
+            hipLaunchKernelGGL((bwd_dq_half_kernel<T, DP, 2, 8, false>), grid8, dim3(512), 0, st, p);
           }
           w8 = true;
         }
       }
-      if (!w8) {
-        if (ld_qg) {
-          hipLaunchKernelGGL((bwd_dkdv_half_kernel<T, DP, R, W, false, !B && DP == 64>), grid, dim3(64 * W), 0, st, p);
-        } else {
-          hipLaunchKernelGGL((bwd_dkdv_half_kernel<T, DP, R, W, B>), grid, dim3(64 * W), 0, st, p);
+      if (wide && !w8) hipLaunchKernelGGL((bwd_dq_half_kernel<T, DP, 2, W, false>), grid2, dim3(64 * W), 0, st, p);
+    }
+    // otherwise, at D = 64 with the same grid condition, 8-wave work-groups of 32-row tiles
+    // (256 rows): the K/V stage staged once for twice the rows.  Causal 16K dq 0.466 -> 0.412 ms,
+    // 32K 1.675 -> 1.589 ms.
+    if (!wide) {
+      if constexpr (DP == 64) {
+        if ((int64_t)grid2.x * grid2.y >= 512) {
+          if (ld_kv) {
+            hipLaunchKernelGGL((bwd_dq_half_kernel<T, DP, R, 8, false, !B>), grid2, dim3(512), 0, st, p);
+          } else {
+            hipLaunchKernelGGL((bwd_dq_half_kernel<T, DP, R, 8, B>), grid2, dim3(512), 0, st, p);
+          }
+          wide = true;
         }
       }
-      e = hipGetLastError();
     }
-  } else {
-    // fp32: the key (dq) and row (dK/dV) loops split over grid z for under-filled grids, as above
-    const dim3 grid((p.N + 32 * W - 1) / (32 * W), p.BH, (unsigned)(p.split > 1 ? p.split : 1));
-    const int kq = p.causal ? 1 : 0, kkv = p.causal ? 2 : 0;
-    const CombineOut cq{p.part, p.dq, {p.dqs[0], p.dqs[1], p.dqs[2]}, p.scale, kq};
-    const CombineOut ck{p.part + p.part_stride, p.dk, {p.dks[0], p.dks[1], p.dks[2]}, p.scale, kkv};
-    const CombineOut cv{p.part + 2 * p.part_stride, p.dv, {p.dvs[0], p.dvs[1], p.dvs[2]}, 1.f, kkv};
-    if (stage < 0 || stage == 1) {
-      hipLaunchKernelGGL((bwd_dq_kernel<T, DP, W, B>), grid, dim3(64 * W), 0, st, p);
-      if ((e = hipGetLastError()) != hipSuccess) return e;
-      if (p.split > 1 && stage == 1 && (e = combine_launch<T>(p, &cq, 1, st)) != hipSuccess) return e;
-    }
-    if (stage < 0 || stage == 2) {
-      hipLaunchKernelGGL((bwd_dkdv_kernel<T, DP, W, B>), grid, dim3(64 * W), 0, st, p);
-      if ((e = hipGetLastError()) != hipSuccess) return e;
-      if (p.split > 1 && stage == 2) {
-        const CombineOut kv[2] = {ck, cv};
-        e = combine_launch<T>(p, kv, 2, st);
+    if (!wide) {
+      if (ld_kv) {
+        hipLaunchKernelGGL((bwd_dq_half_kernel<T, DP, R, W, false, !B && DP == 64>), grid, dim3(64 * W), 0, st, p);
+      } else {
+        hipLaunchKernelGGL((bwd_dq_half_kernel<T, DP, R, W, B>), grid, dim3(64 * W), 0, st, p);
       }
     }
-    if (p.split > 1 && stage < 0) {
-      const CombineOut all[3] = {cq, ck, cv};
-      e = combine_launch<T>(p, all, 3, st);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+  }
+  if (stage < 0 || stage == 2) {
+    // dK/dV in 8-wave work-groups (256 keys) at D = 64 where that grid still puts two
+    // work-groups on every CU: 16K 1.109 -> 1.078 ms, causal 16K 0.602 -> 0.569 ms, bf16 16K
+    // 1.053 -> 1.028 ms; at 4K (128 work-groups) 0.101 against 0.130 ms, so smaller grids keep 4.
+    // Non-causal grids of 256-511 work-groups (one round at one per CU) take 8 too: dK/dV B8 H3
+    // N4097 0.290 -> 0.278 ms, B1 H8 8K 0.267 -> 0.261 ms, B2 H8 4K 0.138 -> 0.136 ms
+    bool w8 = false;
+    if constexpr (DP == 64) {
+      const dim3 g8((p.N + 255) / 256, p.BH);
+      if ((int64_t)g8.x * g8.y >= (p.causal ? 512 : 256)) {
+        // LDS-direct staging where every head dim chunk is data (D = 64) and the buffer ranges of
+        // N rows of Q and dO stay below 2^31 bytes
+        if constexpr (!B) {
+          if (ld_qg) {
+            hipLaunchKernelGGL((bwd_dkdv_half_kernel<T, DP, R, 8, false, true>), g8, dim3(512), 0, st, p);
+          } else {
+            hipLaunchKernelGGL((bwd_dkdv_half_kernel<T, DP, R, 8, B>), g8, dim3(512), 0, st, p);
+          }
+        } else {
+          hipLaunchKernelGGL((bwd_dkdv_half_kernel<T, DP, R, 8, B>), g8, dim3(512), 0, st, p);
+        }
+        w8 = true;
+      }
     }
+    if (!w8) {
+      if (ld_qg) {
+        hipLaunchKernelGGL((bwd_dkdv_half_kernel<T, DP, R, W, false, !B && DP == 64>), grid, dim3(64 * W), 0, st, p);
+      } else {
+        hipLaunchKernelGGL((bwd_dkdv_half_kernel<T, DP, R, W, B>), grid, dim3(64 * W), 0, st, p);
+      }
+    }
+    e = hipGetLastError();
   }
   return e;
 }
@@ -1920,9 +1466,10 @@ static hipError_t bwd_launch1(const BwdParams& p, int stage, hipStream_t st) {
 }
 
 hipError_t launch_bwd(const BwdParams& p, int dtype, int stage, hipStream_t st) {
+  if (stage < 0 && bwd_short_takes(dtype, p.N, p.dp)) return launch_bwd_short(p, dtype, p.ds_out ? 1 : 0, st);
   if (dtype == ELSA_F16) return bwd_launch1<f16>(p, stage, st);
   if (dtype == ELSA_BF16) return bwd_launch1<bf16>(p, stage, st);
-  return bwd_launch1<float>(p, stage, st);
+  return stage == 0 ? pre_launch<float>(p, st) : launch_bwd_f32(p, stage, st);
 }
 
 template <typename T, int DP>
@@ -1961,8 +1508,7 @@ static hipError_t db_launch2(const BwdParams& p, float* dbias, int bb, int hb, i
   hipLaunchKernelGGL((dbias_kernel<T, DP>), grid, dim3(64), 0, st, p, dbias, bb, hb, nsplit, part);
   if ((e = hipGetLastError()) != hipSuccess || nsplit == 1) return e;
   const int64_t n = (int64_t)bb * hb * p.N * p.N;
-  hipLaunchKernelGGL(dbias_reduce_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, part, dbias, nsplit, n);
-  return hipGetLastError();
+  return launch_dbias_reduce(part, dbias, nsplit, n, st);
 }
 
 template <typename T>

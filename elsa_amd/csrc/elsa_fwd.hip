@@ -3,7 +3,8 @@
 //
 // Phase 1 (replaces the Triton summary kernels of the reference,
 // attention_parallel_scan.py:123-372 and attention.py:22-106):
-//   one workgroup = 32*WAVES query rows of one head x one K partition.
+//   one workgroup = 32*WAVES query rows of one head x one K partition (fp32: phase1_x3_kernel, which
+//   forms the fp32 products on the bf16 MFMA; 64-row blocks at D > 64 on the fp32 one, phase1_kernel).
 //   Each wave owns a 32-row tile and computes S^T = K Q^T on 32x32 MFMA tiles
 //   (Q^T fragments live in registers for the whole partition, K tiles come from
 //   LDS), folds the running (m, z) in registers, and accumulates
@@ -175,7 +176,7 @@ __device__ inline void emit4(const Phase1Params& p, int64_t ridx, int64_t ooff, 
 
 template <typename T, int DP, int WAVES, bool HAS_BIAS>
 __global__ __launch_bounds__(64 * WAVES) void phase1_kernel(const Phase1Params p) {
-  static_assert(sizeof(T) == 4, "fp32 fold (fp16 / bf16: phase1_half_kernel)");
+  static_assert(sizeof(T) == 4, "fp32 fold of 64-row blocks at D > 64 (others: phase1_x3_kernel)");
   using C = FwdCfg<T, DP>;
   using M = Mfma<T>;
   // The fp32 MFMA takes one operand element per lane and k-step, and the contraction order
@@ -380,6 +381,261 @@ __global__ __launch_bounds__(64 * WAVES) void phase1_kernel(const Phase1Params p
     }
 }
 
+constexpr float kLazyTau = 8.0f;
+constexpr float kLazySum = 256.0f;  // 2^kLazyTau
+
+// ------------------------------------------------------------------ Phase 1, fp32 on the bf16 MFMA
+// The fp32 fold with both products formed from three bf16 parts per operand (Split3).  One workgroup
+// = 32*WAVES query rows x one K partition, 32-key stages.  A wave holds its rows' Q^T parts in
+// registers; the K and V stage tiles are split once by the thread that loads them and kept in LDS as
+// three row-major bf16 planes each, read as row fragments (K) and with the transposing load (V), as in
+// phase1_half_kernel.  Each product sums its small partial products first and its leading ones last,
+// and a stage's P^T V goes into a fresh accumulator that is added to the running one: N/32 roundings
+// of a running sum per output element instead of N/2.
+// Bound: the matrix cores.  48 MFMAs of 8 passes per 32 x 32 score tile (d64) against the 64 of 16
+// passes of the fp32 MFMA fold (phase1_kernel).  Forward ms, phase1_kernel -> this (relative error
+// against 64 bits): B1 H8 d64 16K 4.60 -> 2.64 (1.65e-6 -> 3.8e-7; 1.25 PFLOP/s of MFMA work, above the
+// 1.14 a large bf16 library product reaches), 8K 1.175 -> 0.673 (1.2e-6 -> 2.9e-7), 1K 0.0356 -> 0.0250,
+// B8 H3 N197 0.0149 -> 0.0135, d128 4K 0.670 -> 0.343 (7.1e-7 -> 2.3e-7), causal 4K 0.196 -> 0.115.
+template <int DP>
+struct X3Tile {
+  static constexpr bool SWZ = DP == 64;
+  static constexpr int KT = 32;
+  static constexpr int KS = SWZ ? DP : DP + 8;
+  __device__ static inline int off(int r, int col) { return SWZ ? lds_swz_off(r, col) : r * KS + col; }
+};
+
+template <int DP, int WAVES, bool HAS_BIAS>
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(DP >= 128 ? 1 : 2, 2)))
+void phase1_x3_kernel(const Phase1Params p) {
+  using Tile = X3Tile<DP>;
+  using M = Mfma<bf16>;
+  constexpr int KT = Tile::KT, KS = Tile::KS, NKK = DP / 16, NDT = DP / 32;
+  constexpr int NT = 64 * WAVES, BM = 32 * WAVES;
+  constexpr int CPR = DP / 8;        // 8-element chunks per key row
+  constexpr int TCH = KT * CPR;      // chunks per stage tile
+  static_assert((2 * TCH) % NT == 0 && TCH % 64 == 0, "whole chunks per thread, whole waves per tensor");
+  constexpr int NCH = 2 * TCH / NT;  // chunks per thread, K's first
+
+  __shared__ __attribute__((aligned(16))) bf16 Kp[2][3][KT * KS];
+  __shared__ __attribute__((aligned(16))) bf16 Vp[2][3][KT * KS];
+
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 31, g = lane >> 5;
+  const bool lpt = p.causal && p.q_start == 0 && p.q_len == p.N && p.part_len % BM == 0;
+  const WgCoord wg = lpt ? causal_longest_first((int)gridDim.x, p.BH, p.P, p.part_len / BM) : phase1_order(p.causal);
+  const int bh = wg.y, kb = wg.z;
+  const int q_end = p.q_start + p.q_len;
+  const int wg_row0 = p.q_start + wg.x * BM;
+  const int wg_last = min(q_end, wg_row0 + BM) - 1;
+  const int k_begin = kb * p.part_len;
+  int k_end = min(p.N, k_begin + p.part_len);
+  if (p.causal) k_end = min(k_end, wg_last + 1);
+  if (k_begin >= k_end) return;  // every row of this workgroup sees the identity here
+
+  const int row0 = wg_row0 + wave * 32;
+  const int my_row = row0 + c;
+  const bool row_ok = my_row < q_end;
+  const int bi = bh / p.H, hi = bh - (bh / p.H) * p.H;
+  const float* __restrict__ Q = static_cast<const float*>(p.q) + bi * p.qs[0] + hi * p.qs[1];
+  const float* __restrict__ K = static_cast<const float*>(p.k) + bi * p.ks[0] + hi * p.ks[1];
+  const float* __restrict__ V = static_cast<const float*>(p.v) + bi * p.vs[0] + hi * p.vs[1];
+
+  // stage chunks: chunk ci = tid + i NT of the 2 TCH chunks (K's, then V's), key ci % TCH / CPR; keys
+  // past k_end and head dims past D read as zeros from the buffer range
+  const uint32_t krs = (uint32_t)p.ks[2] * 4u, vrs = (uint32_t)p.vs[2] * 4u;
+  const auto rk = make_rsrc(K + (int64_t)k_begin * p.ks[2], (uint32_t)(k_end - k_begin) * krs);
+  const auto rv = make_rsrc(V + (int64_t)k_begin * p.vs[2], (uint32_t)(k_end - k_begin) * vrs);
+  Chunk16 reg[NCH][2];
+  auto gload = [&](int t0) {
+    const uint32_t kt = (uint32_t)(t0 - k_begin);
+    static_for<0, NCH>([&](auto I) {
+      constexpr int i = decltype(I)::value;
+      const int ci = tid + i * NT;
+      const bool is_v = wave * 64 + i * NT >= TCH;  // wave-uniform
+      const int cj = ci % TCH, key = cj / CPR, d0 = (cj % CPR) * 8;
+      const uint32_t rs = is_v ? vrs : krs;
+      const uint32_t off = d0 < p.D ? (kt + (uint32_t)key) * rs + (uint32_t)d0 * 4u : kBufferOff;
+      if (is_v) {
+        reg[i][0] = buffer_load16(rv, off, 0);
+        reg[i][1] = buffer_load16(rv, off + 16u, 0);
+      } else {
+        reg[i][0] = buffer_load16(rk, off, 0);
+        reg[i][1] = buffer_load16(rk, off + 16u, 0);
+      }
+    });
+  };
+  auto sstore = [&](int buf) {
+    static_for<0, NCH>([&](auto I) {
+      constexpr int i = decltype(I)::value;
+      const int ci = tid + i * NT;
+      const bool is_v = wave * 64 + i * NT >= TCH;
+      const int cj = ci % TCH, key = cj / CPR, d0 = (cj % CPR) * 8;
+      float x[8];
+#pragma unroll
+      for (int t = 0; t < 8; ++t) x[t] = __uint_as_float(reg[i][t >> 2][t & 3]);
+      const Split3 s3 = split3_any(x);
+      bf16(*dst)[KT * KS] = is_v ? Vp[buf] : Kp[buf];
+      const int o = Tile::off(key, d0);
+      *reinterpret_cast<bf16x8*>(&dst[0][o]) = s3.h;
+      *reinterpret_cast<bf16x8*>(&dst[1][o]) = s3.m;
+      *reinterpret_cast<bf16x8*>(&dst[2][o]) = s3.l;
+    });
+  };
+  gload(k_begin);
+
+  // Q^T parts: lane (c, g) holds Q[row c][d = 16 kk + 8 g .. + 7]
+  Split3 qf[NKK];
+#pragma unroll
+  for (int kk = 0; kk < NKK; ++kk) {
+    const int d0 = 16 * kk + 8 * g;
+    float x[8];
+    const bool ok = row_ok && d0 < p.D;
+    const float* src = Q + (int64_t)(row_ok ? my_row : p.q_start) * p.qs[2] + (d0 < p.D ? d0 : 0);
+    const f32x4 a = *reinterpret_cast<const f32x4*>(src), b = *reinterpret_cast<const f32x4*>(src + 4);
+#pragma unroll
+    for (int t = 0; t < 8; ++t) x[t] = ok ? (t < 4 ? a[t & 3] : b[t & 3]) : 0.f;
+    qf[kk] = split3_any(x);
+  }
+
+  // lane offsets: row fragments of K (row swap23(c), chunk g + 2 kk), transposing reads of V
+  const int tr_row = 8 * (lane >> 5) + ((lane & 15) >> 2);
+  const int tr_col = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+  int o_row[NKK], o_tr[NDT][2];
+#pragma unroll
+  for (int kk = 0; kk < NKK; ++kk) o_row[kk] = Tile::off(swap23(c), g * 8 + kk * 16);
+#pragma unroll
+  for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) o_tr[dt][h] = Tile::off(tr_row + 4 * h, dt * 32 + tr_col);
+  auto tr_frag = [&](const bf16* plane, int j, int dt) __attribute__((always_inline)) {
+    const i16x4 lo = lds_read_tr16(plane + 16 * j * KS + o_tr[dt][0]);
+    const i16x4 hi4 = lds_read_tr16(plane + 16 * j * KS + o_tr[dt][1]);
+    const i16x8 both = {lo[0], lo[1], lo[2], lo[3], hi4[0], hi4[1], hi4[2], hi4[3]};
+    return __builtin_bit_cast(bf16x8, both);
+  };
+
+  f32x16 oacc[NDT];
+#pragma unroll
+  for (int dt = 0; dt < NDT; ++dt) oacc[dt] = f32x16{};
+  // lazy maximum, as in phase1_half_kernel: p stays at or below 2^kLazyTau
+  float m_run = kNegInf, m_true = kNegInf, z_lane = 0.f;
+  const float cs = p.scale_log2;
+  const bool bias_vec = HAS_BIAS && bias_rows_vectorizable(p.bias);
+  const int ntiles = (k_end - k_begin + KT - 1) / KT;
+
+  sstore(0);
+  __syncthreads();
+  for (int it = 0; it < ntiles; ++it) {
+    const int buf = it & 1, t0 = k_begin + it * KT;
+    const bool has_next = it + 1 < ntiles;
+    if (has_next) gload(t0 + KT);
+    if (!p.causal || t0 <= row0 + 31) {  // a causal wave whose rows all precede this stage adds nothing
+      f32x16 s = f32x16{};
+      {
+        bf16x8 kh[NKK];
+#pragma unroll
+        for (int kk = 0; kk < NKK; ++kk) {
+          kh[kk] = *reinterpret_cast<const bf16x8*>(&Kp[buf][0][o_row[kk]]);
+          const bf16x8 km = *reinterpret_cast<const bf16x8*>(&Kp[buf][1][o_row[kk]]);
+          const bf16x8 kl = *reinterpret_cast<const bf16x8*>(&Kp[buf][2][o_row[kk]]);
+          s = mma3_small(kh[kk], km, kl, qf[kk], s);
+        }
+#pragma unroll
+        for (int kk = 0; kk < NKK; ++kk) s = M::mma(kh[kk], qf[kk].h, s);
+      }
+      float mx = kNegInf;
+      if constexpr (HAS_BIAS) {
+        const int64_t roff = bi * p.bias.sb + hi * p.bias.sh + (int64_t)(row_ok ? my_row : p.q_start) * p.bias.sq;
+        float bv[16];
+        bias_keys16(p.bias, roff, t0 + 8 * g, k_end, bias_vec, bv);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int key = t0 + key_of_reg(r, g);
+          const bool ok = row_ok && key < k_end && (!p.causal || key <= my_row);
+          s[r] = ok ? fmaf(s[r], cs, bv[r] * p.bias_log2) : kNegInf;
+          mx = fmaxf(mx, s[r]);
+        }
+      } else {
+        if ((t0 + KT > k_end) || (p.causal && (t0 + KT - 1 > row0))) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int key = t0 + key_of_reg(r, g);
+            if (!(key < k_end && (!p.causal || key <= my_row))) s[r] = kNegInf;
+          }
+        }
+#pragma unroll
+        for (int r = 0; r < 16; r += 2) mx = fmaxf(fmaxf(mx, s[r]), s[r + 1]);
+      }
+      mx = wave_max_pair(mx);
+      const float m_tile = HAS_BIAS ? mx : mx * cs;
+      m_true = fmaxf(m_true, m_tile);
+      if (__any(m_tile > m_run + kLazyTau)) {
+        const float m_new = fmaxf(m_run, m_tile);
+        const float alpha = (m_run == kNegInf) ? 0.f : fast_exp2(m_run - m_new);
+        z_lane *= alpha;
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) oacc[dt][r] *= alpha;
+        m_run = m_new;
+      }
+      const float nm = (m_run == kNegInf) ? 0.f : -m_run;
+      float zs = 0.f;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float pr = HAS_BIAS ? fast_exp2(s[r] + nm) : fast_exp2(fmaf(s[r], cs, nm));
+        s[r] = pr;
+        zs += pr;
+      }
+      z_lane += zs;
+      Split3 pf[2];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        float x[8];
+#pragma unroll
+        for (int t = 0; t < 8; ++t) x[t] = s[j * 8 + t];
+        pf[j] = split3_reg(x);
+      }
+#pragma unroll
+      for (int dt = 0; dt < NDT; ++dt) {
+        f32x16 st = f32x16{};
+        bf16x8 vh[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          vh[j] = tr_frag(Vp[buf][0], j, dt);
+          const bf16x8 vm = tr_frag(Vp[buf][1], j, dt), vl = tr_frag(Vp[buf][2], j, dt);
+          st = mma3_small(vh[j], vm, vl, pf[j], st);
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j) st = M::mma(vh[j], pf[j].h, st);
+        oacc[dt] += st;
+      }
+    }
+    if (has_next) sstore(buf ^ 1);
+    __syncthreads();
+  }
+
+  const float z_raw = wave_sum_pair(z_lane);
+  if (!row_ok) return;
+  // renormalise to the exact row maximum (m_run <= m_true <= m_run + kLazyTau)
+  const float f = (m_true == kNegInf) ? 1.f : fast_exp2(m_run - m_true);
+  const float z = z_raw * f;
+  const int64_t ridx = ((int64_t)kb * p.BH + bh) * p.rows_pad + (my_row - p.q_start);
+  const int64_t orow = (int64_t)bh * p.N + my_row;
+  const int64_t ooff = bi * p.os[0] + hi * p.os[1] + (int64_t)my_row * p.os[2];
+  if (g == 0) emit_state(p, ridx, orow, m_true, z);
+#pragma unroll
+  for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+    for (int q4 = 0; q4 < 4; ++q4) {
+      const int d = dt * 32 + q4 * 8 + 4 * g;
+      if (d < p.D)
+        emit4<float>(p, ridx, ooff, d, z, oacc[dt][4 * q4] * f, oacc[dt][4 * q4 + 1] * f, oacc[dt][4 * q4 + 2] * f,
+                     oacc[dt][4 * q4 + 3] * f);
+    }
+}
+
 // ------------------------------------------------------------------ Phase 1, fp16 / bf16
 // Each wave owns RT 32-row tiles (RT = 2 for head dims <= 64) so one K/V
 // fragment read from LDS feeds RT MFMAs.  K and V are staged row-major with
@@ -394,8 +650,6 @@ __global__ __launch_bounds__(64 * WAVES) void phase1_kernel(const Phase1Params p
 // -m_run (the MFMA's accumulator input, a register set refreshed only when the lazy max
 // moves), so its output is already score - m_run and p = exp2 of it, with no per-score
 // scale-and-subtract.
-constexpr float kLazyTau = 8.0f;
-constexpr float kLazySum = 256.0f;  // 2^kLazyTau
 
 // PV32 (fp16 inputs with fp32 summaries): the P.V product takes p unrounded, as the reference's
 // summary kernel does under SUMMARY_DOT_FP32 (attention_parallel_scan.py:701, :902;
@@ -1575,11 +1829,39 @@ static hipError_t launch1h_d(const Phase1Params& p, int block_m, hipStream_t st)
   }
 }
 
+template <int DP, int W, bool B>
+static hipError_t launch1x3(const Phase1Params& p, hipStream_t st) {
+  const dim3 grid((p.q_len + 32 * W - 1) / (32 * W), p.BH, p.P);
+  hipLaunchKernelGGL((phase1_x3_kernel<DP, W, B>), grid, dim3(64 * W), 0, st, p);
+  return hipGetLastError();
+}
+
+// Waves of the fp32 fold.  64-row blocks: 2 (head dims above 64 keep the fp32 MFMA, whose LDS leaves
+// room for several of these small work-groups: B64 H8 N64 d128 0.023 against 0.032 ms).  Otherwise 8
+// waves (256 rows), whose stage is split once for twice the rows, where the 256-row work-groups still
+// fill the chip (one per CU) in no more rounds than the 128-row ones (two per CU) and, for a causal
+// call, whole row blocks make up a partition (its longest-first order): forward d64 16K 2.92 -> 2.72
+// ms, 4K 0.200 -> 0.187, B8 H3 N1025 0.0562 -> 0.0539, causal 4K 0.121 -> 0.115; but B2 H8 N4097 with two
+// partitions (544 work-groups, a third round for 32) 0.456 -> 0.493, B4 H12 N577 0.040 -> 0.060 and
+// causal B1 H3 N5000 (640-key partitions) 0.081 -> 0.094 stay on 4.  Head dims above 64: one wave per
+// SIMD at 4 waves, two at 8 (4K 0.449 -> 0.343 ms); at most 256 rows or fewer than 128 work-groups of
+// 256 keep 4 there (B2 H3 N197 0.017 against 0.021 ms).
 template <int DP>
 static hipError_t launch1_f32_wb(const Phase1Params& p, int block_m, hipStream_t st) {
   const bool b = p.bias.ptr != nullptr;
-  if (block_m == 64) return b ? launch1<float, DP, 2, true>(p, st) : launch1<float, DP, 2, false>(p, st);
-  return b ? launch1<float, DP, 4, true>(p, st) : launch1<float, DP, 4, false>(p, st);
+  if (block_m == 64) {
+    if constexpr (DP == 128) {
+      return b ? launch1<float, DP, 2, true>(p, st) : launch1<float, DP, 2, false>(p, st);
+    } else {
+      return b ? launch1x3<DP, 2, true>(p, st) : launch1x3<DP, 2, false>(p, st);
+    }
+  }
+  if constexpr (DP >= 64) {
+    const int64_t w4 = (int64_t)((p.q_len + 127) / 128) * p.BH * p.P, w8 = (int64_t)((p.q_len + 255) / 256) * p.BH * p.P;
+    const bool fills = w8 >= 192 && (w8 + 255) / 256 <= (w4 + 511) / 512 && (!p.causal || p.part_len % 256 == 0);
+    if (DP == 128 ? p.q_len > 256 && w8 >= 128 : fills) return b ? launch1x3<DP, 8, true>(p, st) : launch1x3<DP, 8, false>(p, st);
+  }
+  return b ? launch1x3<DP, 4, true>(p, st) : launch1x3<DP, 4, false>(p, st);
 }
 
 hipError_t launch_phase1(const Phase1Params& p, int dtype, int block_m, hipStream_t st) {

@@ -138,7 +138,14 @@ int bwd_splits(int dtype, int dp, int64_t bh, int64_t n, bool bias, bool causal)
 
 // stage < 0: preprocess, dq and dk/dv; 0: preprocess only; 1: dq only; 2: dk/dv only.
 hipError_t launch_bwd(const BwdParams& p, int dtype, int stage, hipStream_t stream);
+hipError_t launch_bwd_f32(const BwdParams& p, int stage, hipStream_t stream);
 hipError_t launch_row_stats(const BwdParams& p, float* row_m, float* row_z, int dtype, hipStream_t stream);
+// The whole backward of a sequence of at most 64 rows in one launch (elsa_bwd_short.hip).  ds_mode 0:
+// no dS; 1: dS of every (batch, head) to p.ds_out, [BH][N][N]; 2: dS summed over the batch, one partial
+// [H][N][N] to p.ds_out for each of bwd_short_groups ranges of it.
+bool bwd_short_takes(int dtype, int n, int dp);
+int bwd_short_groups(int batch, int heads);
+hipError_t launch_bwd_short(const BwdParams& p, int dtype, int ds_mode, hipStream_t stream);
 // Number of ranges the dbias reduction over broadcast (b, h) pairs is cut into (1 = direct).
 int dbias_splits(int N, int batch, int heads, int bias_batch, int bias_heads);
 // part: nsplit * bias_batch * bias_heads * N * N floats of scratch when nsplit > 1.
@@ -153,6 +160,8 @@ hipError_t launch_debug_mfma_rate(int variant, const void* src, float* out, int 
 int dbias_sum_splits(int B, int H, int bias_batch, int bias_heads);
 hipError_t launch_dbias_sum(const float* ds, float* dbias, int B, int H, int N, int bias_batch, int bias_heads,
                             float* part, hipStream_t stream);
+// dbias[e] = sum over split < nsplit of part[split * n + e], in a fixed order
+hipError_t launch_dbias_reduce(const float* part, float* dbias, int nsplit, int64_t n, hipStream_t stream);
 // n floats of zeros (a kernel, so that graph capture records no memset node)
 hipError_t launch_zero_fill(float* dst, int64_t n, hipStream_t stream);
 

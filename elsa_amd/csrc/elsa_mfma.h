@@ -4,7 +4,8 @@
 // matrix cores:
 //   fp16 : v_mfma_f32_32x32x16_f16   (A, B: 8 halves per lane, C/D: 16 floats)
 //   bf16 : v_mfma_f32_32x32x16_bf16  (A, B: 8 bf16 per lane,  C/D: 16 floats)
-//   fp32 : v_mfma_f32_32x32x2_f32    (A, B: 1 float per lane,  C/D: 16 floats)
+//   fp32 : v_mfma_f32_32x32x2_f32    (A, B: 1 float per lane,  C/D: 16 floats) in the row stats,
+//          dbias and 64-row D > 64 folds; three bf16 parts per operand (Split3) in the others
 //
 // Operand layout (lane l, c = l % 32, g = l / 32, item t < KP):
 //   A[i][k] : lane with c == i holds k = g*KP + t        (row of A per lane)
@@ -79,6 +80,64 @@ __device__ __host__ constexpr inline int swap23(int i) {
 __device__ __host__ constexpr inline int key_of_reg(int r, int g) { return 16 * (r >> 3) + 8 * g + (r & 7); }
 
 __device__ inline float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
+
+// fp32 operands on the bf16 matrix cores: x = h + m + l with h, m and l bf16 (8 + 8 + 8 significant
+// bits), and a product of two such sums as the six partial products of order 2^-16 and above,
+//   x y ~ h h' + (h m' + m h') + (m m' + h l' + l h'),
+// each exact in the MFMA and summed in fp32.  The dropped ones (m l', l m', l l') are below 2^-23 of
+// |x y| (2^-26 on average, of either sign): less than one fp32 rounding.  Six v_mfma_f32_32x32x16_bf16
+// (8 passes each) take 48 passes where the eight v_mfma_f32_32x32x2_f32 (16 passes each) of the same
+// 16-long contraction take 128.
+struct Split3 {
+  bf16x8 h, m, l;
+};
+__device__ inline bf16x8 to_bf16x8(const float (&x)[8]) {
+  bf16x8 r;
+#pragma unroll
+  for (int t = 0; t < 8; ++t) r[t] = static_cast<bf16>(x[t]);
+  return r;
+}
+// (no contraction: x is the rounded fp32 value whatever else the caller does with it)
+// finite values well below the fp32 range (probabilities, dS): h, m and l each rounded to nearest
+__device__ inline Split3 split3_reg(const float (&x)[8]) {
+#pragma clang fp contract(off)
+  Split3 o;
+  float r[8];
+  o.h = to_bf16x8(x);
+#pragma unroll
+  for (int t = 0; t < 8; ++t) r[t] = x[t] - static_cast<float>(o.h[t]);
+  o.m = to_bf16x8(r);
+#pragma unroll
+  for (int t = 0; t < 8; ++t) r[t] -= static_cast<float>(o.m[t]);
+  o.l = to_bf16x8(r);
+  return o;
+}
+// any input: h truncated, so that no finite value becomes infinite, and an infinity or NaN alone in h
+// (its m and l are 0, not infinity - infinity)
+__device__ inline Split3 split3_any(const float (&x)[8]) {
+#pragma clang fp contract(off)
+  Split3 o;
+  float r[8], h[8];
+#pragma unroll
+  for (int t = 0; t < 8; ++t) {
+    h[t] = __uint_as_float(__float_as_uint(x[t]) & 0xffff0000u);
+    r[t] = fabsf(x[t]) < __builtin_huge_valf() ? x[t] - h[t] : 0.f;
+  }
+  o.h = to_bf16x8(h);
+  o.m = to_bf16x8(r);
+#pragma unroll
+  for (int t = 0; t < 8; ++t) r[t] -= static_cast<float>(o.m[t]);
+  o.l = to_bf16x8(r);
+  return o;
+}
+// acc + a b without the leading product: the five smaller partial products, least first
+__device__ inline f32x16 mma3_small(const bf16x8& ah, const bf16x8& am, const bf16x8& al, const Split3& b, f32x16 acc) {
+  acc = Mfma<bf16>::mma(al, b.h, acc);
+  acc = Mfma<bf16>::mma(ah, b.l, acc);
+  acc = Mfma<bf16>::mma(am, b.m, acc);
+  acc = Mfma<bf16>::mma(am, b.h, acc);
+  return Mfma<bf16>::mma(ah, b.m, acc);
+}
 
 // Load KP elements (one MFMA operand fragment) from memory; `ok` false gives zeros.
 template <typename T>
@@ -205,6 +264,35 @@ __device__ inline WgCoord xcd_order_paired() {
   const int l = xcd * per + min(xcd, rem) + slot;
   const int gx = gridDim.x, gy = gridDim.y;
   return {l % gx, (l / gx) % gy, l / (gx * gy)};
+}
+// Causal backward grids (grid x = row or key block, y = head, z = range of a split), heaviest block
+// first over everything an XCD runs: the columns (head, range) are dealt to the XCDs whole when their
+// number is a multiple of 8, and an XCD's j-th work-group takes block rank j / C of its C columns.
+// The first 64 work-groups of an XCD start at once, two to each of its 32 CUs (the j-th and the
+// (j + 32)-th on one): the second layer is handed out lightest first, so that every CU gets about the
+// same work, and where it has only m < 32 work-groups the heaviest 32 - m of the first layer go to the CUs
+// that get no second one.  heavy_last: the block with the highest index has the most work.
+__device__ inline WgCoord causal_bwd_order(bool heavy_last) {
+  const int gx = gridDim.x, gy = gridDim.y, cols = gy * gridDim.z;
+  const int lin = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
+  int blk, col;
+  if (cols & 7) {
+    blk = lin / cols;
+    col = lin - blk * cols;
+  } else {
+    const int C = cols >> 3, per = gx * C, m = min(32, per - 32);
+    int slot = lin >> 3;
+    if (m > 0) {
+      if (slot < 32) {
+        slot = slot < m ? slot + 32 - m : slot - m;
+      } else if (slot < 32 + m) {
+        slot = 32 + (32 + m - 1 - slot);
+      }
+    }
+    blk = slot / C;
+    col = (lin & 7) * C + slot - blk * C;
+  }
+  return {heavy_last ? gx - 1 - blk : blk, col % gy, col / gy};
 }
 // Non-causal Phase 1 (grid x = row block, y = head, z = K partition) with the panels (head,
 // partition) dealt to the XCDs in turn, each panel whole: the dispatcher sends workgroup L to

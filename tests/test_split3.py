@@ -1,0 +1,53 @@
+"""CPU model of the fp32 kernels' products: x = h + m + l in bf16 parts and the six partial products of
+order 2^-16 and above (split3_any, split3_reg and mma3_small in elsa_mfma.h)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+
+def _bf16_rne(x):
+    u = np.asarray(x, np.float32).view(np.uint32).astype(np.uint64)
+    u = (u + 0x7FFF + ((u >> 16) & 1)) & 0xFFFF0000
+    return u.astype(np.uint32).view(np.float32)
+
+
+def _bf16_trunc(x):
+    return (np.asarray(x, np.float32).view(np.uint32) & np.uint32(0xFFFF0000)).view(np.float32)
+
+
+def _split(x, truncate_h):
+    h = _bf16_trunc(x) if truncate_h else _bf16_rne(x)
+    r = np.where(np.isfinite(x), x - np.where(np.isfinite(x), h, 0), 0).astype(np.float32)
+    m = _bf16_rne(r)
+    return h, m, _bf16_rne(r - m)
+
+
+@pytest.mark.parametrize("truncate_h", [True, False])
+def test_three_parts_hold_every_bit(truncate_h):
+    rng = np.random.default_rng(5)
+    x = (rng.standard_normal(200_000) * 2.0 ** rng.integers(-100, 100, 200_000)).astype(np.float32)
+    h, m, l = _split(x, truncate_h)
+    assert np.array_equal(h.astype(np.float64) + m + l, x.astype(np.float64))
+
+
+def test_infinities_and_the_largest_values_stay_in_the_first_part():
+    x = np.array([np.inf, -np.inf, np.finfo(np.float32).max, -np.finfo(np.float32).max, 0.0], np.float32)
+    h, m, l = _split(x, True)
+    assert np.array_equal(np.isinf(h), np.isinf(x))
+    assert not np.isnan(m).any() and not np.isnan(l).any()
+    fin = np.isfinite(x)
+    assert np.array_equal(h[fin].astype(np.float64) + m[fin] + l[fin], x[fin].astype(np.float64))
+
+
+@pytest.mark.parametrize("truncate_a,truncate_b", [(True, True), (True, False), (False, False)])
+def test_dropped_products_are_below_an_fp32_rounding(truncate_a, truncate_b):
+    rng = np.random.default_rng(6)
+    a, b = (rng.standard_normal(400_000).astype(np.float32) for _ in range(2))
+    ah, am, al = (t.astype(np.float64) for t in _split(a, truncate_a))
+    bh, bm, bl = (t.astype(np.float64) for t in _split(b, truncate_b))
+    kept = al * bh + ah * bl + am * bm + am * bh + ah * bm + ah * bh
+    err = np.abs(kept - a.astype(np.float64) * b) / np.abs(a.astype(np.float64) * b)
+    # |m| < 2^-7 |x| and |l| <= 2^-16 |x| (h truncated): m l' + l m' + l l' < 2 * 2^-23 + 2^-32
+    assert err.max() < 2.0 ** -22
+    assert np.sqrt((err ** 2).mean()) < 2.0 ** -24
