@@ -695,7 +695,7 @@ int elsa_bwd_dbias(const elsa_bwd_args* a, float* dbias, int32_t bias_batch, int
     // dS summed over the batch inside the backward, one partial per range of it (at most batch: they fit the
     // dS buffer), then over the ranges
     elsa::BwdParams p = bwd_params(a);
-    const int groups = elsa::bwd_short_groups(a->batch, a->heads);
+    const int groups = elsa::bwd_short_groups(a->dtype, p.dp, a->batch, a->heads);
     p.ds_out = groups > 1 ? ds : dbias;
     if ((e = elsa::launch_bwd_short(p, a->dtype, 2, st)) != hipSuccess) return hip_fail(e, "backward launch");
     if (groups == 1) return ELSA_OK;

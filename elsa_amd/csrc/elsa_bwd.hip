@@ -1272,7 +1272,8 @@ static hipError_t pre_launch(const BwdParams& p, hipStream_t st) {
 // workgroup, register budget capped for 2 waves per SIMD (measured on MI355X at
 // B1 H8 N16K d64: dq 1.36 ms / dk-dv 1.68 ms versus 2.27 / 2.76 ms with 64-wide
 // wave tiles at 1 wave per SIMD).  fp32 keeps the 32-wide kernels above.
-// Sequences of at most 64 rows at head dims up to 32 (Swin's 49-token windows): 2-wave
+// Single stages (elsa_bwd_stage; the whole backward is bwd_short_kernel) of
+// sequences of at most 64 rows at head dims up to 32 (Swin's 49-token windows): 2-wave
 // work-groups of 64 rows or keys, so that no wave of a work-group lies wholly past N (with 4
 // waves of 32, waves 2 and 3 only staged and waited).  The split backward never applies there
 // (bwd_splits).  Wider heads keep 4 waves: at D = 64 the 2-wave fp16/bf16 dK/dV kernel spills

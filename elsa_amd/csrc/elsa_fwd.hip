@@ -406,7 +406,7 @@ struct X3Tile {
 };
 
 template <int DP, int WAVES, bool HAS_BIAS>
-__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(DP >= 128 ? 1 : 2, 2)))
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(DP >= 128 ? 1 : 2, DP == 32 ? 8 : 2)))
 void phase1_x3_kernel(const Phase1Params p) {
   using Tile = X3Tile<DP>;
   using M = Mfma<bf16>;
@@ -657,9 +657,11 @@ void phase1_x3_kernel(const Phase1Params p) {
 // go through the fp16 MFMA (exact products, fp32 sums): p is carried to about 22 bits.
 //
 // 2 waves per SIMD, except the 1- and 2-wave variants at D >= 64 (sequences of at most 64
-// keys): their register staging of a whole 64-key stage does not fit that budget.
+// keys): their register staging of a whole 64-key stage does not fit that budget.  The one-tile D <= 32
+// variants run as many as their registers allow (3-5): on short windows the loads' latency is the time, and
+// more of them overlap (512 windows x 3 heads, N49, fp16 bias 0.0203 -> 0.0144 ms; 3 waves, 134 VGPRs).
 template <typename T, int DP, int RT, int WAVES, bool HAS_BIAS, bool PRE, bool PV32 = false, bool LD = false>
-__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu((WAVES <= 2 && DP >= 64) ? 1 : 2, 2)))
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu((WAVES <= 2 && DP >= 64) ? 1 : 2, DP == 32 && RT == 1 ? 8 : 2)))
 void phase1_half_kernel(const Phase1Params p) {
   static_assert(!(PRE && HAS_BIAS), "the prescaled fold has no bias");
   static_assert(!PV32 || (std::is_same<T, f16>::value && !PRE), "PV32 is the fp16 fold with fp32 summaries");

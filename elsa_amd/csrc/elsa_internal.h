@@ -144,7 +144,7 @@ hipError_t launch_row_stats(const BwdParams& p, float* row_m, float* row_z, int 
 // no dS; 1: dS of every (batch, head) to p.ds_out, [BH][N][N]; 2: dS summed over the batch, one partial
 // [H][N][N] to p.ds_out for each of bwd_short_groups ranges of it.
 bool bwd_short_takes(int dtype, int n, int dp);
-int bwd_short_groups(int batch, int heads);
+int bwd_short_groups(int dtype, int dp, int batch, int heads);
 hipError_t launch_bwd_short(const BwdParams& p, int dtype, int ds_mode, hipStream_t stream);
 // Number of ranges the dbias reduction over broadcast (b, h) pairs is cut into (1 = direct).
 int dbias_splits(int N, int batch, int heads, int bias_batch, int bias_heads);
