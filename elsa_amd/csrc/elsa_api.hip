@@ -435,9 +435,6 @@ elsa::BwdParams bwd_params(const elsa_bwd_args* a) {
   p.lse_lo = reinterpret_cast<float*>(base + 2 * align256(rows * 4));
   p.dp = elsa::pad_head_dim(a->head_dim);
   p.split = elsa::bwd_splits(a->dtype, p.dp, p.BH, p.N, a->bias.ptr != nullptr, a->is_causal != 0);
-  // 16-bit kernels: rows (dK/dV) or keys (dq) per range, whole 64-row stages; the fp32 ones deal their
-  // stages out in turn and every range holds a partial (split_len 1 makes the combine read them all)
-  p.split_len = a->dtype == ELSA_F32 ? 1 : p.split > 1 ? (int)((((int64_t)p.N + p.split - 1) / p.split + 63) / 64 * 64) : p.N;
   p.part = p.split > 1 ? reinterpret_cast<float*>(base + 3 * align256(rows * 4)) : nullptr;
   p.part_stride = (int64_t)(align256((size_t)p.split * rows * p.dp * 4) / 4);
   const int H = a->heads, N = a->seq_len, D = a->head_dim;

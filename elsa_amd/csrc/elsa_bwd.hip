@@ -186,10 +186,7 @@ void bwd_dq_half_kernel(const BwdParams p) {
 
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 31,
             g = lane >> 5;
-  // causal: the work of a row block grows with its index; each XCD takes its range of
-  // row blocks heaviest first (paired heavy with light where the grid fits in one round)
-  WgCoord wg = (p.causal && WAVES == 4) ? xcd_order_paired() : xcd_order();
-  if (p.causal) wg.x = (int)gridDim.x - 1 - wg.x;
+  const WgCoord wg = p.causal ? causal_bwd_order(true, WAVES == 4) : xcd_order();
   const int bh = wg.y;
   const int wg_row0 = wg.x * BM;
   const int wg_last = min(p.N, wg_row0 + BM) - 1;
@@ -252,15 +249,11 @@ void bwd_dq_half_kernel(const BwdParams p) {
     live[rt] = ok && lse[rt] < __builtin_huge_valf();
   }
   const int k_end = p.causal ? wg_last + 1 : p.N;
-  // split (the 4-wave one-tile kernel only): this work-group's keys [k_lo, k_hi), whole 64-key
-  // stages (one range when unsplit).  D = 128 never splits (bwd_splits) but keeps these run-time
-  // bounds: with constant ones its register allocation spilled (20 bytes per lane, 468 biased;
-  // 16K dq 1.698 -> 1.653 ms without)
-  const int k_lo = CAN_SPLIT ? min(k_end, wg.z * p.split_len) : 0;
-  const int k_hi = CAN_SPLIT ? min(k_end, k_lo + p.split_len) : k_end;
-  // a causal key range past this row block's last row adds nothing: no partial is written, and
-  // the combine (bwd_combine_kernel, kind 1) skips the same ranges
-  if (CAN_SPLIT && p.split > 1 && p.causal && k_lo >= k_hi) return;
+  // split (the 4-wave one-tile kernel only; 1 otherwise): work-group z takes the 64-key stages z, z + split,
+  // ..., so that the ranges differ by at most one stage, under a causal mask too; one without a stage
+  // writes zeros.  D = 128 never splits (bwd_splits) but keeps these run-time bounds: with constant
+  // ones its register allocation spilled (20 bytes per lane, 468 biased; 16K dq 1.698 -> 1.653 ms without)
+  const int k_lo = CAN_SPLIT ? wg.z * KT : 0, k_step = CAN_SPLIT ? p.split * KT : KT;
   // -D of this lane's row: the dP^T product starts from it and yields dP - D directly.  The
   // 16 registers per row tile of that constant would spill in the bias, D = 128 and two-tile
   // variants, which subtract D from each score instead.
@@ -375,7 +368,7 @@ static_for<0, NCH>([&](auto I) {
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt) acc[rt][dt] = f32x16{};
 
-  const int ntiles = (k_hi - k_lo + KT - 1) / KT;
+  const int ntiles = k_end > k_lo ? (k_end - k_lo + k_step - 1) / k_step : 0;
   // stage keys [t0, t0 + KT) from LDS buffer buf into the dQ accumulators
   auto compute = [&](int t0, const T* ks, const T* vs) __attribute__((always_inline)) {
     if (!p.causal || t0 <= row0 + ROWS_W - 1) {
@@ -453,14 +446,14 @@ static_for<0, NCH>([&](auto I) {
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     for (int it = 0; it < ntiles; it += 2) {
-      const int t0 = k_lo + it * KT;
-      if (it + 1 < ntiles) ldload(t0 + KT, Ks1, Vs1);
+      const int t0 = k_lo + it * k_step;
+      if (it + 1 < ntiles) ldload(t0 + k_step, Ks1, Vs1);
       compute(t0, Ks[0], Vs[0]);
       __builtin_amdgcn_s_waitcnt(0);
       __syncthreads();
       if (it + 1 < ntiles) {
-        if (it + 2 < ntiles) ldload(t0 + 2 * KT, Ks[0], Vs[0]);
-        compute(t0 + KT, Ks1, Vs1);
+        if (it + 2 < ntiles) ldload(t0 + 2 * k_step, Ks[0], Vs[0]);
+        compute(t0 + k_step, Ks1, Vs1);
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
       }
@@ -472,12 +465,12 @@ static_for<0, NCH>([&](auto I) {
     // two-tile variant (255 VGPRs with one set)
     gload(k_lo, S0);
     sstore(0, S0);
-    if (ntiles > 1) gload(k_lo + KT, S1);
+    if (ntiles > 1) gload(k_lo + k_step, S1);
     __syncthreads();
     auto step = [&](int it, auto NEXT, auto FREE) __attribute__((always_inline)) {
       const int buf = it & 1;
-      const int t0 = k_lo + it * KT;
-      if (it + 2 < ntiles) gload(t0 + 2 * KT, FREE);
+      const int t0 = k_lo + it * k_step;
+      if (it + 2 < ntiles) gload(t0 + 2 * k_step, FREE);
       compute(t0, Ks[buf], Vs[buf]);
       if (it + 1 < ntiles) sstore(buf ^ 1, NEXT);
       __syncthreads();
@@ -492,9 +485,9 @@ static_for<0, NCH>([&](auto I) {
     __syncthreads();
     for (int it = 0; it < ntiles; ++it) {
       const int buf = it & 1;
-      const int t0 = k_lo + it * KT;
+      const int t0 = k_lo + it * k_step;
       const bool has_next = it + 1 < ntiles;
-      if (has_next) gload(t0 + KT, S0);
+      if (has_next) gload(t0 + k_step, S0);
       compute(t0, Ks[buf], Vs[buf]);
       if (has_next) sstore(buf ^ 1, S0);
       __syncthreads();
@@ -564,9 +557,7 @@ void bwd_dkdv_half_kernel(const BwdParams p) {
 
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 31,
             g = lane >> 5;
-  // causal: the work of a key block shrinks with its index (heaviest first; paired heavy with
-  // light where the grid fits in one round)
-  const WgCoord wg = (p.causal && WAVES == 4) ? xcd_order_paired() : xcd_order();
+  const WgCoord wg = p.causal ? causal_bwd_order(false, WAVES == 4) : xcd_order();
   const int bh = wg.y;
   const int wg_key0 = wg.x * BN;
   const int key0 = wg_key0 + wave * KEYS_W;
@@ -705,15 +696,12 @@ static_for<0, NCH>([&](auto I) {
     }
   };
 
-  // split (the 4-wave one-tile kernel only): this work-group's rows [r_lo, r_hi), whole 64-row
-  // stages (one range when unsplit)
+  // split (the 4-wave one-tile kernel only), as in the dq kernel: the row stages z, z + split, ... from the
+  // causal key block's first one on
   constexpr bool CAN_SPLIT = KRT == 1 && WAVES == 4 && !HAS_BIAS && DP <= 64;
-  const int r_lo = max(p.causal ? (wg_key0 / RTS) * RTS : 0, CAN_SPLIT ? wg.z * p.split_len : 0);
-  const int r_hi = CAN_SPLIT ? min(p.N, wg.z * p.split_len + p.split_len) : p.N;
-  const int ntiles = r_hi > r_lo ? (r_hi - r_lo + RTS - 1) / RTS : 0;
-  // a causal row range before this key block's first row adds nothing: no partials are written,
-  // and the combine (bwd_combine_kernel, kind 2) skips the same ranges
-  if (CAN_SPLIT && p.split > 1 && p.causal && ntiles == 0) return;
+  const int r_lo = (p.causal ? (wg_key0 / RTS) * RTS : 0) + (CAN_SPLIT ? wg.z * RTS : 0);
+  const int r_step = CAN_SPLIT ? p.split * RTS : RTS;
+  const int ntiles = p.N > r_lo ? (p.N - r_lo + r_step - 1) / r_step : 0;
   // stage rows [t0, t0 + RTS) from LDS buffer buf into the dK / dV accumulators
   auto compute = [&](int buf, int t0, const T* qs, const T* gs) __attribute__((always_inline)) {
     if (!p.causal || t0 + RTS - 1 >= key0) {
@@ -835,15 +823,15 @@ static_for<0, NCH>([&](auto I) {
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     for (int it = 0; it < ntiles; it += 2) {
-      const int t0 = r_lo + it * RTS;
-      if (it + 1 < ntiles) ldload(t0 + RTS, Qs1, Gs1);
+      const int t0 = r_lo + it * r_step;
+      if (it + 1 < ntiles) ldload(t0 + r_step, Qs1, Gs1);
       compute(0, t0, Qs[0], Gs[0]);
       if (it + 1 < ntiles) ldstore(1);
       __builtin_amdgcn_s_waitcnt(0);
       __syncthreads();
       if (it + 1 < ntiles) {
-        if (it + 2 < ntiles) ldload(t0 + 2 * RTS, Qs[0], Gs[0]);
-        compute(1, t0 + RTS, Qs1, Gs1);
+        if (it + 2 < ntiles) ldload(t0 + 2 * r_step, Qs[0], Gs[0]);
+        compute(1, t0 + r_step, Qs1, Gs1);
         if (it + 2 < ntiles) ldstore(0);
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
@@ -854,12 +842,12 @@ static_for<0, NCH>([&](auto I) {
   // left, while stage it + 1 waits in the other one for the end of this stage
   gload(r_lo, S0);
   sstore(0, S0);
-  if (ntiles > 1) gload(r_lo + RTS, S1);
+  if (ntiles > 1) gload(r_lo + r_step, S1);
   __syncthreads();
   auto step = [&](int it, auto NEXT, auto FREE) __attribute__((always_inline)) {
     const int buf = it & 1;
-    const int t0 = r_lo + it * RTS;
-    if (it + 2 < ntiles) gload(t0 + 2 * RTS, FREE);
+    const int t0 = r_lo + it * r_step;
+    if (it + 2 < ntiles) gload(t0 + 2 * r_step, FREE);
     compute(buf, t0, Qs[buf], Gs[buf]);
     if (it + 1 < ntiles) sstore(buf ^ 1, NEXT);
     __syncthreads();
@@ -1173,6 +1161,26 @@ static int f32_ragged_splits(int dp, int64_t bh, int64_t n) {
   return best;
 }
 
+// The same for fp16 / bf16 at d64 without a causal mask, between 257 and 1024 4-wave work-groups: a CU's k
+// work-groups take floor(k / 2) rounds of two together, and an odd one alone 0.52 of a round; a round is the
+// keys of a range + 200, the combine 65 + 0.0031 x work-groups x head dim per range, in keys (0.061 us).
+// Split only where it saves a tenth (the unsplit kernels have 8-wave variants).  Whole backward ms, bf16: B2
+// H8 N4097 (528 work-groups) 0.420 -> 0.326 (1 -> 3 ranges), B1 H8 N5000 0.289 -> 0.236 (3), B3 H8 N3000
+// 0.313 -> 0.264 (2), B1 H8 N6000 0.348 -> 0.311 (2); B8 H3 N4097 (0.438 against 0.456 with 2), B8 H3 N2305
+// (0.153, 0.175) and B4 H8 N1500 (0.101, 0.114) stay at 1.
+static int half_ragged_splits(int64_t bh, int64_t n) {
+  const int64_t w4 = bh * ((n + 127) / 128);
+  auto cost = [&](int s) {
+    const int64_t k = (w4 * s + 255) / 256, len = ((n + s - 1) / s + 63) / 64 * 64;
+    return ((double)(k / 2) + (k % 2 ? 0.52 : 0.0)) * (double)(len + 200) +
+           (s > 1 ? 65 + 0.0031 * (double)(w4 * 64) * s : 0.0);
+  };
+  int best = 1;
+  for (int s = 2; s <= 8 && n / s >= 256; ++s)
+    if (cost(s) < cost(best)) best = s;
+  return cost(best) < 0.9 * cost(1) ? best : 1;
+}
+
 int bwd_splits(int dtype, int dp, int64_t bh, int64_t n, bool bias, bool causal) {
   if (bias || (dp > 64 && dtype != ELSA_F32)) return 1;
   if (dp > 64) return f32_ragged_splits(dp, bh, n);
@@ -1191,6 +1199,7 @@ int bwd_splits(int dtype, int dp, int64_t bh, int64_t n, bool bias, bool causal)
   // 0.800 -> 0.723 (2 -> 4).  fp16 went both ways (B2 H8 N2049 0.103 -> 0.085 ms, but B1 H12 N2048
   // 0.076 -> 0.083 and B1 H8 N5000 0.169 -> 0.177), so 16-bit calls count every work-group.
   if (dtype == ELSA_F32 && !causal && dp == 64 && wgs > 256) return f32_ragged_splits(dp, bh, n);
+  if (dtype != ELSA_F32 && !causal && dp == 64 && wgs > 256 && wgs <= 1024) return half_ragged_splits(bh, n);
   const int64_t min_range = dtype == ELSA_F32 ? 64 : 256;
   const bool live_only = causal && dtype == ELSA_F32 && wgs <= 512;
   int s = 1;
@@ -1202,15 +1211,9 @@ int bwd_splits(int dtype, int dp, int64_t bh, int64_t n, bool bias, bool causal)
 
 // out[b, h, n, d] = scale * sum over the split ranges of part[z][b*H + h][n][d], 4 head-dim
 // elements per thread (head dims are multiples of 8); grid y picks one of up to three such sums.
-// kind 0 sums every range.  Causal calls skip the ranges whose work-groups wrote nothing (the
-// split kernels are the 4-wave ones: 128 rows or keys per work-group):
-//   kind 1 (dQ of row n): key ranges z with z * split_len >= k_end = min(N, 128 * (n / 128 + 1));
-//   kind 2 (dK, dV of key n): row ranges z with (z + 1) * split_len <= 128 * (n / 128).
-// Every kind skips ranges that start at or past N.  Those ranges would add zeros, so the sums are
-// the same up to the sign of a zero.
 template <typename T>
 __global__ __launch_bounds__(256) void bwd_combine_kernel(CombineOut c0, CombineOut c1, CombineOut c2, int split,
-                                                          int split_len, int64_t sstride, int H, int N, int D,
+                                                          int64_t sstride, int H, int N, int D,
                                                           int dp) {
   const CombineOut& cj = blockIdx.y == 0 ? c0 : (blockIdx.y == 1 ? c1 : c2);
   const float* __restrict__ part = cj.part;
@@ -1223,17 +1226,9 @@ __global__ __launch_bounds__(256) void bwd_combine_kernel(CombineOut c0, Combine
   if (row >= sstride / dp) return;
   const int d = (int)(i - row * c4) * 4;
   const int64_t bh = row / N, n = row - bh * N;
-  // ranges that start at or past N (split_len is rounded up to whole stages) hold nothing either
-  int z_lo = 0, z_hi = min(split, (N + split_len - 1) / split_len);
-  if (cj.kind == 1) {
-    const int k_end = min(N, 128 * ((int)n / 128 + 1));
-    z_hi = min(z_hi, (k_end + split_len - 1) / split_len);
-  } else if (cj.kind == 2) {
-    z_lo = 128 * ((int)n / 128) / split_len;  // < z_hi: 128 * (n / 128) <= n < N
-  }
   const float* src = part + row * dp + d;
-  f32x4 acc = *reinterpret_cast<const f32x4*>(src + z_lo * sstride);
-  for (int z = z_lo + 1; z < z_hi; ++z) {
+  f32x4 acc = *reinterpret_cast<const f32x4*>(src);
+  for (int z = 1; z < split; ++z) {
     const f32x4 v = *reinterpret_cast<const f32x4*>(src + z * sstride);
     acc[0] += v[0];
     acc[1] += v[1];
@@ -1252,7 +1247,7 @@ static hipError_t combine_launch(const BwdParams& p, const CombineOut* c, int n,
   const int64_t rows = (int64_t)p.BH * p.N;
   const int64_t threads = rows * (p.D / 4);
   hipLaunchKernelGGL(bwd_combine_kernel<T>, dim3((unsigned)((threads + 255) / 256), (unsigned)n), dim3(256), 0, st,
-                     c[0], c[n > 1 ? 1 : 0], c[n > 2 ? 2 : 0], p.split, p.split_len, rows * p.dp, p.H, p.N, p.D,
+                     c[0], c[n > 1 ? 1 : 0], c[n > 2 ? 2 : 0], p.split, rows * p.dp, p.H, p.N, p.D,
                      p.dp);
   return hipGetLastError();
 }
@@ -1320,10 +1315,9 @@ static hipError_t bwd_launch3(const BwdParams& p, int stage, hipStream_t st) {
       // an under-filled grid (short sequences, few heads): the key (dq) or row (dK/dV) loop cut
       // into p.split ranges over grid z, fp32 partials summed by a combine launch
       const dim3 gs(grid.x, grid.y, (unsigned)p.split);
-      const int kq = p.causal ? 1 : 0, kkv = p.causal ? 2 : 0;
-      const CombineOut cq{p.part, p.dq, {p.dqs[0], p.dqs[1], p.dqs[2]}, p.scale, kq};
-      const CombineOut ck{p.part + p.part_stride, p.dk, {p.dks[0], p.dks[1], p.dks[2]}, p.scale, kkv};
-      const CombineOut cv{p.part + 2 * p.part_stride, p.dv, {p.dvs[0], p.dvs[1], p.dvs[2]}, 1.f, kkv};
+      const CombineOut cq{p.part, p.dq, {p.dqs[0], p.dqs[1], p.dqs[2]}, p.scale};
+      const CombineOut ck{p.part + p.part_stride, p.dk, {p.dks[0], p.dks[1], p.dks[2]}, p.scale};
+      const CombineOut cv{p.part + 2 * p.part_stride, p.dv, {p.dvs[0], p.dvs[1], p.dvs[2]}, 1.f};
       if (stage < 0 || stage == 1) {
         if (ld_kv) {
           hipLaunchKernelGGL((bwd_dq_half_kernel<T, DP, R, W, false, DP == 64>), gs, dim3(64 * W), 0, st, p);

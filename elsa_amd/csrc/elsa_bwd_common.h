@@ -153,7 +153,6 @@ struct CombineOut {
   void* out;
   int64_t os[3];
   float scale;
-  int kind;
 };
 // one launch for up to three sums (n = 1, 2 or 3 of c[0..2]) into fp32 outputs
 hipError_t combine_launch_f32(const BwdParams& p, const CombineOut* c, int n, hipStream_t st);

@@ -89,7 +89,7 @@ void bwd_dq_x3_kernel(const BwdParams p) {
 
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 31,
             g = lane >> 5;
-  const WgCoord wg = p.causal ? causal_bwd_order(true) : xcd_order();
+  const WgCoord wg = p.causal ? causal_bwd_order(true, WAVES <= 4 && DP <= 64) : xcd_order();
   const int bh = wg.y;
   const int wg_row0 = wg.x * BM;
   const int wg_last = min(p.N, wg_row0 + BM) - 1;
@@ -231,7 +231,7 @@ void bwd_dkdv_x3_kernel(const BwdParams p) {
 
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 31,
             g = lane >> 5;
-  const WgCoord wg = p.causal ? causal_bwd_order(false) : xcd_order();
+  const WgCoord wg = p.causal ? causal_bwd_order(false, WAVES <= 4 && DP == 32) : xcd_order();
   const int bh = wg.y;
   const int wg_key0 = wg.x * BN;
   const int key0 = wg_key0 + wave * 32, my_key = key0 + c;
@@ -418,9 +418,9 @@ template <int DP, bool B>
 static hipError_t bwd_f32_b(const BwdParams& p, int stage, hipStream_t st) {
   hipError_t e = hipSuccess;
   const CombineOut all[3] = {
-      {p.part, p.dq, {p.dqs[0], p.dqs[1], p.dqs[2]}, p.scale, 0},
-      {p.part + p.part_stride, p.dk, {p.dks[0], p.dks[1], p.dks[2]}, p.scale, 0},
-      {p.part + 2 * p.part_stride, p.dv, {p.dvs[0], p.dvs[1], p.dvs[2]}, 1.f, 0}};
+      {p.part, p.dq, {p.dqs[0], p.dqs[1], p.dqs[2]}, p.scale},
+      {p.part + p.part_stride, p.dk, {p.dks[0], p.dks[1], p.dks[2]}, p.scale},
+      {p.part + 2 * p.part_stride, p.dv, {p.dvs[0], p.dvs[1], p.dvs[2]}, 1.f}};
   // the key (dq) and row (dK/dV) loops split over grid z for under-filled grids
   const unsigned gz = p.split > 1 ? p.split : 1;
   const dim3 g2((p.N + 63) / 64, p.BH, gz), g4((p.N + 127) / 128, p.BH, gz), g8((p.N + 255) / 256, p.BH, gz);

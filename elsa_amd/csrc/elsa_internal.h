@@ -118,10 +118,10 @@ struct BwdParams {
   float scale_log2;  // scale * log2(e)
   // element strides (batch, head, row) of q, k, v, out, dout and of dq, dk, dv
   int64_t qs[3], ks[3], vs[3], os[3], gs[3], dqs[3], dks[3], dvs[3];
-  // split > 1 (bwd_splits): the 4-wave dq and dK/dV kernels cut their key (dq) or row (dK/dV)
-  // loop into `split` ranges of split_len (a multiple of 64; of 32 for fp32) over grid z, and write unscaled fp32
-  // partials, [split][BH][N][dp] each for dq, dK and dV from part on; a combine kernel sums them
-  int split, split_len, dp;
+  // split > 1 (bwd_splits): the dq and dK/dV kernels deal the stages of their key (dq) or row (dK/dV) loop
+  // out over `split` work-groups (grid z) in turn, and write unscaled fp32 partials, [split][BH][N][dp] each
+  // for dq, dK and dV from part on; a combine kernel sums them
+  int split, dp;
   float* part;
   int64_t part_stride;  // floats from the dq partials to the dK ones and from those to the dV ones
 };
@@ -129,11 +129,8 @@ struct BwdParams {
 // Ranges the backward (fp16, bf16 and fp32) cuts its loops into when its unsplit grid (128 rows or
 // keys per work-group) leaves the chip under-filled: doubled from 1 while the doubled grid stays
 // within 512 work-groups (causal fp32: 512 that hold work) and n / (2 * split) is at least 256 (64
-// for fp32).  Each range is
-// split_len = ceil(n / split) rounded up to whole stages (64 rows; 32 for fp32), so the last one can be shorter
-// (B1 H4 N2049: 576, 576, 576 and 321 rows) or start past n (B1 H2 N2049: 8 ranges of 320, the last
-// from 2240); the launch lasts as long as the longest range,
-// which no choice of whole-stage ranges makes shorter.  Biased calls and head dims above 64 keep 1.
+// for fp32); ragged fp32 grids and fp32 at D = 128 by the rounds they take.  Biased calls and 16-bit head
+// dims above 64 keep 1.
 int bwd_splits(int dtype, int dp, int64_t bh, int64_t n, bool bias, bool causal);
 
 // stage < 0: preprocess, dq and dk/dv; 0: preprocess only; 1: dq only; 2: dk/dv only.

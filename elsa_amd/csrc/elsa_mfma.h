@@ -250,29 +250,15 @@ __device__ inline WgCoord xcd_order() {
   const int gx = gridDim.x, gy = gridDim.y, l = xcd_linear();
   return {l % gx, (l / gx) % gy, l / (gx * gy)};
 }
-// xcd_order for causal backward grids that fit the chip in one round of two work-groups per CU
-// (more than 256, at most 512 work-groups of the 4-wave kernels), whose work-groups are numbered
-// heaviest first within each head: the second half of each XCD's work-groups comes lightest
-// first, so that the CU that takes the j-th work-group of the first half also takes the j-th
-// lightest, and every CU gets about the same work.
-__device__ inline WgCoord xcd_order_paired() {
-  const int n = gridDim.x * gridDim.y * gridDim.z;
-  const int lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-  const int per = n >> 3, rem = n & 7, xcd = lin & 7;
-  int slot = lin >> 3;
-  if (n > 256 && n <= 512 && rem == 0 && (per & 1) == 0 && slot >= per / 2) slot = per + per / 2 - 1 - slot;
-  const int l = xcd * per + min(xcd, rem) + slot;
-  const int gx = gridDim.x, gy = gridDim.y;
-  return {l % gx, (l / gx) % gy, l / (gx * gy)};
-}
 // Causal backward grids (grid x = row or key block, y = head, z = range of a split), heaviest block
 // first over everything an XCD runs: the columns (head, range) are dealt to the XCDs whole when their
 // number is a multiple of 8, and an XCD's j-th work-group takes block rank j / C of its C columns.
 // The first 64 work-groups of an XCD start at once, two to each of its 32 CUs (the j-th and the
 // (j + 32)-th on one): the second layer is handed out lightest first, so that every CU gets about the
 // same work, and where it has only m < 32 work-groups the heaviest 32 - m of the first layer go to the CUs
-// that get no second one.  heavy_last: the block with the highest index has the most work.
-__device__ inline WgCoord causal_bwd_order(bool heavy_last) {
+// that get no second one.  two_per_cu false (one work-group per CU): heaviest first throughout.
+// heavy_last: the block with the highest index has the most work.
+__device__ inline WgCoord causal_bwd_order(bool heavy_last, bool two_per_cu) {
   const int gx = gridDim.x, gy = gridDim.y, cols = gy * gridDim.z;
   const int lin = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
   int blk, col;
@@ -280,7 +266,7 @@ __device__ inline WgCoord causal_bwd_order(bool heavy_last) {
     blk = lin / cols;
     col = lin - blk * cols;
   } else {
-    const int C = cols >> 3, per = gx * C, m = min(32, per - 32);
+    const int C = cols >> 3, per = gx * C, m = two_per_cu ? min(32, per - 32) : 0;
     int slot = lin >> 3;
     if (m > 0) {
       if (slot < 32) {
