@@ -95,7 +95,16 @@ int plan_fwd(const elsa_fwd_args* a, elsa_fwd_plan* pl) {
     // 0.594 ms with 2 partitions against 0.605 ms with 4 (2048 workgroups); 64K 9.06 / 9.17 /
     // 9.35 ms with 4 / 8 / 16; the forward at 1K and at ViT's 1025 tokens (B8 H3) stays within
     // 3% from 1 to 8 partitions
-    int64_t p = cdiv(1024, q_tiles);
+    // Unbiased fp16/bf16 calls without a causal mask below 4K keys: one 128-row work-group per CU, or two 256-row
+    // ones, are enough; a single partition also needs no Phase 2.  Forward ms against the 1024 target, fp16:
+    // B4 H8 1K 0.0230 -> 0.0180 (2 -> 1 partitions), B8 H8 1K 0.0366 -> 0.0279 (2 -> 1), B4 H8 2K 0.0589 -> 0.0507
+    // (4 -> 2), d128 B2 H8 2K 0.0597 -> 0.0517 (4 -> 1), B8 H8 1K 0.0690 -> 0.0527 (2 -> 1), d32 B8 H8 1K 0.0252 ->
+    // 0.0205 (2 -> 1); B2 H8 2K keeps 4 (0.0359 against 0.0403 with 2).  d128 from 4K: 512 (B1 H8 4K 0.0924 ->
+    // 0.0852, 4 -> 2; 1: 0.0926)
+    int64_t target = 1024;
+    if (a->dtype != ELSA_F32 && !a->is_causal && !a->bias.ptr && (n < 4096 || dp > 64))
+      target = bm == 128 && n < 4096 ? 256 : 512;
+    int64_t p = cdiv(target, q_tiles);
     p = std::min<int64_t>(p, std::max<int64_t>(1, n / 512));
     if (a->dtype == ELSA_F32) {
       // fp32 from 1024 keys without a causal mask, where the 1024 work-group target leaves the last round of
@@ -128,7 +137,8 @@ int plan_fwd(const elsa_fwd_args* a, elsa_fwd_plan* pl) {
     // -> 0.010 (2 -> 4 partitions), N512 0.0099 -> 0.0084 (1 -> 4), causal N1025 0.0139 -> 0.0121
     // (3 -> 5); B8 H3 N1025 (240 work-groups) keeps its two (5: 0.026 against 0.021 ms), and shorter
     // sequences their one fused partition (B8 H3 N197: more measured slower)
-    if (a->dtype != ELSA_F32 && dp <= 64 && n >= 512 && q_tiles * p < 192)
+    // (d128 B2 H4 N1000 0.0287 -> 0.0192, 1 -> 4)
+    if (a->dtype != ELSA_F32 && (dp <= 64 || (!a->is_causal && !a->bias.ptr)) && n >= 512 && q_tiles * p < 192)
       p = std::max<int64_t>(p, std::min<int64_t>(cdiv(256, q_tiles), std::max<int64_t>(1, n / 128)));
     if (n >= 8192) p = std::max<int64_t>(p, 2);
     // causal from 8K keys: partitions of n/4 keys within [2048, 8192].  About half of the

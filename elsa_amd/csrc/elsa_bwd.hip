@@ -161,10 +161,39 @@ __device__ inline typename Mfma<T>::frag tr_frag_at(const T* tile, int r0, int c
 }
 
 
+// acc of group 1 added into acc of group 0: head dim tiles dt in LDS buffer dt % 2
+template <int NDT, int WAVES>
+__device__ inline void add_groups(f32x16 (&acc)[NDT], float* b0, float* b1, int grp, int wave, int lane) {
+  auto at = [&](int dt, int q4) {
+    return reinterpret_cast<f32x4*>(dt & 1 ? b1 : b0) + (((dt >> 1) * 4 + q4) * WAVES + wave) * 64 + lane;
+  };
+  if (grp == 1) {
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4)
+        *at(dt, q4) = f32x4{acc[dt][4 * q4], acc[dt][4 * q4 + 1], acc[dt][4 * q4 + 2], acc[dt][4 * q4 + 3]};
+  }
+  __syncthreads();
+  if (grp == 0) {
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4) {
+        const f32x4 v = *at(dt, q4);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) acc[dt][4 * q4 + t] += v[t];
+      }
+  }
+}
+
 // LD (the two-tile 8-wave kernel at D = 64): the K and V stage tiles go straight from global memory
 // into LDS (buffer_load_dwordx4 ... lds, one stage ahead) instead of through staging registers.
-template <typename T, int DP, int RT, int WAVES, bool HAS_BIAS, bool LD = false>
-__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2)))
+// G = 2: two groups of WAVES waves on the same rows, group g taking every other stage of the work-group's
+// keys; group 1 hands its sums to group 0 through LDS at the end.  Grids of at most one work-group per CU
+// then run two waves per SIMD without partials in memory.
+template <typename T, int DP, int RT, int WAVES, bool HAS_BIAS, bool LD = false, int G = 1>
+__global__ __launch_bounds__(64 * WAVES * G) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void bwd_dq_half_kernel(const BwdParams p) {
   using M = Mfma<T>;
   typedef typename M::frag F;
@@ -178,15 +207,21 @@ void bwd_dq_half_kernel(const BwdParams p) {
   constexpr int NCH = KT * CPR / NT;
   static_assert(!LD || ((WAVES == 4 || WAVES == 8) && DP == 64 && !HAS_BIAS && KT == 64 && KS == 72),
                 "LDS-direct staging: the 4- and 8-wave D = 64 kernels, padded 144-byte rows");
+  static_assert(G == 1 || (G == 2 && RT == 1 && WAVES == 4 && !HAS_BIAS), "two-group variants");
   // LD: one array per buffer (see bwd_dkdv_half_kernel)
-  __shared__ __attribute__((aligned(16))) T Ks[LD ? 1 : 2][KT * KS];
-  __shared__ __attribute__((aligned(16))) T Vs[LD ? 1 : 2][KT * KS];
-  __shared__ __attribute__((aligned(16))) T Ks1[LD ? KT * KS : 1];
-  __shared__ __attribute__((aligned(16))) T Vs1[LD ? KT * KS : 1];
+  __shared__ __attribute__((aligned(16))) T Ks_s[G][LD ? 1 : 2][KT * KS];
+  __shared__ __attribute__((aligned(16))) T Vs_s[G][LD ? 1 : 2][KT * KS];
+  __shared__ __attribute__((aligned(16))) T Ks1_s[G][LD ? KT * KS : 1];
+  __shared__ __attribute__((aligned(16))) T Vs1_s[G][LD ? KT * KS : 1];
 
-  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 31,
+  const int grp = G == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / NT);
+  const int tid = threadIdx.x - grp * NT, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 31,
             g = lane >> 5;
-  const WgCoord wg = p.causal ? causal_bwd_order(true, WAVES == 4) : xcd_order();
+  T(*Ks)[KT * KS] = Ks_s[grp];
+  T(*Vs)[KT * KS] = Vs_s[grp];
+  T* Ks1 = Ks1_s[grp];
+  T* Vs1 = Vs1_s[grp];
+  const WgCoord wg = p.causal ? causal_bwd_order(true, WAVES * G == 4) : xcd_order();
   const int bh = wg.y;
   const int wg_row0 = wg.x * BM;
   const int wg_last = min(p.N, wg_row0 + BM) - 1;
@@ -235,7 +270,7 @@ void bwd_dq_half_kernel(const BwdParams p) {
       const float dsum = (pair[0] + pair[1]) + (pair[2] + pair[3]);
       float lhi, llo;
       lse2_split(p.row_m[ri], p.row_z[ri], lhi, llo);
-      if (ok && g == 0 && (!CAN_SPLIT || wg.z == 0)) {
+      if (ok && g == 0 && grp == 0 && (!CAN_SPLIT || wg.z == 0)) {
         p.d_row[ri] = dsum;
         p.lse_row[ri] = lhi;
         p.lse_lo[ri] = llo;
@@ -253,7 +288,7 @@ void bwd_dq_half_kernel(const BwdParams p) {
   // ..., so that the ranges differ by at most one stage, under a causal mask too; one without a stage
   // writes zeros.  D = 128 never splits (bwd_splits) but keeps these run-time bounds: with constant
   // ones its register allocation spilled (20 bytes per lane, 468 biased; 16K dq 1.698 -> 1.653 ms without)
-  const int k_lo = CAN_SPLIT ? wg.z * KT : 0, k_step = CAN_SPLIT ? p.split * KT : KT;
+  const int k_lo = CAN_SPLIT ? (wg.z * G + grp) * KT : 0, k_step = CAN_SPLIT ? p.split * G * KT : KT;
   // -D of this lane's row: the dP^T product starts from it and yields dP - D directly.  The
   // 16 registers per row tile of that constant would spill in the bias, D = 128 and two-tile
   // variants, which subtract D from each score instead.
@@ -369,6 +404,8 @@ static_for<0, NCH>([&](auto I) {
     for (int dt = 0; dt < NDT; ++dt) acc[rt][dt] = f32x16{};
 
   const int ntiles = k_end > k_lo ? (k_end - k_lo + k_step - 1) / k_step : 0;
+  // both groups meet every barrier: the first one's stages are the most
+  const int nloop = G == 1 ? ntiles : max(0, (k_end - (int)wg.z * G * KT + k_step - 1) / k_step);
   // stage keys [t0, t0 + KT) from LDS buffer buf into the dQ accumulators
   auto compute = [&](int t0, const T* ks, const T* vs) __attribute__((always_inline)) {
     if (!p.causal || t0 <= row0 + ROWS_W - 1) {
@@ -445,15 +482,15 @@ static_for<0, NCH>([&](auto I) {
     if (ntiles > 0) ldload(k_lo, Ks[0], Vs[0]);
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
-    for (int it = 0; it < ntiles; it += 2) {
+    for (int it = 0; it < nloop; it += 2) {
       const int t0 = k_lo + it * k_step;
       if (it + 1 < ntiles) ldload(t0 + k_step, Ks1, Vs1);
-      compute(t0, Ks[0], Vs[0]);
+      if (G == 1 || it < ntiles) compute(t0, Ks[0], Vs[0]);
       __builtin_amdgcn_s_waitcnt(0);
       __syncthreads();
-      if (it + 1 < ntiles) {
+      if (it + 1 < nloop) {
         if (it + 2 < ntiles) ldload(t0 + 2 * k_step, Ks[0], Vs[0]);
-        compute(t0 + k_step, Ks1, Vs1);
+        if (G == 1 || it + 1 < ntiles) compute(t0 + k_step, Ks1, Vs1);
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
       }
@@ -471,27 +508,34 @@ static_for<0, NCH>([&](auto I) {
       const int buf = it & 1;
       const int t0 = k_lo + it * k_step;
       if (it + 2 < ntiles) gload(t0 + 2 * k_step, FREE);
-      compute(t0, Ks[buf], Vs[buf]);
+      if (G == 1 || it < ntiles) compute(t0, Ks[buf], Vs[buf]);
       if (it + 1 < ntiles) sstore(buf ^ 1, NEXT);
       __syncthreads();
     };
-    for (int it = 0; it < ntiles; it += 2) {
+    for (int it = 0; it < nloop; it += 2) {
       step(it, S1, S0);
-      if (it + 1 < ntiles) step(it + 1, S0, S1);
+      if (it + 1 < nloop) step(it + 1, S0, S1);
     }
   } else {
     gload(k_lo, S0);
     sstore(0, S0);
     __syncthreads();
-    for (int it = 0; it < ntiles; ++it) {
+    for (int it = 0; it < nloop; ++it) {
       const int buf = it & 1;
       const int t0 = k_lo + it * k_step;
       const bool has_next = it + 1 < ntiles;
       if (has_next) gload(t0 + k_step, S0);
-      compute(t0, Ks[buf], Vs[buf]);
+      if (G == 1 || it < ntiles) compute(t0, Ks[buf], Vs[buf]);
       if (has_next) sstore(buf ^ 1, S0);
       __syncthreads();
     }
+  }
+  if constexpr (G == 2) {
+    // group 1's sums through the stage buffers (free after the last barrier), lane by lane
+    float* red[2] = {reinterpret_cast<float*>(Ks_s), reinterpret_cast<float*>(Vs_s)};
+    static_assert(sizeof(Ks_s) >= ((NDT + 1) / 2) * 4 * 4 * 64 * 16, "room for the sums of half the head dim tiles");
+    add_groups<NDT, WAVES>(acc[0], red[0], red[1], grp, wave, lane);
+    if (grp == 1) return;
   }
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
@@ -529,8 +573,9 @@ static_for<0, NCH>([&](auto I) {
 // fragments alone need more than the 256 registers of that budget, so 1 wave per SIMD
 // LD (8 waves, D = 64, no bias): the Q and dO stage tiles go straight from global memory into LDS
 // (buffer_load_dwordx4 ... lds, one stage ahead) instead of through staging registers.
-template <typename T, int DP, int KRT, int WAVES, bool HAS_BIAS, bool LD = false>
-__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(DP >= 128 ? 1 : 2, 2)))
+// G = 2: two groups of waves on the same keys and alternate row stages, as in bwd_dq_half_kernel.
+template <typename T, int DP, int KRT, int WAVES, bool HAS_BIAS, bool LD = false, int G = 1>
+__global__ __launch_bounds__(64 * WAVES * G) __attribute__((amdgpu_waves_per_eu(DP >= 128 ? 1 : 2, 2)))
 void bwd_dkdv_half_kernel(const BwdParams p) {
   using M = Mfma<T>;
   typedef typename M::frag F;
@@ -548,16 +593,24 @@ void bwd_dkdv_half_kernel(const BwdParams p) {
                 "LDS-direct staging: the one-tile D = 64 kernels");
   // LD: one array per buffer, so that the compiler sees the loads into one buffer leave the other
   // one's reads alone (with one two-buffer array it waited for them before every stage's reads)
-  __shared__ __attribute__((aligned(16))) T Qs[LD ? 1 : 2][RTS * KS];
-  __shared__ __attribute__((aligned(16))) T Gs[LD ? 1 : 2][RTS * KS];
-  __shared__ __attribute__((aligned(16))) T Qs1[LD ? RTS * KS : 1];
-  __shared__ __attribute__((aligned(16))) T Gs1[LD ? RTS * KS : 1];
-  __shared__ __attribute__((aligned(16))) float lse_s[2][RTS];
-  __shared__ __attribute__((aligned(16))) float ndd_s[2][RTS];  // -D of the stage's rows
+  static_assert(G == 1 || (G == 2 && KRT == 1 && WAVES == 4 && !HAS_BIAS && DP <= 64), "two-group variants");
+  __shared__ __attribute__((aligned(16))) T Qs_s[G][LD ? 1 : 2][RTS * KS];
+  __shared__ __attribute__((aligned(16))) T Gs_s[G][LD ? 1 : 2][RTS * KS];
+  __shared__ __attribute__((aligned(16))) T Qs1_s[G][LD ? RTS * KS : 1];
+  __shared__ __attribute__((aligned(16))) T Gs1_s[G][LD ? RTS * KS : 1];
+  __shared__ __attribute__((aligned(16))) float lse_ss[G][2][RTS];
+  __shared__ __attribute__((aligned(16))) float ndd_ss[G][2][RTS];  // -D of the stage's rows
 
-  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 31,
+  const int grp = G == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / NT);
+  const int tid = threadIdx.x - grp * NT, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 31,
             g = lane >> 5;
-  const WgCoord wg = p.causal ? causal_bwd_order(false, WAVES == 4) : xcd_order();
+  T(*Qs)[RTS * KS] = Qs_s[grp];
+  T(*Gs)[RTS * KS] = Gs_s[grp];
+  T* Qs1 = Qs1_s[grp];
+  T* Gs1 = Gs1_s[grp];
+  float(*lse_s)[RTS] = lse_ss[grp];
+  float(*ndd_s)[RTS] = ndd_ss[grp];
+  const WgCoord wg = p.causal ? causal_bwd_order(false, WAVES * G == 4) : xcd_order();
   const int bh = wg.y;
   const int wg_key0 = wg.x * BN;
   const int key0 = wg_key0 + wave * KEYS_W;
@@ -699,9 +752,10 @@ static_for<0, NCH>([&](auto I) {
   // split (the 4-wave one-tile kernel only), as in the dq kernel: the row stages z, z + split, ... from the
   // causal key block's first one on
   constexpr bool CAN_SPLIT = KRT == 1 && WAVES == 4 && !HAS_BIAS && DP <= 64;
-  const int r_lo = (p.causal ? (wg_key0 / RTS) * RTS : 0) + (CAN_SPLIT ? wg.z * RTS : 0);
-  const int r_step = CAN_SPLIT ? p.split * RTS : RTS;
+  const int r_lo = (p.causal ? (wg_key0 / RTS) * RTS : 0) + (CAN_SPLIT ? (wg.z * G + grp) * RTS : 0);
+  const int r_step = CAN_SPLIT ? p.split * G * RTS : RTS;
   const int ntiles = p.N > r_lo ? (p.N - r_lo + r_step - 1) / r_step : 0;
+  const int nloop = G == 1 ? ntiles : max(0, (p.N - (r_lo - grp * RTS) + r_step - 1) / r_step);
   // stage rows [t0, t0 + RTS) from LDS buffer buf into the dK / dV accumulators
   auto compute = [&](int buf, int t0, const T* qs, const T* gs) __attribute__((always_inline)) {
     if (!p.causal || t0 + RTS - 1 >= key0) {
@@ -822,16 +876,16 @@ static_for<0, NCH>([&](auto I) {
     }
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
-    for (int it = 0; it < ntiles; it += 2) {
+    for (int it = 0; it < nloop; it += 2) {
       const int t0 = r_lo + it * r_step;
       if (it + 1 < ntiles) ldload(t0 + r_step, Qs1, Gs1);
-      compute(0, t0, Qs[0], Gs[0]);
+      if (G == 1 || it < ntiles) compute(0, t0, Qs[0], Gs[0]);
       if (it + 1 < ntiles) ldstore(1);
       __builtin_amdgcn_s_waitcnt(0);
       __syncthreads();
-      if (it + 1 < ntiles) {
+      if (it + 1 < nloop) {
         if (it + 2 < ntiles) ldload(t0 + 2 * r_step, Qs[0], Gs[0]);
-        compute(1, t0 + r_step, Qs1, Gs1);
+        if (G == 1 || it + 1 < ntiles) compute(1, t0 + r_step, Qs1, Gs1);
         if (it + 2 < ntiles) ldstore(0);
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
@@ -848,14 +902,22 @@ static_for<0, NCH>([&](auto I) {
     const int buf = it & 1;
     const int t0 = r_lo + it * r_step;
     if (it + 2 < ntiles) gload(t0 + 2 * r_step, FREE);
-    compute(buf, t0, Qs[buf], Gs[buf]);
+    if (G == 1 || it < ntiles) compute(buf, t0, Qs[buf], Gs[buf]);
     if (it + 1 < ntiles) sstore(buf ^ 1, NEXT);
     __syncthreads();
   };
-  for (int it = 0; it < ntiles; it += 2) {
+  for (int it = 0; it < nloop; it += 2) {
     step(it, S1, S0);
-    if (it + 1 < ntiles) step(it + 1, S0, S1);
+    if (it + 1 < nloop) step(it + 1, S0, S1);
   }
+  }
+  if constexpr (G == 2) {  // group 1's sums through the stage buffers, 16 KB per head dim tile
+    constexpr int TB = 4 * WAVES * 64 * 4;
+    static_assert(sizeof(Qs_s) >= (LD || DP == 32 ? 1 : 2) * TB * 4 && (!LD || sizeof(Qs1_s) >= TB * 4), "room for the sums");
+    float *b0 = reinterpret_cast<float*>(Qs_s), *b1 = reinterpret_cast<float*>(Gs_s);
+    add_groups<NDT, WAVES>(dk[0], b0, LD ? reinterpret_cast<float*>(Qs1_s) : b0 + TB, grp, wave, lane);
+    add_groups<NDT, WAVES>(dv[0], b1, LD ? reinterpret_cast<float*>(Gs1_s) : b1 + TB, grp, wave, lane);
+    if (grp == 1) return;
   }
 #pragma unroll
   for (int kt = 0; kt < KRT; ++kt) {
@@ -1311,37 +1373,55 @@ static hipError_t bwd_launch3(const BwdParams& p, int stage, hipStream_t st) {
   constexpr int R = 1;  // one 32-wide tile per wave: 2 waves per SIMD beat wider tiles at 1
   const dim3 grid((p.N + 32 * R * W - 1) / (32 * R * W), p.BH);
   if constexpr (!B && DP <= 64) {
+    // an under-filled grid (short sequences, few heads): the key (dq) or row (dK/dV) loop cut into p.split
+    // ranges over grid z, fp32 partials summed by a combine launch.  pair: work-groups of two wave groups, at
+    // most one per CU, that take two ranges each and add them in LDS, where that leaves no partials (and
+    // the ranges would occupy more than half the CUs anyway) or the ranges would go two to a CU.  Whole
+    // backward ms, fp16 d64: B8 H3 N1025 0.0614 -> 0.0501, N577 0.0382 -> 0.0314, 4K 0.150 -> 0.137, B2 H8 1K
+    // 0.0482 -> 0.0434, B4 H3 N1025 0.0470 -> 0.0409, 2K 0.0638 -> 0.0593; but N512 0.0235 -> 0.0254 and 1K
+    // 0.0349 -> 0.0364 (the pairs share half as many CUs).  Causal splits keep one range per work-group:
+    // two to a CU they balance.
+    const int64_t wgs = (int64_t)grid.x * grid.y, ranges = wgs * p.split;
+    const bool pair = p.split % 2 == 0 && !p.causal && ranges <= 512 && ranges > (p.split == 2 ? 128 : 256);
     if (p.split > 1) {
-      // an under-filled grid (short sequences, few heads): the key (dq) or row (dK/dV) loop cut
-      // into p.split ranges over grid z, fp32 partials summed by a combine launch
-      const dim3 gs(grid.x, grid.y, (unsigned)p.split);
+      BwdParams ps = p;
+      if (pair) ps.split = p.split / 2;
+      const dim3 gs(grid.x, grid.y, (unsigned)ps.split);
       const CombineOut cq{p.part, p.dq, {p.dqs[0], p.dqs[1], p.dqs[2]}, p.scale};
       const CombineOut ck{p.part + p.part_stride, p.dk, {p.dks[0], p.dks[1], p.dks[2]}, p.scale};
       const CombineOut cv{p.part + 2 * p.part_stride, p.dv, {p.dvs[0], p.dvs[1], p.dvs[2]}, 1.f};
       if (stage < 0 || stage == 1) {
-        if (ld_kv) {
-          hipLaunchKernelGGL((bwd_dq_half_kernel<T, DP, R, W, false, DP == 64>), gs, dim3(64 * W), 0, st, p);
+        if (pair && ld_kv) {
+          hipLaunchKernelGGL((bwd_dq_half_kernel<T, DP, R, W, false, DP == 64, 2>), gs, dim3(128 * W), 0, st, ps);
+        } else if (pair) {
+          hipLaunchKernelGGL((bwd_dq_half_kernel<T, DP, R, W, false, false, 2>), gs, dim3(128 * W), 0, st, ps);
+        } else if (ld_kv) {
+          hipLaunchKernelGGL((bwd_dq_half_kernel<T, DP, R, W, false, DP == 64>), gs, dim3(64 * W), 0, st, ps);
         } else {
-          hipLaunchKernelGGL((bwd_dq_half_kernel<T, DP, R, W, false>), gs, dim3(64 * W), 0, st, p);
+          hipLaunchKernelGGL((bwd_dq_half_kernel<T, DP, R, W, false>), gs, dim3(64 * W), 0, st, ps);
         }
         if ((e = hipGetLastError()) != hipSuccess) return e;
-        if (stage == 1 && (e = combine_launch<T>(p, &cq, 1, st)) != hipSuccess) return e;
+        if (stage == 1 && ps.split > 1 && (e = combine_launch<T>(ps, &cq, 1, st)) != hipSuccess) return e;
       }
       if (stage < 0 || stage == 2) {
-        if (ld_qg) {
-          hipLaunchKernelGGL((bwd_dkdv_half_kernel<T, DP, R, W, false, DP == 64>), gs, dim3(64 * W), 0, st, p);
+        if (pair && ld_qg) {
+          hipLaunchKernelGGL((bwd_dkdv_half_kernel<T, DP, R, W, false, DP == 64, 2>), gs, dim3(128 * W), 0, st, ps);
+        } else if (pair) {
+          hipLaunchKernelGGL((bwd_dkdv_half_kernel<T, DP, R, W, false, false, 2>), gs, dim3(128 * W), 0, st, ps);
+        } else if (ld_qg) {
+          hipLaunchKernelGGL((bwd_dkdv_half_kernel<T, DP, R, W, false, DP == 64>), gs, dim3(64 * W), 0, st, ps);
         } else {
-          hipLaunchKernelGGL((bwd_dkdv_half_kernel<T, DP, R, W, false>), gs, dim3(64 * W), 0, st, p);
+          hipLaunchKernelGGL((bwd_dkdv_half_kernel<T, DP, R, W, false>), gs, dim3(64 * W), 0, st, ps);
         }
         if ((e = hipGetLastError()) != hipSuccess) return e;
       }
       // the whole backward sums the three gradients' partials in one launch
-      if (stage < 0) {
+      if (ps.split > 1 && stage < 0) {
         const CombineOut all[3] = {cq, ck, cv};
-        e = combine_launch<T>(p, all, 3, st);
-      } else if (stage == 2) {
+        e = combine_launch<T>(ps, all, 3, st);
+      } else if (ps.split > 1 && stage == 2) {
         const CombineOut kv[2] = {ck, cv};
-        e = combine_launch<T>(p, kv, 2, st);
+        e = combine_launch<T>(ps, kv, 2, st);
       }
       return e;
     }
@@ -1400,6 +1480,12 @@ static hipError_t bwd_launch3(const BwdParams& p, int stage, hipStream_t st) {
           wide = true;
         }
       }
+    }
+    if constexpr (DP == 128 && !B) {
+      // at most one 4-wave work-group per CU: two groups of waves on alternate stages (B2 H8 2K dq 0.0745 ->
+      // 0.0648 ms, B1 H4 N1000 0.0342 -> 0.0305)
+      if ((wide = (int64_t)grid.x * grid.y <= 256))
+        hipLaunchKernelGGL((bwd_dq_half_kernel<T, DP, R, W, false, false, 2>), grid, dim3(128 * W), 0, st, p);
     }
     if (!wide) {
       if (ld_kv) {

@@ -1814,6 +1814,13 @@ static hipError_t launch1h_wb(const Phase1Params& p, int block_m, hipStream_t st
     // 224 px forward 1.531 -> 1.469 ms, 512 px 4.371 -> 4.253 ms).
     if (block_m == 64) return b ? launch1h<T, DP, 1, 2, true>(p, st) : launch1h<T, DP, 2, 1, false>(p, st);
     if (block_m == 128) return b ? launch1h<T, DP, 1, 4, true>(p, st) : launch1h<T, DP, 1, 4, false>(p, st);
+    // Short partitions (no ping-pong fold) in at most 512 256-row work-groups: one 64-row-per-wave work-group per
+    // SIMD set leaves nothing to overlap its softmax with, two 128-row ones do.  Forward ms, fp16 d64: B8 H3
+    // N1025 0.0236 -> 0.0206, 2K 0.0232 -> 0.0203, B3 H8 N1500 0.0377 -> 0.0333, B1 H8 N3000 0.0376 -> 0.0357, B2 H8 2K
+    // 0.0340 -> 0.0324; level at B16 H3 N1025 (480 work-groups).  (By N, not q_len: a call cut into q-chunks
+    // keeps its kernel and bits.)
+    if (!b && !p.causal && p.part_len < 1024 && (int64_t)((p.N + 255) / 256) * p.BH * p.P <= 512)
+      return launch1h<T, DP, 1, 4, false>(p, st);
     // the planner gives biased calls 128-row blocks (phase1_block_m); the grid follows the kernel
     return b ? launch1h<T, DP, 1, 4, true>(p, st) : launch1h<T, DP, 2, 4, false>(p, st);
   } else {
