@@ -95,17 +95,32 @@ int plan_fwd(const elsa_fwd_args* a, elsa_fwd_plan* pl) {
     // 0.594 ms with 2 partitions against 0.605 ms with 4 (2048 workgroups); 64K 9.06 / 9.17 /
     // 9.35 ms with 4 / 8 / 16; the forward at 1K and at ViT's 1025 tokens (B8 H3) stays within
     // 3% from 1 to 8 partitions
-    // Unbiased fp16/bf16 calls without a causal mask below 4K keys: one 128-row work-group per CU, or two 256-row
-    // ones, are enough; a single partition also needs no Phase 2.  Forward ms against the 1024 target, fp16:
-    // B4 H8 1K 0.0230 -> 0.0180 (2 -> 1 partitions), B8 H8 1K 0.0366 -> 0.0279 (2 -> 1), B4 H8 2K 0.0589 -> 0.0507
-    // (4 -> 2), d128 B2 H8 2K 0.0597 -> 0.0517 (4 -> 1), B8 H8 1K 0.0690 -> 0.0527 (2 -> 1), d32 B8 H8 1K 0.0252 ->
-    // 0.0205 (2 -> 1); B2 H8 2K keeps 4 (0.0359 against 0.0403 with 2).  d128 from 4K: 512 (B1 H8 4K 0.0924 ->
-    // 0.0852, 4 -> 2; 1: 0.0926)
-    int64_t target = 1024;
-    if (a->dtype != ELSA_F32 && !a->is_causal && !a->bias.ptr && (n < 4096 || dp > 64))
-      target = bm == 128 && n < 4096 ? 256 : 512;
-    int64_t p = cdiv(target, q_tiles);
+    int64_t p = cdiv(1024, q_tiles);
     p = std::min<int64_t>(p, std::max<int64_t>(1, n / 512));
+    // the launcher's condition for the ping-pong fold (512-row work-groups over partitions of >= 1024 keys)
+    const bool pp = !a->is_causal && !a->bias.ptr && a->dtype != ELSA_F32 && dp == 64 && bm == 256 &&
+                    !(a->dtype == ELSA_F16 && a->summary_dtype == ELSA_F32);
+    // Unbiased fp16/bf16 calls without a causal mask, below 4K keys or at head dim 128: the count that minimises
+    // rounds x (partition keys + 100) + the merge.  A CU runs two work-groups together in one round, an odd
+    // one alone in 0.555 of it; 100 keys for a work-group's fixed cost; Phase 2: 2 us for its launch and 0.108
+    // per work-group for its bytes (all in keys of one round: 0.0215 us for 128 rows at d64, 0.043 for 256 rows
+    // or d128).  Ping-pong partitions: 0.64 x rounds of one work-group per CU x (partition keys + 768), as
+    // below.  Forward ms against the 1024 target: fp16 B4 H8 1K 0.0202 -> 0.0162 (2 -> 1 partitions), B8 H8 1K
+    // 0.0326 -> 0.0242 (2 -> 1), B10 H6 N1800 0.0874 -> 0.0630 (3 -> 1), B8 H3 N2305 0.0585 -> 0.0514 (4 -> 2), B4 H8 2K
+    // 0.0564 -> 0.0492 (4 -> 2), d32 B8 H8 1K 0.0256 -> 0.0195 (2 -> 1), d128 B2 H8 2K 0.0562 -> 0.0493 (4 -> 1), B8
+    // H8 1K 0.0583 -> 0.0461 (2 -> 1), B1 H8 4K 0.0907 -> 0.0850 (4 -> 2); B2 H8 2K, B2 H3 N3000 and B12 H8 N1111 keep
+    // 4, 5 and 2
+    if (a->dtype != ELSA_F32 && !a->is_causal && !a->bias.ptr && (n < 4096 || dp > 64)) {
+      auto cost = [&](int64_t c) {
+        const int64_t len = cdiv(cdiv(n, c), kt) * kt, parts = cdiv(n, len), wgs = q_tiles * parts, k = cdiv(wgs, 256);
+        const double merge = c > 1 ? (bm == 256 || dp > 64 ? 45 : 90) + 0.108 * (double)wgs : 0.0;
+        if (pp && len >= 1024) return 0.64 * (double)(cdiv(bh * cdiv(q_rows, 512) * parts, 256) * (len + 768)) + merge;
+        return ((double)(k / 2) + (k % 2 ? 0.555 : 0.0)) * (double)(len + 100) + merge;
+      };
+      p = 1;
+      for (int64_t c = 2; c <= n / 512; ++c)
+        if (cost(c) < cost(p)) p = c;
+    }
     if (a->dtype == ELSA_F32) {
       // fp32 from 1024 keys without a causal mask, where the 1024 work-group target leaves the last round of
       // the chip mostly empty: rounds x (partition keys + 130) over 256-row work-groups, one per CU (the
@@ -159,8 +174,6 @@ int plan_fwd(const elsa_fwd_args* a, elsa_fwd_plan* pl) {
     // 0.134 (4 -> 2 partitions), B2 H8 4K 0.097 -> 0.079 (4 -> 2), B4 H8 4K 0.158 -> 0.133 (2 -> 1),
     // B8 H3 N4097 0.155 -> 0.128 (3 -> 1), B1 H4 16K 0.269 -> 0.256 (4 -> 2), B1 H8 N6000 0.129 ->
     // 0.092 (6 -> 2), B1 H8 N12000 0.352 -> 0.323 (3 -> 2); the north star keeps 2.
-    const bool pp = !a->is_causal && !a->bias.ptr && a->dtype != ELSA_F32 && dp == 64 && bm == 256 &&
-                    !(a->dtype == ELSA_F16 && a->summary_dtype == ELSA_F32);
     if (pp && n >= 4096) {
       const int64_t tiles = bh * cdiv(q_rows, 512);
       const int64_t p_lo = n >= 8192 ? 2 : 1, p_hi = std::max<int64_t>(p_lo, n / 1024);
