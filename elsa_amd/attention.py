@@ -289,6 +289,16 @@ def _twopass_attention(q, k, v, *, bias, is_causal, block_m, block_n, q_chunk_si
                        phase2_warps, phase1_stages, phase2_stages, input_precision, algorithm, out_bnhd):
     """twopass_attention; ``out_bnhd`` returns a [B,H,N,D] view of [B,N,H,D] memory (for
     callers that go on to ``transpose(1, 2).reshape(B, N, H*D)``, which is then free)."""
+    # default options on plain operands, which the checks below would pass through unchanged (host side of a
+    # call 10.1 -> 6.0 us)
+    if (block_m is None and block_n is None and q_chunk_size is None and summary_dtype is None
+            and phase1_warps is None and phase2_warps is None and phase1_stages is None and phase2_stages is None
+            and input_precision == "auto" and (algorithm == "auto" or algorithm == "paper_scan")
+            and isinstance(q, torch.Tensor) and q.is_cuda):
+        mod = _lib.torch_module()
+        code = mod.plain_code(q, k, v, bias)
+        if code >= 0:
+            return mod.attention_forward(q, k, v, bias, bool(is_causal), code, 0, 0, bool(out_bnhd))
     _check_qkv(q, k, v, "twopass_attention")
     if algorithm not in ("auto", "paper_scan"):
         raise ValueError("only algorithm='paper_scan' is available in this strict release")

@@ -13,6 +13,7 @@
 // inference call (twopass_attention) with the same host side in C++: one planner query, the
 // workspace and elsa_fwd, without row state.
 #include <ATen/hip/HIPContext.h>
+#include <torch/csrc/autograd/python_variable.h>
 #include <torch/extension.h>
 
 #include <array>
@@ -271,6 +272,45 @@ at::Tensor attention_forward(const at::Tensor& q, const at::Tensor& k, const at:
       .out;
 }
 
+// ---- calls with default options on operands the kernels read in place
+// plain_code takes q, k, v and bias as Python passed them and returns the type code of the plain case
+// (four-dimensional GPU tensors of one supported type, device and shape, strides and bases the ABI accepts,
+// no bias or a four-dimensional one used as it is), else -1: the Python layer then validates, copies or
+// raises as it always does.  It accepts only what the Python layer passes through unchanged.
+bool plain_operand(const at::Tensor& t) {
+  return t.layout() == at::kStrided && t.is_cuda() && t.dim() == 4 && t.size(3) % 8 == 0 && t.stride(3) == 1 &&
+         t.stride(0) % 8 == 0 && t.stride(1) % 8 == 0 && t.stride(2) % 8 == 0 && t.stride(0) >= 0 && t.stride(1) >= 0 &&
+         t.stride(2) >= t.size(3) && t.numel() > 0 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+}
+bool plain_type(at::ScalarType t) { return t == at::kHalf || t == at::kBFloat16 || t == at::kFloat; }
+
+bool plain_call(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v) {
+  return plain_type(q.scalar_type()) && k.scalar_type() == q.scalar_type() && v.scalar_type() == q.scalar_type() &&
+         q.dim() == 4 && q.sizes() == k.sizes() && q.sizes() == v.sizes() && q.size(3) <= 128 &&
+         k.device() == q.device() && v.device() == q.device() && plain_operand(q) && plain_operand(k) && plain_operand(v);
+}
+
+// b: None, or a bias that _canonical_bias (attention.py) returns unchanged
+bool plain_bias(PyObject* b, const at::Tensor& q) {
+  if (b == Py_None) return true;
+  if (!THPVariable_CheckExact(b)) return false;
+  const at::Tensor& t = THPVariable_Unpack(b);
+  const int64_t n = q.size(2);
+  if (t.layout() != at::kStrided || t.device() != q.device() || t.dim() != 4 || t.size(2) != n || t.size(3) != n ||
+      (t.size(0) != 1 && t.size(0) != q.size(0)) || (t.size(1) != 1 && t.size(1) != q.size(1)) ||
+      !plain_type(t.scalar_type()) || t.stride(3) != 1)
+    return false;
+  for (int i = 0; i < 4; ++i)
+    if (t.stride(i) <= 0 && t.size(i) != 1) return false;
+  return true;
+}
+
+int64_t plain_code(py::handle qh, py::handle kh, py::handle vh, py::handle bias) {
+  if (!THPVariable_CheckExact(qh.ptr()) || !THPVariable_CheckExact(kh.ptr()) || !THPVariable_CheckExact(vh.ptr())) return -1;
+  const at::Tensor &q = THPVariable_Unpack(qh.ptr()), &k = THPVariable_Unpack(kh.ptr()), &v = THPVariable_Unpack(vh.ptr());
+  return plain_call(q, k, v) && plain_bias(bias.ptr(), q) ? code_of(q.scalar_type()) : -1;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -278,6 +318,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("qkv_attention_train", &qkv_attention_train, "fused-qkv two-pass attention with recompute backward");
   m.def("attention_train", &attention_train, "two-pass attention on q, k, v with recompute backward");
   m.def("attention_forward", &attention_forward, "two-pass attention forward on q, k, v (inference)");
+  m.def("plain_code", &plain_code, "type code of operands (and bias) that need no Python check or copy, else -1");
   m.def("current_stream", [] { return reinterpret_cast<int64_t>(current_stream()); },
         "raw handle of the stream the launches go to");
   m.def("abi_version", [] { return elsa_abi_version(); });

@@ -98,3 +98,36 @@ def test_short_backward_is_the_same_from_run_to_run():
         runs.append(torch.autograd.grad(out, (q, k, v, bias), do))
     for r in runs[1:]:
         assert all(torch.equal(a, b) for a, b in zip(runs[0], r))
+
+
+def test_default_calls_match_calls_with_a_knob():
+    """A call with default options skips the Python checks where its operands are plain; the same call with a
+    knob that changes nothing (phase1_warps) goes through them: the same bits, and what they refuse stays refused."""
+    g = torch.Generator(device="cuda").manual_seed(4)
+    base = torch.randn((2, 50, 3, 3, 32), generator=g, device="cuda").half()
+    views = {"dense": lambda t: t.contiguous(), "strided": lambda t: t, "odd": lambda t: t[..., :20],
+             "misaligned": lambda t: t.contiguous().reshape(-1)[4:4 + 2 * 3 * 48 * 32].view(2, 3, 48, 32)}
+    for name, view in views.items():
+        q, k, v = (view(t) for t in base.permute(2, 0, 3, 1, 4).unbind(0))
+        n = q.shape[2]
+        for bias in (None, torch.randn((1, 3, n, n), generator=g, device="cuda").half(),
+                     torch.randn((3, n, n), generator=g, device="cuda"),
+                     torch.randn((1, 3, n, n), generator=g, device="cuda").double(),
+                     torch.randn((2, 1, 1, n), generator=g, device="cuda").half().expand(2, 1, n, n)):
+            for causal in (False, True):
+                a = elsa_amd.twopass_attention(q, k, v, bias=bias, is_causal=causal)
+                b = elsa_amd.twopass_attention(q, k, v, bias=bias, is_causal=causal, phase1_warps=4)
+                assert torch.equal(a, b), name
+                ins = [t.detach().clone(memory_format=torch.preserve_format).requires_grad_(True) for t in (q, k, v)]
+                x = elsa_amd.twopass_attention_train(*ins, bias=bias, is_causal=causal)
+                y = elsa_amd.twopass_attention_train(*ins, bias=bias, is_causal=causal, phase1_warps=4)
+                gx, gy = (torch.autograd.grad(o, ins, torch.ones_like(o)) for o in (x, y))
+                assert torch.equal(x, y) and all(torch.equal(s, t) for s, t in zip(gx, gy)), name
+    q = base.permute(2, 0, 3, 1, 4)[0]
+    for bad, err in (((q, q[:, :, :20], q), "identical shapes"), ((q, q.float(), q), "one dtype"),
+                     ((q.double(),) * 3, "supported dtypes"), ((q, q.cpu(), q), "one device"), ((q[0],) * 3, "B,H,N,D")):
+        for call in (elsa_amd.twopass_attention, elsa_amd.twopass_attention_train):
+            with pytest.raises(ValueError, match=err):
+                call(*bad)
+    with pytest.raises(ValueError, match="bias"):
+        elsa_amd.twopass_attention(q, q, q, bias=torch.zeros((2, 3, 49, 50), device="cuda"))
