@@ -20,7 +20,8 @@ ROOT = PKG.parent
 CSRC = PKG / "csrc"
 LIB = PKG / "libelsa_hip.so"
 TORCH_MODULE = PKG / "_elsa_torch.so"
-SOURCES = ("elsa_fwd.hip", "elsa_bwd.hip", "elsa_bwd_f32.hip", "elsa_bwd_short.hip", "elsa_api.hip")
+SOURCES = ("elsa_fwd.hip", "elsa_bwd.hip", "elsa_bwd_f32.hip", "elsa_bwd_short.hip", "elsa_bwd_d128.hip",
+           "elsa_api.hip")
 ARCH = "gfx950"
 
 # Packed fp32 VALU forms are disabled for all device code (only scalar / packed-16-bit VALU).

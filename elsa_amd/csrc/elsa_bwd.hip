@@ -161,32 +161,6 @@ __device__ inline typename Mfma<T>::frag tr_frag_at(const T* tile, int r0, int c
 }
 
 
-// acc of group 1 added into acc of group 0: head dim tiles dt in LDS buffer dt % 2
-template <int NDT, int WAVES>
-__device__ inline void add_groups(f32x16 (&acc)[NDT], float* b0, float* b1, int grp, int wave, int lane) {
-  auto at = [&](int dt, int q4) {
-    return reinterpret_cast<f32x4*>(dt & 1 ? b1 : b0) + (((dt >> 1) * 4 + q4) * WAVES + wave) * 64 + lane;
-  };
-  if (grp == 1) {
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4)
-        *at(dt, q4) = f32x4{acc[dt][4 * q4], acc[dt][4 * q4 + 1], acc[dt][4 * q4 + 2], acc[dt][4 * q4 + 3]};
-  }
-  __syncthreads();
-  if (grp == 0) {
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
-        const f32x4 v = *at(dt, q4);
-#pragma unroll
-        for (int t = 0; t < 4; ++t) acc[dt][4 * q4 + t] += v[t];
-      }
-  }
-}
-
 // LD (the two-tile 8-wave kernel at D = 64): the K and V stage tiles go straight from global memory
 // into LDS (buffer_load_dwordx4 ... lds, one stage ahead) instead of through staging registers.
 // G = 2: two groups of WAVES waves on the same rows, group g taking every other stage of the work-group's
@@ -1495,6 +1469,10 @@ static hipError_t bwd_launch3(const BwdParams& p, int stage, hipStream_t st) {
       }
     }
     if ((e = hipGetLastError()) != hipSuccess) return e;
+  }
+  if constexpr (DP == 128 && !B) {
+    if ((stage < 0 || stage == 2) && (int64_t)p.N * p.qs[2] * es < lim && (int64_t)p.N * p.gs[2] * es < lim)
+      return launch_dkdv_d128(p, std::is_same<T, f16>::value ? ELSA_F16 : ELSA_BF16, st);
   }
   if (stage < 0 || stage == 2) {
     // dK/dV in 8-wave work-groups (256 keys) at D = 64 where that grid still puts two

@@ -89,22 +89,27 @@ struct TileLane {
     }
     return s;
   }
-  // fp32: the same with the own operand's parts from own(kk)
+  // the same with the own operand from own(kk)
   template <typename Get>
   __device__ inline f32x16 dot_with(const E* tile, Get&& own) const {
     f32x16 s = f32x16{};
-    bf16x8 h[NKK], oh[NKK];
+    if constexpr (F32) {
+      bf16x8 h[NKK], oh[NKK];
 #pragma unroll
-    for (int kk = 0; kk < NKK; ++kk) {
-      h[kk] = *reinterpret_cast<const bf16x8*>(tile + o_row[kk]);
-      const bf16x8 m = *reinterpret_cast<const bf16x8*>(tile + S::PLANE + o_row[kk]);
-      const bf16x8 l = *reinterpret_cast<const bf16x8*>(tile + 2 * S::PLANE + o_row[kk]);
-      const Split3 o = own(kk);
-      oh[kk] = o.h;
-      s = mma3_small(h[kk], m, l, o, s);
+      for (int kk = 0; kk < NKK; ++kk) {
+        h[kk] = *reinterpret_cast<const bf16x8*>(tile + o_row[kk]);
+        const bf16x8 m = *reinterpret_cast<const bf16x8*>(tile + S::PLANE + o_row[kk]);
+        const bf16x8 l = *reinterpret_cast<const bf16x8*>(tile + 2 * S::PLANE + o_row[kk]);
+        const Split3 o = own(kk);
+        oh[kk] = o.h;
+        s = mma3_small(h[kk], m, l, o, s);
+      }
+#pragma unroll
+      for (int kk = 0; kk < NKK; ++kk) s = Mfma<bf16>::mma(h[kk], oh[kk], s);
+    } else {
+#pragma unroll
+      for (int kk = 0; kk < NKK; ++kk) s = Mfma<T>::mma(*reinterpret_cast<const F*>(tile + o_row[kk]), own(kk), s);
     }
-#pragma unroll
-    for (int kk = 0; kk < NKK; ++kk) s = Mfma<bf16>::mma(h[kk], oh[kk], s);
     return s;
   }
   // acc[dt] += tile^T w over the stage's 32 rows.  fp32: each stage's product goes into a fresh
@@ -147,6 +152,32 @@ struct TileLane {
   }
 };
 
+// acc of group 1 added into acc of group 0: head dim tiles dt in LDS buffer dt % 2
+template <int NDT, int WAVES>
+__device__ inline void add_groups(f32x16 (&acc)[NDT], float* b0, float* b1, int grp, int wave, int lane) {
+  auto at = [&](int dt, int q4) {
+    return reinterpret_cast<f32x4*>(dt & 1 ? b1 : b0) + (((dt >> 1) * 4 + q4) * WAVES + wave) * 64 + lane;
+  };
+  if (grp == 1) {
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4)
+        *at(dt, q4) = f32x4{acc[dt][4 * q4], acc[dt][4 * q4 + 1], acc[dt][4 * q4 + 2], acc[dt][4 * q4 + 3]};
+  }
+  __syncthreads();
+  if (grp == 0) {
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4) {
+        const f32x4 v = *at(dt, q4);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) acc[dt][4 * q4 + t] += v[t];
+      }
+  }
+}
+
 // One sum of a split backward's partials (bwd_combine_kernel).
 struct CombineOut {
   const float* part;
@@ -155,6 +186,8 @@ struct CombineOut {
   float scale;
 };
 // one launch for up to three sums (n = 1, 2 or 3 of c[0..2]) into fp32 outputs
+// dk/dv of fp16 / bf16 head dims above 64, unbiased (elsa_bwd_d128.hip)
+hipError_t launch_dkdv_d128(const BwdParams& p, int dtype, hipStream_t st);
 hipError_t combine_launch_f32(const BwdParams& p, const CombineOut* c, int n, hipStream_t st);
 
 }  // namespace elsa
