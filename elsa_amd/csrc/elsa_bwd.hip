@@ -380,6 +380,7 @@ static_for<0, NCH>([&](auto I) {
   const int ntiles = k_end > k_lo ? (k_end - k_lo + k_step - 1) / k_step : 0;
   // both groups meet every barrier: the first one's stages are the most
   const int nloop = G == 1 ? ntiles : max(0, (k_end - (int)wg.z * G * KT + k_step - 1) / k_step);
+  const bool bias_vec = HAS_BIAS && bias_rows_vectorizable(p.bias);
   // stage keys [t0, t0 + KT) from LDS buffer buf into the dQ accumulators
   auto compute = [&](int t0, const T* ks, const T* vs) __attribute__((always_inline)) {
     if (!p.causal || t0 <= row0 + ROWS_W - 1) {
@@ -408,12 +409,15 @@ static_for<0, NCH>([&](auto I) {
           const bool full = (t0 + KT <= k_end) && (!p.causal || t0 + KT - 1 <= row0 + rt * 32);
           const float nl = -lse[rt];
           if constexpr (HAS_BIAS) {
+            float bv[16];
+            bias_keys16(p.bias, bi * p.bias.sb + hi * p.bias.sh + (int64_t)min(my_row, p.N - 1) * p.bias.sq,
+                        t0 + sub * 32 + 8 * g, k_end, bias_vec, bv);
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
               const int key = t0 + sub * 32 + key_of_reg(r, g);
               const bool ok = live[rt] && key < k_end && (!p.causal || key <= my_row);
               const float x = fmaf(s[r], p.scale_log2, nl);
-              const float pr = ok ? fast_exp2(fmaf(load_bias_b(p.bias, bi, hi, my_row, key), kLog2e, x)) : 0.f;
+              const float pr = ok ? fast_exp2(fmaf(bv[r], kLog2e, x)) : 0.f;
               ds[r] = pr * (dp[r] - dd[rt]);
             }
           } else {
@@ -795,13 +799,16 @@ static_for<0, NCH>([&](auto I) {
             const f32x4 l0 = *reinterpret_cast<const f32x4*>(lp), l1 = *reinterpret_cast<const f32x4*>(lp + 4);
             float pr[8];
             if constexpr (HAS_BIAS) {
+              float bv[8];
+              bias_rows<8>(p.bias, bi * p.bias.sb + hi * p.bias.sh + (int64_t)min(my_key, p.N - 1) * p.bias.sk,
+                           t0 + sub * 32 + 16 * j + 8 * g, p.N, bv);
 #pragma unroll
               for (int t = 0; t < 8; ++t) {
                 const int row = t0 + sub * 32 + key_of_reg(8 * j + t, g);
                 const float lr = t < 4 ? l0[t] : l1[t - 4];
                 const bool ok = key_ok[kt] && row < p.N && (!p.causal || row >= my_key);
                 const float x = fmaf(s[8 * j + t], p.scale_log2, -lr);
-                pr[t] = ok ? fast_exp2(fmaf(load_bias_b(p.bias, bi, hi, row, my_key), kLog2e, x)) : 0.f;
+                pr[t] = ok ? fast_exp2(fmaf(bv[t], kLog2e, x)) : 0.f;
               }
               if (p.ds_out != nullptr && key_ok[kt]) {  // lanes of one t: 32 consecutive keys of a row
                 float* dso = p.ds_out + (int64_t)bh * p.N * p.N + my_key;
@@ -974,7 +981,7 @@ __global__ __launch_bounds__(64 * WAVES) void row_stats_kernel(const BwdParams p
       const int key = t0 + key_of_reg(r, g);
       const bool ok = row_ok && key < k_end && (!p.causal || key <= my_row);
       float x = s[r] * p.scale_log2;
-      if constexpr (HAS_BIAS) x = ok ? fmaf(load_bias_b(p.bias, bi, hi, my_row, key), kLog2e, x) : x;
+      if constexpr (HAS_BIAS) x = ok ? fmaf(load_bias(p.bias, bi, hi, my_row, key), kLog2e, x) : x;
       s[r] = ok ? x : kNegInf;
       mx = fmaxf(mx, s[r]);
     }
@@ -1065,7 +1072,7 @@ __global__ __launch_bounds__(64) void dbias_kernel(const BwdParams p, float* dbi
         bool ok = row_ok && key < p.N && lse > kNegInf && (!p.causal || key <= my_row);
         // s*c - LSE2 rounded once (then LSE2's low part), before the bias: as the dq and dk/dv kernels
         const float x = fmaf(s[r], p.scale_log2, -lse) - lse_lo;
-        const float pr = ok ? fast_exp2(fmaf(load_bias_b(p.bias, b, h, my_row, key), kLog2e, x)) : 0.f;
+        const float pr = ok ? fast_exp2(fmaf(load_bias(p.bias, b, h, my_row, key), kLog2e, x)) : 0.f;
         acc[r] += pr * (dp[r] - dd);
       }
     }

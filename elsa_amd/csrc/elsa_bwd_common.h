@@ -1,17 +1,9 @@
 // Pieces of the backward that its 16-bit kernels (elsa_bwd.hip) and fp32 kernels (elsa_bwd_f32.hip) share.
 #pragma once
 
-#include "elsa_internal.h"
-#include "elsa_mfma.h"
+#include "elsa_bias.h"
 
 namespace elsa {
-
-__device__ inline float load_bias_b(const BiasView& b, int bi, int hi, int row, int key) {
-  const int64_t off = (int64_t)bi * b.sb + (int64_t)hi * b.sh + (int64_t)row * b.sq + (int64_t)key * b.sk;
-  if (b.dtype == ELSA_F32) return static_cast<const float*>(b.ptr)[off];
-  if (b.dtype == ELSA_F16) return static_cast<float>(static_cast<const f16*>(b.ptr)[off]);
-  return static_cast<float>(static_cast<const bf16*>(b.ptr)[off]);
-}
 
 // LSE2 = m + log2(max(z, 1e-30)) (attention_bwd.py:224), formed in double and split into its fp32
 // rounding hi and the remainder lo, so that the fp32 kernels' p = exp2(s*c - LSE2) does not carry

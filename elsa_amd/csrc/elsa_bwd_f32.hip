@@ -145,6 +145,7 @@ void bwd_dq_x3_kernel(const BwdParams p) {
   const float dd = row_ok ? pair[0] : 0.f;
   const TileLane<float, DP> ln(lane);
 
+  const bool bias_vec = HAS_BIAS && bias_rows_vectorizable(p.bias);
   f32x16 acc[NDT];
 #pragma unroll
   for (int dt = 0; dt < NDT; ++dt) acc[dt] = f32x16{};
@@ -153,15 +154,14 @@ void bwd_dq_x3_kernel(const BwdParams p) {
     if (p.causal && t0 > row0 + 31) return;  // a causal wave whose rows all precede this stage
     f32x16 s = ln.dot(kt, qf);
     const bool full = (t0 + TT <= k_end) && (!p.causal || t0 + TT - 1 <= row0);
+    float bv[HAS_BIAS ? 16 : 1];
+    if constexpr (HAS_BIAS)
+      bias_keys16(p.bias, bi * p.bias.sb + hi * p.bias.sh + rsafe * p.bias.sq, t0 + 8 * g, k_end, bias_vec, bv);
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       // s*c - LSE2 with one rounding of the (small) difference, then LSE2's low part
       float x = fmaf(s[r], p.scale_log2, -lse) - lse_lo;
-      if constexpr (HAS_BIAS) {
-        const int key = t0 + key_of_reg(r, g);
-        const bool ok = row_ok && key < k_end;
-        if (ok) x = fmaf(load_bias_b(p.bias, bi, hi, my_row, key), kLog2e, x);
-      }
+      if constexpr (HAS_BIAS) x = row_ok ? fmaf(bv[r], kLog2e, x) : x;
       s[r] = fast_exp2(x);
     }
     if (!full) {
@@ -300,15 +300,15 @@ void bwd_dkdv_x3_kernel(const BwdParams p) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const f32x4 a = row_vals(st_s[buf][0], q), b = row_vals(st_s[buf][1], q);
+      float bv[4];
+      if constexpr (HAS_BIAS)
+        bias_rows<4>(p.bias, bi * p.bias.sb + hi * p.bias.sh + ksafe * p.bias.sk, t0 + key_of_reg(4 * q, g), p.N, bv);
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         const int r = 4 * q + t;
         // s*c - LSE2 with one rounding of the (small) difference, then LSE2's low part
         float x = fmaf(s[r], p.scale_log2, -a[t]) - b[t];
-        if constexpr (HAS_BIAS) {
-          const int row = t0 + key_of_reg(r, g);
-          if (key_ok && row < p.N) x = fmaf(load_bias_b(p.bias, bi, hi, row, my_key), kLog2e, x);
-        }
+        if constexpr (HAS_BIAS) x = key_ok && t0 + key_of_reg(r, g) < p.N ? fmaf(bv[t], kLog2e, x) : x;
         s[r] = fast_exp2(x);
       }
     }

@@ -81,7 +81,7 @@ void bwd_short_kernel(const BwdParams p, int groups) {
       if (p.bias.sb != 0 || bi == (int)blockIdx.x) {
 #pragma unroll 8
         for (int r = wave; r < N; r += 4)
-          if (lane < N) bias_s[r * BS + lane] = load_bias_b(p.bias, bi, hi, r, lane);
+          if (lane < N) bias_s[r * BS + lane] = load_bias(p.bias, bi, hi, r, lane);
       }
     }
 #pragma unroll

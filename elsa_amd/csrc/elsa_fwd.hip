@@ -26,8 +26,7 @@
 //   at or before the row are read: later ones are the identity, so this is the
 //   inclusive prefix at the row's own partition (the value the reference's
 //   Hillis-Steele scan hands to its finalize, attention_parallel_scan.py:745).
-#include "elsa_internal.h"
-#include "elsa_mfma.h"
+#include "elsa_bias.h"
 
 namespace elsa {
 
@@ -58,66 +57,6 @@ struct FwdCfg {
 int phase1_key_tile(int dtype, int dp) {
   if (dtype == ELSA_F32) return dp >= 64 ? 32 : 64;
   return 64;
-}
-
-__device__ inline float load_bias(const BiasView& b, int bi, int hi, int row, int key) {
-  const int64_t off = (int64_t)bi * b.sb + (int64_t)hi * b.sh + (int64_t)row * b.sq + (int64_t)key * b.sk;
-  if (b.dtype == ELSA_F32) return static_cast<const float*>(b.ptr)[off];
-  if (b.dtype == ELSA_F16) return static_cast<float>(static_cast<const f16*>(b.ptr)[off]);
-  return static_cast<float>(static_cast<const bf16*>(b.ptr)[off]);
-}
-
-// Bias rows that 16-byte loads can read: 16-bit values, key stride 1, batch / head / row
-// strides in multiples of 8 elements and a 16-byte aligned base.
-__device__ inline bool bias_rows_vectorizable(const BiasView& b) {
-  return b.dtype != ELSA_F32 && b.sk == 1 && b.sq % 8 == 0 && b.sb % 8 == 0 && b.sh % 8 == 0 &&
-         reinterpret_cast<uintptr_t>(b.ptr) % 16 == 0;
-}
-
-// Bias of one query row (element offset row_off) at keys key0 + 16 j + t (j < 2, t < 8) into
-// v[8 j + t]: the keys the D-layout registers of one 32-key sub-tile hold (key_of_reg).
-// Keys at or past k_end read as 0 (the caller masks them).  vec: one 16-byte load per 8 keys.
-template <typename B16>
-__device__ inline void bias_keys16_vec(const BiasView& b, int64_t row_off, int key0, int k_end, float (&v)[16]) {
-  typedef B16 b8 __attribute__((ext_vector_type(8)));
-  const B16* base = static_cast<const B16*>(b.ptr) + row_off;
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int k = key0 + 16 * j;
-    if (k + 8 <= k_end) {
-      const b8 c = *reinterpret_cast<const b8*>(base + k);
-#pragma unroll
-      for (int t = 0; t < 8; ++t) v[8 * j + t] = static_cast<float>(c[t]);
-    } else {
-#pragma unroll
-      for (int t = 0; t < 8; ++t) v[8 * j + t] = k + t < k_end ? static_cast<float>(base[k + t]) : 0.f;
-    }
-  }
-}
-
-__device__ inline void bias_keys16(const BiasView& b, int64_t row_off, int key0, int k_end, bool vec, float (&v)[16]) {
-  if (vec) {
-    if (b.dtype == ELSA_F16)
-      bias_keys16_vec<f16>(b, row_off, key0, k_end, v);
-    else
-      bias_keys16_vec<bf16>(b, row_off, key0, k_end, v);
-    return;
-  }
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int key = key0 + 16 * (r >> 3) + (r & 7);
-    float x = 0.f;
-    if (key < k_end) {
-      const int64_t off = row_off + (int64_t)key * b.sk;
-      if (b.dtype == ELSA_F32)
-        x = static_cast<const float*>(b.ptr)[off];
-      else if (b.dtype == ELSA_F16)
-        x = static_cast<float>(static_cast<const f16*>(b.ptr)[off]);
-      else
-        x = static_cast<float>(static_cast<const bf16*>(b.ptr)[off]);
-    }
-    v[r] = x;
-  }
 }
 
 __device__ inline void store4(void* base, int64_t off, int dtype, float a, float b, float c, float d) {
@@ -1821,6 +1760,10 @@ static hipError_t launch1h_wb(const Phase1Params& p, int block_m, hipStream_t st
     // keeps its kernel and bits.)
     if (!b && !p.causal && p.part_len < 1024 && (int64_t)((p.N + 255) / 256) * p.BH * p.P <= 512)
       return launch1h<T, DP, 1, 4, false>(p, st);
+    // Causal calls below 16K keys too: their work-groups differ in length, and the diagonal blocks waste half as
+    // much.  Forward ms, bf16: B2 H8 N4097 0.0676 -> 0.0623, 8K 0.1018 -> 0.0968, B4 H8 4K 0.1038 -> 0.0987, B8 H3 N4097
+    // 0.0873 -> 0.0853, B2 H12 N3000 0.0569 -> 0.0532, d32 B2 H8 N4097 0.0536 -> 0.0413; 16K 0.322 -> 0.334.
+    if (!b && p.causal && p.part_len % 128 == 0 && p.N < 16384) return launch1h<T, DP, 1, 4, false>(p, st);
     // the planner gives biased calls 128-row blocks (phase1_block_m); the grid follows the kernel
     return b ? launch1h<T, DP, 1, 4, true>(p, st) : launch1h<T, DP, 2, 4, false>(p, st);
   } else {
