@@ -112,21 +112,25 @@ __device__ inline Split3 split3_reg(const float (&x)[8]) {
   o.l = to_bf16x8(r);
   return o;
 }
-// any input: h truncated, so that no finite value becomes infinite, and an infinity or NaN alone in h
-// (its m and l are 0, not infinity - infinity)
+// any input: h truncated, so that no finite value becomes infinite.  An infinity or NaN goes to l, which
+// meets only the other operand's h (of its sign, 0 only for 0): as h it also met m and l, of either sign
+// or 0, and a product with infinity came out NaN.  h and m are then those of the largest finite value, whose
+// products with the other operand's l stay finite for values up to 2^16.  (Selects on a finite test
+// instead: forward B1 H8 8K 0.680 -> 0.692 ms, training step 4K 0.761 -> 0.766.)
 __device__ inline Split3 split3_any(const float (&x)[8]) {
 #pragma clang fp contract(off)
   Split3 o;
   float r[8], h[8];
 #pragma unroll
   for (int t = 0; t < 8; ++t) {
-    h[t] = __uint_as_float(__float_as_uint(x[t]) & 0xffff0000u);
-    r[t] = fabsf(x[t]) < __builtin_huge_valf() ? x[t] - h[t] : 0.f;
+    const float f = __builtin_amdgcn_fmed3f(x[t], -__FLT_MAX__, __FLT_MAX__);
+    h[t] = __uint_as_float(__float_as_uint(f) & 0xffff0000u);
+    r[t] = f - h[t];
   }
   o.h = to_bf16x8(h);
   o.m = to_bf16x8(r);
 #pragma unroll
-  for (int t = 0; t < 8; ++t) r[t] -= static_cast<float>(o.m[t]);
+  for (int t = 0; t < 8; ++t) r[t] = (x[t] - h[t]) - static_cast<float>(o.m[t]);
   o.l = to_bf16x8(r);
   return o;
 }

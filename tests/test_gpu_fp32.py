@@ -94,9 +94,22 @@ def test_fp32_infinite_value_stays_in_its_column():
         v = v.clone()
         v[0, 0, 7, 5] = float("inf")
         out = elsa_amd.twopass_attention(q, k, v)
-        assert not torch.isfinite(out[..., 5]).any()
+        assert (out[..., 5] == float("inf")).all()
         keep = [d for d in range(64) if d != 5]
         assert torch.equal(out[..., keep], ref[..., keep])
+
+
+def test_fp32_key_at_minus_infinity_drops_out():
+    # q > 0 where one key is -inf: its score is -inf, so the others' softmax
+    for n in (40, 300):
+        q, k, v, do = _inputs((1, 1, n, 64), n)
+        q[..., 3] = q[..., 3].abs() + 0.1
+        k[0, 0, 9, 3] = float("-inf")
+        out = elsa_amd.twopass_attention(q, k, v)
+        rest = [i for i in range(n) if i != 9]
+        want = torch.softmax(q.double() @ k[:, :, rest].double().transpose(-1, -2).contiguous() / 8, -1) @ v[:, :, rest].double()
+        rel = ((out.double() - want).norm() / want.norm()).item()
+        assert rel <= BOUND, (n, rel)
 
 
 def test_fp32_strided_operands_match_dense_ones():

@@ -17,10 +17,12 @@ def _bf16_trunc(x):
 
 
 def _split(x, truncate_h):
-    h = _bf16_trunc(x) if truncate_h else _bf16_rne(x)
-    r = np.where(np.isfinite(x), x - np.where(np.isfinite(x), h, 0), 0).astype(np.float32)
-    m = _bf16_rne(r)
-    return h, m, _bf16_rne(r - m)
+    big = np.finfo(np.float32).max
+    f = np.fmin(np.fmax(x, -big), big).astype(np.float32)
+    h = _bf16_trunc(f) if truncate_h else _bf16_rne(f)
+    m = _bf16_rne(f - h)
+    r = (x - h) - m
+    return h, m, np.where(np.isfinite(x), _bf16_rne(r), r)
 
 
 @pytest.mark.parametrize("truncate_h", [True, False])
@@ -31,13 +33,26 @@ def test_three_parts_hold_every_bit(truncate_h):
     assert np.array_equal(h.astype(np.float64) + m + l, x.astype(np.float64))
 
 
-def test_infinities_and_the_largest_values_stay_in_the_first_part():
+def test_infinities_stay_in_the_last_part_and_the_largest_values_finite():
     x = np.array([np.inf, -np.inf, np.finfo(np.float32).max, -np.finfo(np.float32).max, 0.0], np.float32)
     h, m, l = _split(x, True)
-    assert np.array_equal(np.isinf(h), np.isinf(x))
-    assert not np.isnan(m).any() and not np.isnan(l).any()
+    assert np.isfinite(h).all() and np.isfinite(m).all()
+    assert np.array_equal(np.isinf(l), np.isinf(x))
     fin = np.isfinite(x)
     assert np.array_equal(h[fin].astype(np.float64) + m[fin] + l[fin], x[fin].astype(np.float64))
+
+
+def test_products_with_an_infinity_are_the_fp32_ones():
+    rng = np.random.default_rng(7)
+    b = (rng.standard_normal(1000) * 2.0 ** rng.integers(-20, 14, 1000)).astype(np.float32)
+    for a in (np.inf, -np.inf):
+        ah, am, al = _split(np.full(1000, a, np.float32), True)
+        for truncate_b, y in ((True, b), (False, np.clip(np.abs(b), 0, 256).astype(np.float32))):
+            # operands are truncated; probabilities, at most 2^8, are rounded
+            bh, bm, bl = _split(y, truncate_b)
+            with np.errstate(over="ignore"):
+                got = al * bh + ah * bl + am * bm + am * bh + ah * bm + ah * bh
+            assert np.array_equal(got, np.float32(a) * y)
 
 
 @pytest.mark.parametrize("truncate_a,truncate_b", [(True, True), (True, False), (False, False)])
