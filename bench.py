@@ -80,11 +80,13 @@ def _args():
 
 
 # rocprofv3 kernel-name fragment -> bench kernel name
-_KERNEL_KEYS = (("phase1_half_kernel", "phase1_fold"), ("phase1_pp_kernel", "phase1_fold"), ("phase1_kernel", "phase1_fold"),
+_KERNEL_KEYS = (("phase1_half_kernel", "phase1_fold"), ("phase1_pp_kernel", "phase1_fold"),
+                ("phase1_x3_kernel", "phase1_fold"), ("phase1_kernel", "phase1_fold"),
                 ("phase2_kernel", "phase2_merge"), ("phase2_np_kernel", "phase2_merge"),
                 ("bwd_pre_kernel", "bwd_preprocess"),
-                ("bwd_dq_half_kernel", "bwd_dq"), ("bwd_dq_kernel", "bwd_dq"),
-                ("bwd_dkdv_half_kernel", "bwd_dkdv"), ("bwd_dkdv_kernel", "bwd_dkdv"))
+                ("bwd_dq_half_kernel", "bwd_dq"), ("bwd_dq_x3_kernel", "bwd_dq"), ("bwd_dq_kernel", "bwd_dq"),
+                ("bwd_dkdv_half_kernel", "bwd_dkdv"), ("bwd_dkdv_x3_kernel", "bwd_dkdv"),
+                ("bwd_dkdv_d128_kernel", "bwd_dkdv"), ("bwd_dkdv_kernel", "bwd_dkdv"))
 
 
 def _read_pmc(path, counter):
@@ -182,7 +184,7 @@ def _kernel_ms(lib, stream, q, k, v, do, causal, block_n, steps):
     three backward stages run on that forward's output and row state.  A plan of one partition
     is timed as ``elsa_fwd`` runs it, one Phase-1 launch with the finalize fused into its epilogue
     (phase2_merge is then 0: no launch); where the dq kernel runs the preprocess (fp16/bf16 at
-    d = 64) bwd_preprocess is 0 the same way.  Returns (ms by kernel, the forward plan, the
+    d = 64, fp32) bwd_preprocess is 0 the same way.  Returns (ms by kernel, the forward plan, the
     forward output)."""
     import torch
 
@@ -210,10 +212,10 @@ def _kernel_ms(lib, stream, q, k, v, do, causal, block_n, steps):
     chunks = [(s_, min(qc, N - s_)) for s_ in range(0, N, qc)]
 
     fused = plan["partitions"] == 1
-    # fp16/bf16 at d = 64 (dense operands, N rows under 2 GiB) and fp32 at d <= 64: the dq kernels run
+    # fp16/bf16 at d = 64 (dense operands, N rows under 2 GiB) and fp32: the dq kernels run
     # the preprocess of their rows, and a whole backward (elsa_bwd) launches no preprocess kernel
     pre_fused = ((q.dtype in (torch.float16, torch.bfloat16) and D == 64 and N * D * q.element_size() < 2**31)
-                 or (q.dtype == torch.float32 and D <= 64))
+                 or q.dtype == torch.float32)
     # each launch set takes the stream handle it launches on
     launches = {
         "phase1_fold": ((lambda h: [lib.elsa_fwd(ctypes.byref(fa), h)]) if fused else

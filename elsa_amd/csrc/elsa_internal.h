@@ -129,8 +129,8 @@ struct BwdParams {
 // Ranges the backward (fp16, bf16 and fp32) cuts its loops into when its unsplit grid (128 rows or
 // keys per work-group) leaves the chip under-filled: doubled from 1 while the doubled grid stays
 // within 512 work-groups (causal fp32: 512 that hold work) and n / (2 * split) is at least 256 (64
-// for fp32); ragged fp32 grids and fp32 at D = 128 by the rounds they take.  Biased calls and 16-bit head
-// dims above 64 keep 1.
+// for fp32); ragged fp32 and 16-bit d64 grids without a causal mask, and fp32 at D = 128, by the rounds
+// they take.  Biased calls and 16-bit head dims above 64 keep 1.
 int bwd_splits(int dtype, int dp, int64_t bh, int64_t n, bool bias, bool causal);
 
 // stage < 0: preprocess, dq and dk/dv; 0: preprocess only; 1: dq only; 2: dk/dv only.

@@ -175,7 +175,8 @@ size_t elsa_bwd_workspace_bytes(const elsa_bwd_args* args);
 /* dq, dk, dv from the saved row state (exact recompute of p). */
 int elsa_bwd(const elsa_bwd_args* args, void* stream);
 /* One stage of elsa_bwd: 0 = D/LSE2 preprocess (into the workspace), 1 = dq kernel,
- * 2 = dk/dv kernel (stages 1 and 2 read what stage 0 wrote); -1 = all three. */
+ * 2 = dk/dv kernel (run stage 0 before 1 and 2; a stage may form D and LSE2 again);
+ * -1 = all three. */
 int elsa_bwd_stage(const elsa_bwd_args* args, int32_t stage, void* stream);
 /* Recompute the base-2 row state (row_m, row_z) from q, k (and bias). Uses
  * args->q, k, bias, shape fields; writes row_m/row_z [B*H, N]. */
