@@ -161,9 +161,9 @@ int plan_fwd(const elsa_fwd_args* a, elsa_fwd_plan* pl) {
     // Phase 1 + Phase 2 at B1 H8 d64 fp16 against 1024 / 2048 / 4096 / 8192-key partitions:
     // 8K 0.114 / 0.114 / 0.119 / 0.187 ms, 16K 0.380 / 0.342 / 0.343 / 0.366 ms, 32K 1.518 /
     // 1.344 / 1.227 / 1.199 ms.
-    // fp16/bf16 head dims above 64: at least 4096 keys (bf16 B1 H16 8K 0.335 -> 0.315 ms; 16K keeps 4096).
-    const int64_t part_min = a->dtype != ELSA_F32 && dp > 64 ? 4096 : 2048;
-    if (a->is_causal && n >= 8192) p = cdiv(n, std::min<int64_t>(8192, std::max<int64_t>(part_min, n / 4)));
+    // At d128 too: 4096-key partitions gained 6% at bf16 B1 H16 8K (0.335 -> 0.315 ms) and cost few heads up to 1.7
+    // times (H1 8K 0.053 -> 0.091, H2 0.060 -> 0.092, H4 0.101 -> 0.106, H1 12K 0.074 -> 0.094).
+    if (a->is_causal && n >= 8192) p = cdiv(n, std::min<int64_t>(8192, std::max<int64_t>(2048, n / 4)));
     p = std::max<int64_t>(p, 1);
     // the ping-pong fold (fp16/bf16 at d = 64 without bias or causal mask, 16-bit summaries; the
     // launcher's condition) runs 512-row work-groups over partitions of at least 1024 keys: B1 H8 4K
