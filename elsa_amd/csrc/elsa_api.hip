@@ -65,6 +65,13 @@ size_t fwd_workspace_bytes(int64_t parts, int64_t bh, int64_t q_chunk, int64_t d
   return 2 * align256(rows * 4) + align256(rows * d * dtype_size(sdt));
 }
 
+// Element stride from row to row of an operand (an all-zero layout is dense).
+int64_t row_stride(const elsa_layout& l, int64_t d) { return l.batch == 0 && l.head == 0 && l.row == 0 ? d : l.row; }
+// The kernels keep an offset inside a K partition in 32 bits.
+bool partition_fits(int64_t part_len, int64_t row_stride, int dtype) {
+  return part_len * row_stride * (int64_t)dtype_size(dtype) < (int64_t(1) << 31);
+}
+
 // Partition routing for 256 CUs: about 1024 Phase-1 workgroups when the query side alone
 // does not provide them, partitions of >= 512 keys (>= 1024 and one round of the chip where
 // the ping-pong fold runs), and at least two partitions from 8K keys on so long sequences
@@ -85,10 +92,8 @@ int plan_fwd(const elsa_fwd_args* a, elsa_fwd_plan* pl) {
   const int kt = elsa::phase1_key_tile(a->dtype, dp);
   const size_t row_bytes = 8 + (size_t)d * dtype_size(a->summary_dtype);
 
-  int64_t part;
-  if (a->partition_len > 0) {
-    part = std::min<int64_t>(a->partition_len, n);
-  } else {
+  // keys per partition; by_rounds: with the rules that weigh the rounds of the chip
+  auto partition_keys = [&](bool by_rounds) -> int64_t {
     const int64_t q_rows = a->q_chunk > 0 ? std::min<int64_t>(a->q_chunk, n) : n;
     const int64_t q_tiles = bh * cdiv(q_rows, bm);
     // about 1024 Phase-1 workgroups (4 per CU): at B1 H8 d64 fp16 16K, Phase 1 + Phase 2 took
@@ -110,7 +115,7 @@ int plan_fwd(const elsa_fwd_args* a, elsa_fwd_plan* pl) {
     // 0.0564 -> 0.0492 (4 -> 2), d32 B8 H8 1K 0.0256 -> 0.0195 (2 -> 1), d128 B2 H8 2K 0.0562 -> 0.0493 (4 -> 1), B8
     // H8 1K 0.0583 -> 0.0461 (2 -> 1), B1 H8 4K 0.0907 -> 0.0850 (4 -> 2); B2 H8 2K, B2 H3 N3000 and B12 H8 N1111 keep
     // 4, 5 and 2
-    if (a->dtype != ELSA_F32 && !a->is_causal && !a->bias.ptr && (n < 4096 || dp > 64)) {
+    if (by_rounds && a->dtype != ELSA_F32 && !a->is_causal && !a->bias.ptr && (n < 4096 || dp > 64)) {
       auto cost = [&](int64_t c) {
         const int64_t len = cdiv(cdiv(n, c), kt) * kt, parts = cdiv(n, len), wgs = q_tiles * parts, k = cdiv(wgs, 256);
         const double merge = c > 1 ? (bm == 256 || dp > 64 ? 45 : 90) + 0.108 * (double)wgs : 0.0;
@@ -127,7 +132,7 @@ int plan_fwd(const elsa_fwd_args* a, elsa_fwd_plan* pl) {
       // 8-wave fold), 130 keys for a work-group's fixed cost; the count with the least, if 7% below the
       // target's.  Forward ms (Phase 1 + Phase 2, d64): B2 H8 N4097 0.499 -> 0.438 (2 -> 5 partitions), B2 H8
       // 2K 0.105 -> 0.101 (4 -> 2); B1 H8 4K (0.190 against 0.186 with 2) and B8 H3 N1025 keep 4 and 2
-      if (!a->is_causal && n >= 1024) {
+      if (by_rounds && !a->is_causal && n >= 1024) {
         const int64_t tiles = bh * cdiv(q_rows, 256);
         auto cost = [&](int64_t c) {
           const int64_t len = cdiv(cdiv(n, c), kt) * kt;
@@ -189,7 +194,7 @@ int plan_fwd(const elsa_fwd_args* a, elsa_fwd_plan* pl) {
         }
       }
     }
-    part = cdiv(cdiv(n, p), kt) * kt;
+    int64_t part = cdiv(cdiv(n, p), kt) * kt;
     if (!a->is_causal && !a->bias.ptr && a->dtype != ELSA_F32 && dp == 64 && n >= 4096 && part < 1024) part = 1024;
     if (a->is_causal && p > 1) {  // one partition stays whole: its launch applies the finalize
       // causal partitions hold whole row blocks, which Phase 1's longest-first order needs;
@@ -200,7 +205,18 @@ int plan_fwd(const elsa_fwd_args* a, elsa_fwd_plan* pl) {
       const int64_t unit = std::max<int64_t>(kt, bm);
       part = std::max<int64_t>(unit, (cdiv(n, p) + unit / 2) / unit * unit);
     }
-    part = std::min<int64_t>(part, n);
+    return std::min<int64_t>(part, n);
+  };
+  int64_t part;
+  if (a->partition_len > 0) {
+    part = std::min<int64_t>(a->partition_len, n);
+  } else {
+    part = partition_keys(true);
+    // a partition's rows must span less than 2 GiB (check_layout): where the rules by rounds ask for one that
+    // does not (operands with row strides of 2^17 elements and more), the work-group target alone decides
+    const int64_t row = std::max(std::max(row_stride(a->q_layout, d), row_stride(a->k_layout, d)),
+                                 std::max(row_stride(a->v_layout, d), row_stride(a->out_layout, d)));
+    if (row < (int64_t(1) << 25) && !partition_fits(part, row, a->dtype)) part = partition_keys(false);
   }
   const int64_t parts = cdiv(n, part);
   if (parts > 65535) return fail(ELSA_ERR_UNSUPPORTED, "too many K partitions (%lld)", (long long)parts);
@@ -348,7 +364,7 @@ int check_layout(const char* name, const void* ptr, const elsa_layout& l, const 
   int64_t s[3];
   int rc = check_layout_rules(name, ptr, l, a->batch, a->heads, a->seq_len, a->head_dim, output, s);
   if (rc) return rc;
-  if (part_len * s[2] * (int64_t)dtype_size(a->dtype) >= (int64_t(1) << 31))
+  if (!partition_fits(part_len, s[2], a->dtype))
     return fail(ELSA_ERR_UNSUPPORTED, "%s: a K partition spans >= 2 GiB (partition_len %lld x row stride %lld)",
                 name, (long long)part_len, (long long)s[2]);
   return ELSA_OK;

@@ -151,7 +151,8 @@ const char* elsa_last_error(void);
 /* sizeof of the argument structs as compiled into the library (ABI check). */
 size_t elsa_struct_size(int which); /* 0 fwd_args, 1 fwd_plan, 2 bwd_args, 3 bias_desc, 4 layout */
 
-/* Tiling, partition routing and workspace size for a forward call. */
+/* Tiling, partition routing and workspace size for a forward call.  Reads the shape, dtypes, options,
+ * bias.ptr and the layouts: set them before the query. */
 int elsa_fwd_plan_get(const elsa_fwd_args* args, elsa_fwd_plan* plan);
 /* Full forward: for each q-chunk, Phase 1 (summaries -> workspace) then Phase 2. */
 int elsa_fwd(const elsa_fwd_args* args, void* stream);

@@ -33,3 +33,31 @@ def test_long_causal_calls_are_cut_in_four_at_every_head_dim(h, n, parts):
     for d in (32, 64, 128):
         plan = _plan(_fwd_args(_lib.ELSA_BF16, 1, h, n, d, causal=True))
         assert (plan.partitions, plan.partition_len) == (parts, n // parts), (d, plan.partitions)
+
+
+def _accepted(a):
+    """Whether elsa_fwd takes the call: elsa_phase1 runs the same checks before that of its row range."""
+    lib = _lib.load()
+    a.workspace, a.workspace_bytes = 256, 1 << 62
+    rc = lib.elsa_phase1(ctypes.byref(a), -1, 1, None)
+    msg = lib.elsa_last_error()
+    assert rc in (_lib.ELSA_ERR_INVALID, _lib.ELSA_ERR_UNSUPPORTED), msg
+    assert (rc == _lib.ELSA_ERR_INVALID) == (b"row range" in msg), msg
+    return rc == _lib.ELSA_ERR_INVALID
+
+
+# rows so far apart that only the shorter partitions of the work-group target span less than 2 GiB
+@pytest.mark.parametrize("dtype,b,h,n,d,row", [
+    (_lib.ELSA_F32, 1, 3, 4139, 64, 907352), (_lib.ELSA_BF16, 16, 1, 2448, 8, 1661696),
+    (_lib.ELSA_F16, 4, 3, 3654, 128, 801496), (_lib.ELSA_F16, 1, 16, 5474, 80, 349656),
+    (_lib.ELSA_F32, 2, 8, 2048, 64, 1 << 19), (_lib.ELSA_BF16, 4, 8, 1024, 64, 1 << 20)])
+def test_wide_rows_are_cut_into_partitions_below_2_gib(dtype, b, h, n, d, row):
+    a = _fwd_args(dtype, b, h, n, d)
+    a.q_layout = a.k_layout = a.v_layout = a.out_layout = _lib.Layout(8, 8, row)
+    assert _accepted(a)
+    size = 4 if dtype == _lib.ELSA_F32 else 2
+    assert _plan(a).partition_len * row * size < 1 << 31
+    # dense operands of the same shape are not affected, and one partition that spans 2 GiB stays refused
+    assert _accepted(_fwd_args(dtype, b, h, n, d))
+    a.partition_len = -(-(1 << 31) // (row * size))
+    assert a.partition_len > n or not _accepted(a)
