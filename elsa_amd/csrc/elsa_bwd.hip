@@ -1182,26 +1182,28 @@ static int64_t causal_live_wgs(int64_t bh, int64_t n, int s) {
 
 // fp32 grids whose last round of the chip is mostly empty: the range count 1..8 that minimises rounds x
 // (stage rows of a range + 65) plus the combine's traffic, in units of one key or row of one round of the
-// 8-wave dk/dv kernel (0.12 us at d64; the two kernels' rounds as in bwd_f32_waves_dq / _dkdv; 65 for a
-// work-group's fixed cost, 180 + 0.0032 x work-groups x head dim per range for the combine).  Whole
-// backward ms, d64: B2 H8 N4097 (528 work-groups for 512 slots) 1.90 -> 1.45 (1 -> 5 ranges); head dim 128 (one
-// 4-wave work-group per CU): B1 H8 2K 0.670 -> 0.377 (1 -> 2), B4 H2 N300 0.120 -> 0.056 (1 -> 4), B1 H8 4K stays.
+// 8-wave dk/dv kernel (0.12 us at d64; the two kernels' rounds as in dq_wide / dkdv_wide; 65 for a
+// work-group's fixed cost, 180 + 0.0032 x work-groups x head dim per range for the combine).  Split only
+// where the model saves 1.5% and the partials (three per range and row) stay below 512 MiB: on grids of many
+// rounds its half percent (0.4% at d128 B8 H8 N16385) is no gain and costs gigabytes of workspace, where a
+// modelled 2% of few rounds was 13% (H96 N700 d64 0.376 -> 0.327).
+// Whole backward ms, d64: B2 H8 N4097 (528 work-groups for 512 slots) 1.90 -> 1.45 (1 -> 5 ranges); head
+// dim 128 (one 4-wave work-group per CU): B1 H8 2K 0.670 -> 0.377 (1 -> 2), B4 H2 N300 0.120 -> 0.056 (1 -> 4),
+// B1 H8 4K stays.
 static int f32_ragged_splits(int dp, int64_t bh, int64_t n) {
+  constexpr int64_t kPartialBytes = int64_t(512) << 20;
   const int64_t w4 = bh * ((n + 127) / 128), w8 = bh * ((n + 255) / 256);
-  int best = 1;
-  double best_cost = 0;
-  for (int s = 1; s <= 8 && (s == 1 || n / s >= 64); ++s) {
+  auto cost = [&](int s) {
     const double k4 = (double)((w4 * s + 255) / 256), k8 = (double)((w8 * s + 255) / 256);
     const double dq4 = (double)((int64_t)k4 / 2) + ((int64_t)k4 % 2 ? 0.645 : 0.0);
     const double rounds = dp > 64 ? 2.33 * k4 : std::min(0.94 * k8, dq4) + 1.33 * std::min(k8, 0.645 * k4);
     const double len = (double)(((n + s - 1) / s + 31) / 32 * 32);
-    const double cost = rounds * (len + 65) + (s > 1 ? 180 + 0.0032 * (double)(w4 * dp) * s : 0.0);
-    if (s == 1 || cost < best_cost) {
-      best = s;
-      best_cost = cost;
-    }
-  }
-  return best;
+    return rounds * (len + 65) + (s > 1 ? 180 + 0.0032 * (double)(w4 * dp) * s : 0.0);
+  };
+  int best = 1;
+  for (int s = 2; s <= 8 && n / s >= 64 && 3 * s * bh * n * dp * 4 <= kPartialBytes; ++s)
+    if (cost(s) < cost(best)) best = s;
+  return cost(best) < 0.985 * cost(1) ? best : 1;
 }
 
 // The same for fp16 / bf16 at d64 without a causal mask, between 257 and 1024 4-wave work-groups: a CU's k

@@ -61,3 +61,34 @@ def test_wide_rows_are_cut_into_partitions_below_2_gib(dtype, b, h, n, d, row):
     assert _accepted(_fwd_args(dtype, b, h, n, d))
     a.partition_len = -(-(1 << 31) // (row * size))
     assert a.partition_len > n or not _accepted(a)
+
+
+def _bwd_workspace(dtype, b, h, n, d, causal=False):
+    """(bytes asked for, bytes of D and the two parts of LSE2 alone)"""
+    a = _lib.BwdArgs()
+    a.batch, a.heads, a.seq_len, a.head_dim = b, h, n, d
+    a.dtype, a.is_causal = dtype, int(causal)
+    return int(_lib.load().elsa_bwd_workspace_bytes(ctypes.byref(a))), 3 * (-(-b * h * n * 4 // 256) * 256)
+
+
+@pytest.mark.parametrize("b,h,n,d", [(8, 8, 16385, 128), (8, 16, 16385, 64), (7, 15, 40000, 128), (8, 16, 8193, 128),
+                                     (4, 16, 65537, 64)])
+def test_large_fp32_backwards_need_no_partials(b, h, n, d):
+    # up to 12 GiB of partials for a modelled half percent
+    need, rows = _bwd_workspace(_lib.ELSA_F32, b, h, n, d)
+    assert need == rows
+
+
+@pytest.mark.parametrize("b,h,n,d,split", [(2, 8, 4097, 64, 5), (1, 8, 2048, 128, 2), (4, 2, 300, 128, 4)])
+def test_ragged_fp32_backwards_keep_their_ranges(b, h, n, d, split):
+    need, rows = _bwd_workspace(_lib.ELSA_F32, b, h, n, d)
+    assert need == rows + 3 * split * b * h * n * d * 4
+
+
+def test_fp32_partials_stay_below_512_mib():
+    for d in (64, 128):
+        for bh in (1, 3, 8, 16, 24, 48, 96, 200, 1000):
+            for n in (300, 513, 1025, 2049, 4097, 8193, 16385, 32769):
+                for causal in (False, True):
+                    need, rows = _bwd_workspace(_lib.ELSA_F32, 1, bh, n, d, causal)
+                    assert need - rows <= 512 << 20, (d, bh, n, causal, need)
