@@ -476,8 +476,9 @@ elsa::BwdParams bwd_params(const elsa_bwd_args* a) {
   p.lse_lo = reinterpret_cast<float*>(base + 2 * align256(rows * 4));
   p.dp = elsa::pad_head_dim(a->head_dim);
   p.split = elsa::bwd_splits(a->dtype, p.dp, p.BH, p.N, a->bias.ptr != nullptr, a->is_causal != 0);
-  p.part = p.split > 1 ? reinterpret_cast<float*>(base + 3 * align256(rows * 4)) : nullptr;
-  p.part_stride = (int64_t)(align256((size_t)p.split * rows * p.dp * 4) / 4);
+  const int partials = elsa::bwd_partials(a->dtype, p.dp, p.BH, p.N, a->bias.ptr != nullptr, a->is_causal != 0);
+  p.part = partials > 1 ? reinterpret_cast<float*>(base + 3 * align256(rows * 4)) : nullptr;
+  p.part_stride = (int64_t)(align256((size_t)partials * rows * p.dp * 4) / 4);
   const int H = a->heads, N = a->seq_len, D = a->head_dim;
   resolve_layout(a->q_layout, H, N, D, p.qs);
   resolve_layout(a->k_layout, H, N, D, p.ks);
@@ -614,21 +615,17 @@ int elsa_phase2(const elsa_fwd_args* a, int32_t q_start, int32_t q_len, void* st
   return run_phase(a, pl, q_start, q_len, static_cast<hipStream_t>(stream), 2);
 }
 
-// fp32 partials of a split backward (dq, dK, dV): split * rows * dp floats each
-static size_t bwd_part_bytes(const elsa_bwd_args* a) {
-  const int dp = elsa::pad_head_dim(a->head_dim);
-  const int split = elsa::bwd_splits(a->dtype, dp, (int64_t)a->batch * a->heads, a->seq_len, a->bias.ptr != nullptr,
-                                     a->is_causal != 0);
-  if (split <= 1) return 0;
+// D, LSE2 and LSE2's low part, one float per row each; then `ranges` fp32 partials of dq, dK and dV
+static size_t bwd_bytes(const elsa_bwd_args* a, int ranges) {
   const size_t rows = (size_t)a->batch * a->heads * a->seq_len;
-  return 3 * align256((size_t)split * rows * dp * 4);
+  return 3 * align256(rows * 4) +
+         (ranges > 1 ? 3 * align256((size_t)ranges * rows * elsa::pad_head_dim(a->head_dim) * 4) : 0);
 }
 
 size_t elsa_bwd_workspace_bytes(const elsa_bwd_args* a) {
   if (!a || a->batch <= 0 || a->heads <= 0 || a->seq_len <= 0) return 0;
-  const size_t rows = (size_t)a->batch * a->heads * a->seq_len;
-  // D, LSE2 and LSE2's low part, one float per row each; then a split backward's partials
-  return 3 * align256(rows * 4) + bwd_part_bytes(a);
+  return bwd_bytes(a, elsa::bwd_splits(a->dtype, elsa::pad_head_dim(a->head_dim), (int64_t)a->batch * a->heads,
+                                       a->seq_len, a->bias.ptr != nullptr, a->is_causal != 0));
 }
 
 int elsa_bwd(const elsa_bwd_args* a, void* stream) { return elsa_bwd_stage(a, -1, stream); }
@@ -637,7 +634,7 @@ int elsa_bwd_stage(const elsa_bwd_args* a, int32_t stage, void* stream) {
   int rc = check_bwd(a, kUseGrads);
   if (rc) return rc;
   if (stage < -1 || stage > 2) return fail(ELSA_ERR_INVALID, "stage must be -1, 0, 1 or 2 (got %d)", stage);
-  const size_t need = elsa_bwd_workspace_bytes(a);
+  const size_t need = elsa::bwd_workspace_written(a);
   if (!a->workspace || a->workspace_bytes < need)
     return fail(ELSA_ERR_WORKSPACE, "workspace of %zu bytes is smaller than the %zu bytes required", a->workspace_bytes,
                 need);
@@ -779,3 +776,11 @@ int elsa_debug_mfma_rate(int32_t variant, const void* src, float* out, int32_t i
 }
 
 }  // extern "C"
+
+namespace elsa {
+size_t bwd_workspace_written(const elsa_bwd_args* a) {
+  if (!a || a->batch <= 0 || a->heads <= 0 || a->seq_len <= 0) return 0;
+  return bwd_bytes(a, bwd_partials(a->dtype, pad_head_dim(a->head_dim), (int64_t)a->batch * a->heads, a->seq_len,
+                                   a->bias.ptr != nullptr, a->is_causal != 0));
+}
+}  // namespace elsa

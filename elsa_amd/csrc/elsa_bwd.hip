@@ -1254,6 +1254,22 @@ int bwd_splits(int dtype, int dp, int64_t bh, int64_t n, bool bias, bool causal)
   return s;
 }
 
+// 16-bit splits whose ranges work-groups of two wave groups, at most one per CU, take two at a time and add in
+// LDS: where that leaves no partials (and the ranges would occupy more than half the CUs anyway) or the
+// ranges would go two to a CU.  Whole backward ms, fp16 d64: B8 H3 N1025 0.0614 -> 0.0501, N577 0.0382 ->
+// 0.0314, 4K 0.150 -> 0.137, B2 H8 1K 0.0482 -> 0.0434, B4 H3 N1025 0.0470 -> 0.0409, 2K 0.0638 -> 0.0593; but
+// N512 0.0235 -> 0.0254 and 1K 0.0349 -> 0.0364 (the pairs share half as many CUs).  Causal splits keep one
+// range per work-group: two to a CU they balance.
+bool bwd_pairs(int dtype, int split, int64_t bh, int64_t n, bool causal) {
+  const int64_t ranges = bh * ((n + 127) / 128) * split;
+  return dtype != ELSA_F32 && !causal && split % 2 == 0 && ranges <= 512 && ranges > (split == 2 ? 128 : 256);
+}
+
+int bwd_partials(int dtype, int dp, int64_t bh, int64_t n, bool bias, bool causal) {
+  const int split = bwd_splits(dtype, dp, bh, n, bias, causal);
+  return bwd_pairs(dtype, split, bh, n, causal) ? split / 2 : split;
+}
+
 // out[b, h, n, d] = scale * sum over the split ranges of part[z][b*H + h][n][d], 4 head-dim
 // elements per thread (head dims are multiples of 8); grid y picks one of up to three such sums.
 template <typename T>
@@ -1357,15 +1373,8 @@ static hipError_t bwd_launch3(const BwdParams& p, int stage, hipStream_t st) {
   const dim3 grid((p.N + 32 * R * W - 1) / (32 * R * W), p.BH);
   if constexpr (!B && DP <= 64) {
     // an under-filled grid (short sequences, few heads): the key (dq) or row (dK/dV) loop cut into p.split
-    // ranges over grid z, fp32 partials summed by a combine launch.  pair: work-groups of two wave groups, at
-    // most one per CU, that take two ranges each and add them in LDS, where that leaves no partials (and
-    // the ranges would occupy more than half the CUs anyway) or the ranges would go two to a CU.  Whole
-    // backward ms, fp16 d64: B8 H3 N1025 0.0614 -> 0.0501, N577 0.0382 -> 0.0314, 4K 0.150 -> 0.137, B2 H8 1K
-    // 0.0482 -> 0.0434, B4 H3 N1025 0.0470 -> 0.0409, 2K 0.0638 -> 0.0593; but N512 0.0235 -> 0.0254 and 1K
-    // 0.0349 -> 0.0364 (the pairs share half as many CUs).  Causal splits keep one range per work-group:
-    // two to a CU they balance.
-    const int64_t wgs = (int64_t)grid.x * grid.y, ranges = wgs * p.split;
-    const bool pair = p.split % 2 == 0 && !p.causal && ranges <= 512 && ranges > (p.split == 2 ? 128 : 256);
+    // ranges over grid z, fp32 partials summed by a combine launch, or taken in pairs (bwd_pairs)
+    const bool pair = bwd_pairs(std::is_same<T, f16>::value ? ELSA_F16 : ELSA_BF16, p.split, p.BH, p.N, p.causal != 0);
     if (p.split > 1) {
       BwdParams ps = p;
       if (pair) ps.split = p.split / 2;

@@ -132,6 +132,12 @@ struct BwdParams {
 // for fp32); ragged fp32 and 16-bit d64 grids without a causal mask, and fp32 at D = 128, by the rounds
 // they take.  Biased calls and 16-bit head dims above 64 keep 1.
 int bwd_splits(int dtype, int dp, int64_t bh, int64_t n, bool bias, bool causal);
+// Whether work-groups of two wave groups take the ranges of that split two at a time.
+bool bwd_pairs(int dtype, int split, int64_t bh, int64_t n, bool causal);
+// fp32 partials of each gradient that such a split writes (1: none): its ranges, or half of them in pairs.
+int bwd_partials(int dtype, int dp, int64_t bh, int64_t n, bool bias, bool causal);
+// What elsa_bwd asks of its workspace: elsa_bwd_workspace_bytes without the partials that pairs do not write.
+size_t bwd_workspace_written(const elsa_bwd_args* a);
 
 // stage < 0: preprocess, dq and dk/dv; 0: preprocess only; 1: dq only; 2: dk/dv only.
 hipError_t launch_bwd(const BwdParams& p, int dtype, int stage, hipStream_t stream);

@@ -20,6 +20,10 @@
 
 #include "elsa_hip.h"
 
+namespace elsa {  // libelsa_hip.so (elsa_internal.h)
+size_t bwd_workspace_written(const elsa_bwd_args* a);
+}
+
 namespace {
 
 using torch::autograd::AutogradContext;
@@ -160,7 +164,7 @@ at::Tensor bwd_call(const at::Tensor& q, const at::Tensor& k, const at::Tensor& 
   b.dk_layout = layout_of(dk);
   b.dv_layout = layout_of(dv);
   if (!bias.defined() || !dbias_wanted) {
-    const size_t ws_bytes = elsa_bwd_workspace_bytes(&b);
+    const size_t ws_bytes = elsa::bwd_workspace_written(&b);
     const at::Tensor ws = bytes(q, ws_bytes);
     b.workspace = ws.data_ptr();
     b.workspace_bytes = ws_bytes;

@@ -172,6 +172,8 @@ int elsa_fwd_noalloc(const elsa_fwd_args* args, void* stream);
 int elsa_phase1(const elsa_fwd_args* args, int32_t q_start, int32_t q_len, void* stream);
 int elsa_phase2(const elsa_fwd_args* args, int32_t q_start, int32_t q_len, void* stream);
 
+/* Enough for elsa_bwd: D and LSE2 of every row and three fp32 partials per range of a split (calls whose
+ * ranges are added in LDS write fewer). */
 size_t elsa_bwd_workspace_bytes(const elsa_bwd_args* args);
 /* dq, dk, dv from the saved row state (exact recompute of p). */
 int elsa_bwd(const elsa_bwd_args* args, void* stream);

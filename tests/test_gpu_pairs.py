@@ -51,3 +51,23 @@ def test_backward_against_fp64(dt, shape, causal):
             size[i] += (want[i].norm() + other[i]).item() ** 2
     for name, e, sz in zip(("dq", "dk", "dv"), err, size):
         assert (e / sz) ** 0.5 <= BOUND[dt], (name, (e / sz) ** 0.5)
+
+
+@pytest.mark.parametrize("shape,partials", [((8, 3, 1025, 64), 0), ((2, 8, 1024, 32), 2), ((4, 8, 1024, 32), 0),
+                                            ((4, 3, 1025, 64), 2), ((1, 8, 1024, 64), 4)])
+def test_backward_allocates_no_partials_that_pairs_do_not_write(shape, partials):
+    q, k, v, do = (torch.randn(shape, device="cuda").half() for _ in range(4))
+    for t in (q, k, v):
+        t.requires_grad_(True)
+    for _ in range(2):  # the first pass also loads code and starts the engine
+        out = elsa_amd.twopass_attention_train(q, k, v)
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        grads = torch.autograd.grad(out, (q, k, v), do)
+        peak = torch.cuda.max_memory_allocated() - before
+    rows = shape[0] * shape[1] * shape[2]
+    # three gradients, three floats per row, the partials; each allocation rounded up to at most 2 MiB
+    expect = 3 * q.numel() * 2 + 3 * rows * 4 + 3 * partials * q.numel() * 4
+    assert expect <= peak <= expect + (8 << 20), (peak, expect)
+    assert all(g.isfinite().all() for g in grads)
