@@ -1761,9 +1761,15 @@ static hipError_t launch1h_wb(const Phase1Params& p, int block_m, hipStream_t st
     if (!b && !p.causal && p.part_len < 1024 && (int64_t)((p.N + 255) / 256) * p.BH * p.P <= 512)
       return launch1h<T, DP, 1, 4, false>(p, st);
     // Causal calls below 16K keys too: their work-groups differ in length, and the diagonal blocks waste half as
-    // much.  Forward ms, bf16: B2 H8 N4097 0.0676 -> 0.0623, 8K 0.1018 -> 0.0968, B4 H8 4K 0.1038 -> 0.0987, B8 H3 N4097
-    // 0.0873 -> 0.0853, B2 H12 N3000 0.0569 -> 0.0532, d32 B2 H8 N4097 0.0536 -> 0.0413; 16K 0.322 -> 0.334.
-    if (!b && p.causal && p.part_len % 128 == 0 && p.N < 16384) return launch1h<T, DP, 1, 4, false>(p, st);
+    // much.  At D = 64 up to 1024 row blocks (two per slot of the chip: 512 of these work-groups run at once) and 6K
+    // keys per slot on average; past either the last work-groups' lengths no longer matter and the K/V fragments
+    // that a 64-row wave shares between its tiles do.  Forward ms, bf16, 256-row blocks -> these: d64 B2 H8 N4097 0.0676 -> 0.0623, 8K
+    // 0.1018 -> 0.0968, B2 H12 N3000 0.0569 -> 0.0532, d32 B2 H8 N4097 0.0536 -> 0.0413; but d64 H16 8K 0.175 -> 0.182,
+    // H32 8K 0.324 -> 0.359, H8 N16383 0.321 -> 0.340, d48 H16 12K 0.316 -> 0.361, H64 N3000 0.105 -> 0.113 keep 256 rows.  D = 32 gains or is
+    // level throughout (H16 8K 1.12 times as fast, H48 8K 1.04).
+    const int64_t rows = (int64_t)p.BH * p.N;
+    const bool narrow = DP == 32 || (rows <= 1024 * 128 && rows * p.N <= int64_t(6144) * 512 * 256);
+    if (!b && p.causal && p.part_len % 128 == 0 && p.N < 16384 && narrow) return launch1h<T, DP, 1, 4, false>(p, st);
     // the planner gives biased calls 128-row blocks (phase1_block_m); the grid follows the kernel
     return b ? launch1h<T, DP, 1, 4, true>(p, st) : launch1h<T, DP, 2, 4, false>(p, st);
   } else {

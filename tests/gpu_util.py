@@ -96,3 +96,15 @@ def assert_parity(got, exact, ref, tol: float, what: str = "", dtype: str = "fp1
     assert d_ref <= bar_ref, (what, info)
     assert e_got <= bar_exact, (what, info)
     return info
+
+
+def kernel_names(fn) -> list:
+    """Names of the kernels that fn launches."""
+    from torch.profiler import ProfilerActivity, profile
+
+    fn()
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        fn()
+        torch.cuda.synchronize()
+    return [e.name for e in prof.events() if e.device_type == torch.autograd.DeviceType.CUDA]
