@@ -355,9 +355,15 @@ void phase1_x3_kernel(const Phase1Params p) {
   constexpr int TCH = KT * CPR;      // chunks per stage tile
   static_assert((2 * TCH) % NT == 0 && TCH % 64 == 0, "whole chunks per thread, whole waves per tensor");
   constexpr int NCH = 2 * TCH / NT;  // chunks per thread, K's first
+  // 2 waves at D = 64 (at most 64 rows and mostly one or two stages): one buffer of 24 KB, so that LDS holds as
+  // many work-groups of a CU as its registers (4; with two buffers 3, and 1000 windows were a second round).
+  // Forward ms, two buffers -> one (fp32 MFMA fold before): 1000 windows N16 0.0135 -> 0.0092 (0.0098), N33 0.0194
+  // -> 0.0135 (0.0167), N49 0.0210 -> 0.0159 (0.0191), 3000 N64 0.0435 -> 0.0414 (0.0523); level up to 700.  D <= 32,
+  // where two buffers fit, is 2% slower with one.
+  constexpr int NBUF = WAVES == 2 && DP == 64 ? 1 : 2;
 
-  __shared__ __attribute__((aligned(16))) bf16 Kp[2][3][KT * KS];
-  __shared__ __attribute__((aligned(16))) bf16 Vp[2][3][KT * KS];
+  __shared__ __attribute__((aligned(16))) bf16 Kp[NBUF][3][KT * KS];
+  __shared__ __attribute__((aligned(16))) bf16 Vp[NBUF][3][KT * KS];
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 31, g = lane >> 5;
@@ -466,7 +472,7 @@ void phase1_x3_kernel(const Phase1Params p) {
   sstore(0);
   __syncthreads();
   for (int it = 0; it < ntiles; ++it) {
-    const int buf = it & 1, t0 = k_begin + it * KT;
+    const int buf = NBUF == 1 ? 0 : it & 1, t0 = k_begin + it * KT;
     const bool has_next = it + 1 < ntiles;
     if (has_next) gload(t0 + KT);
     if (!p.causal || t0 <= row0 + 31) {  // a causal wave whose rows all precede this stage adds nothing
@@ -551,7 +557,10 @@ void phase1_x3_kernel(const Phase1Params p) {
         oacc[dt] += st;
       }
     }
-    if (has_next) sstore(buf ^ 1);
+    if (has_next) {
+      if constexpr (NBUF == 1) __syncthreads();  // every wave has read this stage
+      sstore(NBUF == 1 ? 0 : buf ^ 1);
+    }
     __syncthreads();
   }
 

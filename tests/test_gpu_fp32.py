@@ -123,3 +123,17 @@ def test_fp32_strided_operands_match_dense_ones():
         res.append((out.detach(), *torch.autograd.grad(out, (q, k, v), do)))
     for a, b in zip(*res):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("n", [1, 9, 31, 32, 33, 49, 64])
+@pytest.mark.parametrize("causal", [False, True])
+def test_fp32_short_windows_against_fp64(n, causal):
+    # one 32-key stage, two, and a ragged second one; more windows than run at once
+    q, k, v, do = _inputs((1100, 1, n, 64), n)
+    out = elsa_amd.twopass_attention(q, k, v, is_causal=causal)
+    ex = _exact(q, k, v, do, None, causal)[0][0]
+    assert ((out.double() - ex).norm() / ex.norm()).item() <= BOUND
+    bias = torch.randn((1, 1, n, n), generator=torch.Generator(device="cuda").manual_seed(n), device="cuda")
+    out = elsa_amd.twopass_attention(q, k, v, bias=bias, is_causal=causal)
+    ex = _exact(q, k, v, do, bias, causal)[0][0]
+    assert ((out.double() - ex).norm() / ex.norm()).item() <= BOUND
