@@ -1475,8 +1475,9 @@ static hipError_t bwd_launch3(const BwdParams& p, int stage, hipStream_t st) {
     }
     if constexpr (DP == 128 && !B) {
       // at most one 4-wave work-group per CU: two groups of waves on alternate stages (B2 H8 2K dq 0.0745 ->
-      // 0.0648 ms, B1 H4 N1000 0.0342 -> 0.0305)
-      if ((wide = (int64_t)grid.x * grid.y <= 256))
+      // 0.0648 ms, B1 H4 N1000 0.0342 -> 0.0305).  Not for one or two stages, where the exchange costs what the
+      // second group saves (whole backward bf16 H8 N128 0.0262 ms against 0.0245, N96 0.0246 and 0.0236; N129 level).
+      if ((wide = p.N > 128 && (int64_t)grid.x * grid.y <= 256))
         hipLaunchKernelGGL((bwd_dq_half_kernel<T, DP, R, W, false, false, 2>), grid, dim3(128 * W), 0, st, p);
     }
     if (!wide) {
@@ -1489,7 +1490,10 @@ static hipError_t bwd_launch3(const BwdParams& p, int stage, hipStream_t st) {
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
   if constexpr (DP == 128 && !B) {
-    if ((stage < 0 || stage == 2) && (int64_t)p.N * p.qs[2] * es < lim && (int64_t)p.N * p.gs[2] * es < lim)
+    // (at most 64 rows: two stages, of which each of its wave groups would take one, and an exchange of 64 KB; dk/dv
+    // bf16 H8 N64 about 2 us more than with the kernel below.  From 65 rows it gains: whole backward H8 N96 0.0246 ->
+    // 0.0236 ms)
+    if ((stage < 0 || stage == 2) && p.N > 64 && (int64_t)p.N * p.qs[2] * es < lim && (int64_t)p.N * p.gs[2] * es < lim)
       return launch_dkdv_d128(p, std::is_same<T, f16>::value ? ELSA_F16 : ELSA_BF16, st);
   }
   if (stage < 0 || stage == 2) {
