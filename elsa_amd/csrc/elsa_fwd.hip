@@ -1805,14 +1805,17 @@ static hipError_t launch1x3(const Phase1Params& p, hipStream_t st) {
 
 // Waves of the fp32 fold.  64-row blocks: 2 (head dims above 64 keep the fp32 MFMA, whose LDS leaves
 // room for several of these small work-groups: B64 H8 N64 d128 0.023 against 0.032 ms).  Otherwise 8
-// waves (256 rows), whose stage is split once for twice the rows, where the 256-row work-groups still
-// fill the chip (one per CU) in no more rounds than the 128-row ones (two per CU) and, for a causal
-// call, whole row blocks make up a partition (its longest-first order): forward d64 16K 2.92 -> 2.72
-// ms, 4K 0.200 -> 0.187, B8 H3 N1025 0.0562 -> 0.0539, causal 4K 0.121 -> 0.115; but B2 H8 N4097 with two
-// partitions (544 work-groups, a third round for 32) 0.456 -> 0.493, B4 H12 N577 0.040 -> 0.060 and
-// causal B1 H3 N5000 (640-key partitions) 0.081 -> 0.094 stay on 4.  Head dims above 64: one wave per
-// SIMD at 4 waves, two at 8 (4K 0.449 -> 0.343 ms); at most 256 rows or fewer than 128 work-groups of
-// 256 keep 4 there (B2 H3 N197 0.017 against 0.021 ms).
+// waves (256 rows, one work-group per CU), whose stage is split once for twice the rows, where their rounds of
+// the chip take less time than those of the 4-wave work-groups (128 rows).  At D = 64 two of the latter share a
+// CU, and an odd one alone takes 0.645 of a round, as in the backward: forward d64 16K 2.92 -> 2.72 ms, 4K 0.200
+// -> 0.187, B8 H3 N1025 0.0562 -> 0.0539; but B2 H8 N4097 in two partitions 0.456 -> 0.493, H96 N100 0.0129 -> 0.0149,
+// H48 N300 0.0252 -> 0.0333, H24 N513 0.0261 -> 0.0361, B4 H12 N577 0.040 -> 0.060 and H48 N129 (144 work-groups of
+// 8) 0.0136 -> 0.0146 stay on 4.  Causal calls
+// there: 8 where they fill the chip in no more rounds and whole row blocks make up a partition (its longest-first
+// order): causal 4K 0.121 -> 0.115, but B1 H3 N5000 (640-key partitions) 0.081 -> 0.094 stays on 4.  Head dims
+// above 64: one 4-wave work-group per CU takes 0.6 to 0.8 of the time of an 8-wave one (4K 0.449 -> 0.343 ms with
+// 8, H200 N197 0.062 -> 0.040, H96 N197 0.0465 -> 0.0381; but H16 N257 0.0210 -> 0.0261 and H48 N257 0.0405 -> 0.0522
+// stay on 4); causal ones, whose rounds hold work-groups without keys, 8 from 128 work-groups.
 template <int DP>
 static hipError_t launch1_f32_wb(const Phase1Params& p, int block_m, hipStream_t st) {
   const bool b = p.bias.ptr != nullptr;
@@ -1825,8 +1828,15 @@ static hipError_t launch1_f32_wb(const Phase1Params& p, int block_m, hipStream_t
   }
   if constexpr (DP >= 64) {
     const int64_t w4 = (int64_t)((p.q_len + 127) / 128) * p.BH * p.P, w8 = (int64_t)((p.q_len + 255) / 256) * p.BH * p.P;
-    const bool fills = w8 >= 192 && (w8 + 255) / 256 <= (w4 + 511) / 512 && (!p.causal || p.part_len % 256 == 0);
-    if (DP == 128 ? p.q_len > 256 && w8 >= 128 : fills) return b ? launch1x3<DP, 8, true>(p, st) : launch1x3<DP, 8, false>(p, st);
+    const int64_t k4 = (w4 + 255) / 256, k8 = (w8 + 255) / 256;
+    bool eight;
+    if (p.causal) {
+      eight = DP == 128 ? p.q_len > 256 && w8 >= 128 : w8 >= 192 && k8 <= (w4 + 511) / 512 && p.part_len % 256 == 0;
+    } else {
+      eight = DP == 128 ? (double)k8 < 0.8 * (double)k4
+                        : w8 >= 192 && 0.94 * (double)k8 < (double)(k4 / 2) + (k4 % 2 ? 0.645 : 0.0);
+    }
+    if (eight) return b ? launch1x3<DP, 8, true>(p, st) : launch1x3<DP, 8, false>(p, st);
   }
   return b ? launch1x3<DP, 4, true>(p, st) : launch1x3<DP, 4, false>(p, st);
 }

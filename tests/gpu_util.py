@@ -4,6 +4,7 @@ from __future__ import annotations
 
 import json
 import os
+import re
 
 import numpy as np
 import torch
@@ -98,8 +99,9 @@ def assert_parity(got, exact, ref, tol: float, what: str = "", dtype: str = "fp1
     return info
 
 
-def kernel_names(fn) -> list:
-    """Names of the kernels that fn launches."""
+def kernels_run(fn) -> list:
+    """(name, template arguments) of the kernels that fn launches: types as f16 / bf16 / f32, numbers and flags as
+    int.  The profiler gives a name mangled where its demangler does not know a type (bf16)."""
     from torch.profiler import ProfilerActivity, profile
 
     fn()
@@ -107,4 +109,17 @@ def kernel_names(fn) -> list:
     with profile(activities=[ProfilerActivity.CUDA]) as prof:
         fn()
         torch.cuda.synchronize()
-    return [e.name for e in prof.events() if e.device_type == torch.autograd.DeviceType.CUDA]
+    types = {"DF16b": "bf16", "DF16_": "f16", "f": "f32", "__bf16": "bf16", "_Float16": "f16", "float": "f32",
+             "true": 1, "false": 0}
+    out = []
+    for name in (e.name for e in prof.events() if e.device_type == torch.autograd.DeviceType.CUDA):
+        m = re.match(r"_ZN4elsa\d+(\w+?_kernel)(?:I(.*?)EE?v)?", name)
+        if m:
+            args = re.findall(r"L[ib](\d+)E|(DF16b|DF16_|f)", (m.group(2) or "") + "E")
+            out.append((m.group(1), [int(n) if n else types[t] for n, t in args]))
+            continue
+        m = re.match(r"(?:void )?elsa::(\w+_kernel)(?:<([^>]*)>)?", name)
+        if m:
+            args = [a.strip() for a in (m.group(2) or "").split(",") if a.strip()]
+            out.append((m.group(1), [types[a] if a in types else int(a) for a in args]))
+    return out

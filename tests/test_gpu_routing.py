@@ -1,11 +1,11 @@
-"""Which kernel (by its mangled name) a call runs, at the lines that the launchers' rules draw, and its result on both sides of them."""
+"""Which kernel a call runs, at the lines that the launchers' rules draw, and its result on both sides of them."""
 from __future__ import annotations
 
 import pytest
 import torch
 
 import elsa_amd
-from gpu_util import TORCH_DT, kernel_names
+from gpu_util import TORCH_DT, kernels_run
 
 pytestmark = pytest.mark.gpu
 
@@ -30,9 +30,9 @@ def _exact_rows(q, k, v, rows, causal):
                                          ((1, 32, 8192, 32), 1)])
 def test_causal_forward_blocks(shape, tiles):
     q, k, v = _inputs(shape, "bf16", 3)
-    names = kernel_names(lambda: elsa_amd.twopass_attention(q, k, v, is_causal=True))
-    dp = 32 if shape[3] <= 32 else 64
-    assert any(f"phase1_half_kernelIDF16bLi{dp}ELi{tiles}ELi4E" in n for n in names), names
+    run = kernels_run(lambda: elsa_amd.twopass_attention(q, k, v, is_causal=True))
+    want = ["bf16", 32 if shape[3] <= 32 else 64, tiles, 4]
+    assert any(name == "phase1_half_kernel" and args[:4] == want for name, args in run), run
     out = elsa_amd.twopass_attention(q, k, v, is_causal=True)
     n = shape[2]
     rows = torch.tensor([0, 1, 127, 128, 255, 256, 511, 512, n // 2, n - 129, n - 2, n - 1], device="cuda")
@@ -51,10 +51,9 @@ def test_head_dim_128_backward(dtype, shape, causal, groups, dq_groups):
     for t in (q, k, v):
         t.requires_grad_(True)
     out = elsa_amd.twopass_attention_train(q, k, v, is_causal=causal)
-    names = kernel_names(lambda: torch.autograd.grad(out, (q, k, v), do, retain_graph=True))
-    assert any("bwd_dkdv_d128_kernel" in x for x in names) == groups, names
-    assert any("bwd_dkdv_half_kernel" in x for x in names) != groups, names
-    assert any("bwd_dq_half_kernel" in x and f"Lb0ELi{dq_groups}EE" in x for x in names), names
+    run = dict(kernels_run(lambda: torch.autograd.grad(out, (q, k, v), do, retain_graph=True)))
+    assert ("bwd_dkdv_d128_kernel" in run) == groups and ("bwd_dkdv_half_kernel" in run) != groups, run
+    assert run["bwd_dq_half_kernel"][1] == 128 and run["bwd_dq_half_kernel"][-1] == dq_groups, run
     dq, dk, dv = torch.autograd.grad(out, (q, k, v), do)
     c, (q64, k64, v64, do64) = shape[3] ** -0.5, (t.detach().double() for t in (q, k, v, do))
     s = torch.matmul(q64, k64.transpose(-1, -2).contiguous()) * c
@@ -70,3 +69,17 @@ def test_head_dim_128_backward(dtype, shape, causal, groups, dq_groups):
     assert ((dq.double() - want_q).norm() / (want_q.norm() + other_q.norm())).item() <= bound
     assert ((dk.double() - want_k).norm() / (want_k.norm() + other.norm())).item() <= bound
     assert ((dv.double() - want_v).norm() / want_v.norm()).item() <= bound
+
+
+# fp32 forwards: 4 or 8 waves by the rounds of the chip (partitions by the planner)
+@pytest.mark.parametrize("shape,waves", [((1, 96, 100, 64), 4), ((1, 48, 300, 64), 4), ((1, 24, 513, 64), 4),
+                                         ((8, 3, 1025, 64), 8), ((1, 8, 4096, 64), 8), ((1, 16, 257, 128), 4),
+                                         ((1, 48, 257, 128), 4), ((1, 200, 197, 128), 8), ((1, 8, 2048, 128), 8)])
+def test_fp32_forward_waves(shape, waves):
+    q, k, v = _inputs(shape, "fp32", 3)
+    run = dict(kernels_run(lambda: elsa_amd.twopass_attention(q, k, v)))
+    assert run["phase1_x3_kernel"][:2] == [shape[3], waves], run
+    out = elsa_amd.twopass_attention(q, k, v)
+    rows = torch.unique(torch.tensor([0, 31, 32, 99, shape[2] // 2, shape[2] - 1], device="cuda"))
+    ex = _exact_rows(q, k, v, rows, False)
+    assert ((out[:, :, rows].double() - ex).norm() / ex.norm()).item() <= 6e-7
