@@ -107,7 +107,8 @@ int plan_fwd(const elsa_fwd_args* a, elsa_fwd_plan* pl) {
                     !(a->dtype == ELSA_F16 && a->summary_dtype == ELSA_F32);
     // Unbiased fp16/bf16 calls without a causal mask, below 4K keys or at head dim 128: the count that minimises
     // rounds x (partition keys + 100) + the merge.  A CU runs two work-groups together in one round, an odd
-    // one alone in 0.555 of it; 100 keys for a work-group's fixed cost; Phase 2: 2 us for its launch and 0.108
+    // one alone in 0.555 of it (0.62 at head dims 65 to 127: d80 H16 N1500 0.0348 ms with 2 partitions, 0.0367 with 1, H6
+    // N2048 0.0270 with 4, 0.0288 with 2); 100 keys for a work-group's fixed cost; Phase 2: 2 us for its launch and 0.108
     // per work-group for its bytes (all in keys of one round: 0.0215 us for 128 rows at d64, 0.043 for 256 rows
     // or d128).  Ping-pong partitions: 0.64 x rounds of one work-group per CU x (partition keys + 768), as
     // below.  Forward ms against the 1024 target: fp16 B4 H8 1K 0.0202 -> 0.0162 (2 -> 1 partitions), B8 H8 1K
@@ -116,15 +117,25 @@ int plan_fwd(const elsa_fwd_args* a, elsa_fwd_plan* pl) {
     // H8 1K 0.0583 -> 0.0461 (2 -> 1), B1 H8 4K 0.0907 -> 0.0850 (4 -> 2); B2 H8 2K, B2 H3 N3000 and B12 H8 N1111 keep
     // 4, 5 and 2
     if (by_rounds && a->dtype != ELSA_F32 && !a->is_causal && !a->bias.ptr && (n < 4096 || dp > 64)) {
+      double lone = dp > 64 && d < 128 ? 0.62 : 0.555;
       auto cost = [&](int64_t c) {
         const int64_t len = cdiv(cdiv(n, c), kt) * kt, parts = cdiv(n, len), wgs = q_tiles * parts, k = cdiv(wgs, 256);
         const double merge = c > 1 ? (bm == 256 || dp > 64 ? 45 : 90) + 0.108 * (double)wgs : 0.0;
         if (pp && len >= 1024) return 0.64 * (double)(cdiv(bh * cdiv(q_rows, 512) * parts, 256) * (len + 768)) + merge;
-        return ((double)(k / 2) + (k % 2 ? 0.555 : 0.0)) * (double)(len + 100) + merge;
+        return ((double)(k / 2) + (k % 2 ? lone : 0.0)) * (double)(len + 100) + merge;
       };
       p = 1;
       for (int64_t c = 2; c <= n / 512; ++c)
         if (cost(c) < cost(p)) p = c;
+      // head dims above 64 under 192 work-groups: partitions down to 128 keys, at most one work-group per CU, where
+      // they pay for the merge (a lone one takes 0.62).  fp16: d128 B2 H4 N1000 0.0287 -> 0.0192 (1 -> 4), B1 H6 N1025
+      // 0.0203 -> 0.0177 (2 -> 4); filled to 256 work-groups regardless, H24 N700 0.0218 -> 0.0244 (1 -> 2), H24 N513 0.0192
+      // -> 0.0207 (1 -> 3; 0.0181 with 2) and H1 N2048 0.0193 -> 0.0207 (4 -> 16)
+      if (dp > 64 && n >= 512 && q_tiles * p < 192) {
+        lone = 0.62;
+        for (int64_t c = p + 1; c <= n / 128 && q_tiles * c <= 256; ++c)
+          if (cost(c) < cost(p)) p = c;
+      }
     }
     if (a->dtype == ELSA_F32) {
       // fp32 from 1024 keys without a causal mask, where the 1024 work-group target leaves the last round of
@@ -157,8 +168,7 @@ int plan_fwd(const elsa_fwd_args* a, elsa_fwd_plan* pl) {
     // -> 0.010 (2 -> 4 partitions), N512 0.0099 -> 0.0084 (1 -> 4), causal N1025 0.0139 -> 0.0121
     // (3 -> 5); B8 H3 N1025 (240 work-groups) keeps its two (5: 0.026 against 0.021 ms), and shorter
     // sequences their one fused partition (B8 H3 N197: more measured slower)
-    // (d128 B2 H4 N1000 0.0287 -> 0.0192, 1 -> 4)
-    if (a->dtype != ELSA_F32 && (dp <= 64 || (!a->is_causal && !a->bias.ptr)) && n >= 512 && q_tiles * p < 192)
+    if (a->dtype != ELSA_F32 && dp <= 64 && n >= 512 && q_tiles * p < 192)
       p = std::max<int64_t>(p, std::min<int64_t>(cdiv(256, q_tiles), std::max<int64_t>(1, n / 128)));
     if (n >= 8192) p = std::max<int64_t>(p, 2);
     // causal from 8K keys: partitions of n/4 keys within [2048, 8192].  About half of the

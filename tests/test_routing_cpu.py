@@ -92,3 +92,25 @@ def test_fp32_partials_stay_below_512_mib():
                 for causal in (False, True):
                     need, rows = _bwd_workspace(_lib.ELSA_F32, 1, bh, n, d, causal)
                     assert need - rows <= 512 << 20, (d, bh, n, causal, need)
+
+
+# fp16 forwards above head dim 64: partitions where they pay for their merge (ms with the count before and after)
+@pytest.mark.parametrize("h,n,d,parts", [
+    (24, 700, 128, 1),   # 0.0244 with 2, 0.0218
+    (24, 513, 128, 2),   # 0.0207 with 3, 0.0181
+    (32, 513, 128, 1),   # 0.0222 with 2, 0.0193
+    (6, 2048, 80, 4),    # 0.0288 with 2, 0.0270
+    (16, 1500, 80, 2),   # 0.0367 with 1, 0.0348
+    (8, 1000, 128, 4),   # 0.0287 with 1, 0.0192
+    (16, 2048, 128, 1)]) # 0.0577 with 4, 0.0498
+def test_wide_head_forward_partitions(h, n, d, parts):
+    assert _plan(_fwd_args(_lib.ELSA_F16, 1, h, n, d)).partitions == parts
+
+
+def test_wide_head_forwards_keep_one_work_group_per_cu_or_partitions_of_512_keys():
+    for h in (1, 2, 3, 6, 8, 12, 16, 24, 48):
+        for n in (512, 600, 1025, 2048, 4095, 8192):
+            for d in (72, 80, 128):
+                plan = _plan(_fwd_args(_lib.ELSA_BF16, 1, h, n, d))
+                wgs = h * -(-n // plan.block_m) * plan.partitions
+                assert plan.partitions == 1 or plan.partition_len >= 512 or (wgs <= 256 and plan.partition_len >= 128)
