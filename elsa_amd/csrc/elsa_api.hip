@@ -486,9 +486,9 @@ elsa::BwdParams bwd_params(const elsa_bwd_args* a) {
   p.lse_lo = reinterpret_cast<float*>(base + 2 * align256(rows * 4));
   p.dp = elsa::pad_head_dim(a->head_dim);
   p.split = elsa::bwd_splits(a->dtype, p.dp, p.BH, p.N, a->bias.ptr != nullptr, a->is_causal != 0);
-  const int partials = elsa::bwd_partials(a->dtype, p.dp, p.BH, p.N, a->bias.ptr != nullptr, a->is_causal != 0);
-  p.part = partials > 1 ? reinterpret_cast<float*>(base + 3 * align256(rows * 4)) : nullptr;
-  p.part_stride = (int64_t)(align256((size_t)partials * rows * p.dp * 4) / 4);
+  p.partials = elsa::bwd_partials(a->dtype, p.dp, p.BH, p.N, a->bias.ptr != nullptr, a->is_causal != 0);
+  p.part = p.partials > 1 ? reinterpret_cast<float*>(base + 3 * align256(rows * 4)) : nullptr;
+  p.part_stride = (int64_t)(align256((size_t)p.partials * rows * p.dp * 4) / 4);
   const int H = a->heads, N = a->seq_len, D = a->head_dim;
   resolve_layout(a->q_layout, H, N, D, p.qs);
   resolve_layout(a->k_layout, H, N, D, p.ks);

@@ -1260,7 +1260,7 @@ int bwd_splits(int dtype, int dp, int64_t bh, int64_t n, bool bias, bool causal)
 // 0.0314, 4K 0.150 -> 0.137, B2 H8 1K 0.0482 -> 0.0434, B4 H3 N1025 0.0470 -> 0.0409, 2K 0.0638 -> 0.0593; but
 // N512 0.0235 -> 0.0254 and 1K 0.0349 -> 0.0364 (the pairs share half as many CUs).  Causal splits keep one
 // range per work-group: two to a CU they balance.
-bool bwd_pairs(int dtype, int split, int64_t bh, int64_t n, bool causal) {
+static bool bwd_pairs(int dtype, int split, int64_t bh, int64_t n, bool causal) {
   const int64_t ranges = bh * ((n + 127) / 128) * split;
   return dtype != ELSA_F32 && !causal && split % 2 == 0 && ranges <= 512 && ranges > (split == 2 ? 128 : 256);
 }
@@ -1373,11 +1373,11 @@ static hipError_t bwd_launch3(const BwdParams& p, int stage, hipStream_t st) {
   const dim3 grid((p.N + 32 * R * W - 1) / (32 * R * W), p.BH);
   if constexpr (!B && DP <= 64) {
     // an under-filled grid (short sequences, few heads): the key (dq) or row (dK/dV) loop cut into p.split
-    // ranges over grid z, fp32 partials summed by a combine launch, or taken in pairs (bwd_pairs)
-    const bool pair = bwd_pairs(std::is_same<T, f16>::value ? ELSA_F16 : ELSA_BF16, p.split, p.BH, p.N, p.causal != 0);
+    // ranges over grid z, fp32 partials summed by a combine launch, or taken in pairs
+    const bool pair = p.partials != p.split;
     if (p.split > 1) {
       BwdParams ps = p;
-      if (pair) ps.split = p.split / 2;
+      ps.split = p.partials;
       const dim3 gs(grid.x, grid.y, (unsigned)ps.split);
       const CombineOut cq{p.part, p.dq, {p.dqs[0], p.dqs[1], p.dqs[2]}, p.scale};
       const CombineOut ck{p.part + p.part_stride, p.dk, {p.dks[0], p.dks[1], p.dks[2]}, p.scale};

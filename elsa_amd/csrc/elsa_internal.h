@@ -121,7 +121,9 @@ struct BwdParams {
   // split > 1 (bwd_splits): the dq and dK/dV kernels deal the stages of their key (dq) or row (dK/dV) loop
   // out over `split` work-groups (grid z) in turn, and write unscaled fp32 partials, [split][BH][N][dp] each
   // for dq, dK and dV from part on; a combine kernel sums them
-  int split, dp;
+  // partials: how many of them each gradient gets: split, or half of it where work-groups of two wave groups
+  // take the ranges two at a time (bwd_partials); part is null where that leaves none (1)
+  int split, partials, dp;
   float* part;
   int64_t part_stride;  // floats from the dq partials to the dK ones and from those to the dV ones
 };
@@ -132,9 +134,8 @@ struct BwdParams {
 // for fp32); ragged fp32 and 16-bit d64 grids without a causal mask, and fp32 at D = 128, by the rounds
 // they take.  Biased calls and 16-bit head dims above 64 keep 1.
 int bwd_splits(int dtype, int dp, int64_t bh, int64_t n, bool bias, bool causal);
-// Whether work-groups of two wave groups take the ranges of that split two at a time.
-bool bwd_pairs(int dtype, int split, int64_t bh, int64_t n, bool causal);
-// fp32 partials of each gradient that such a split writes (1: none): its ranges, or half of them in pairs.
+// fp32 partials of each gradient that such a split writes (1: none): its ranges, or half of them where
+// work-groups of two wave groups take them two at a time.
 int bwd_partials(int dtype, int dp, int64_t bh, int64_t n, bool bias, bool causal);
 // What elsa_bwd asks of its workspace: elsa_bwd_workspace_bytes without the partials that pairs do not write.
 size_t bwd_workspace_written(const elsa_bwd_args* a);
