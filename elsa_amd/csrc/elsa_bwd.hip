@@ -565,7 +565,7 @@ void bwd_dkdv_half_kernel(const BwdParams p) {
   constexpr int RTS = WAVES == 8 ? 128 : Tile::ST, KS = Tile::KS, CPR = Tile::CPR;
   constexpr int NKK = DP / 16, NDT = DP / 32;
   constexpr int NT = 64 * WAVES, KEYS_W = 32 * KRT, BN = KEYS_W * WAVES;
-  static_assert((RTS * CPR) % NT == 0, "staging must divide evenly");
+  static_assert((RTS * CPR) % NT == 0 && NT % CPR == 0, "staging must divide evenly");
   constexpr int NCH = RTS * CPR / NT;
   static_assert(!LD || ((WAVES == 4 || WAVES == 8) && KRT == 1 && DP == 64 && !HAS_BIAS && Tile::SWZ && NCH == 2),
                 "LDS-direct staging: the one-tile D = 64 kernels");
@@ -637,14 +637,10 @@ void bwd_dkdv_half_kernel(const BwdParams p) {
 
   // element offsets of this thread's staging chunks inside a stage (row strides are
   // below 2^25 elements, checked by the API, so the 128 rows of a stage fit in 32 unsigned bits)
-  uint32_t qoff[NCH], goff[NCH];
-  static_for<0, NCH>([&](auto I) {
-    constexpr int i = decltype(I)::value;
-    const int ci = tid + i * NT;
-    const int r = ci / CPR, d0 = (ci % CPR) * 8;
-    qoff[i] = (uint32_t)r * (uint32_t)p.qs[2] + (uint32_t)d0;
-    goff[i] = (uint32_t)r * (uint32_t)p.gs[2] + (uint32_t)d0;
-  });
+  // (chunk tid + NT i sits NT / CPR rows below chunk tid: one offset a tensor.  With one a chunk the 4-wave kernel at
+  // D = 64 spilled 28 bytes per lane and the 8-wave one 16)
+  const uint32_t qoff0 = (uint32_t)(tid / CPR) * (uint32_t)p.qs[2] + (uint32_t)(tid % CPR) * 8u;
+  const uint32_t goff0 = (uint32_t)(tid / CPR) * (uint32_t)p.gs[2] + (uint32_t)(tid % CPR) * 8u;
   // staging registers: set S holds one stage (RTS rows) on its way from global memory to LDS
   Chunk16 qreg[LD ? 1 : 2][LD ? 1 : NCH], greg[LD ? 1 : 2][LD ? 1 : NCH];
   float lreg[2] = {0.f, 0.f}, dreg[2] = {0.f, 0.f};
@@ -697,8 +693,8 @@ static_for<0, NCH>([&](auto I) {
       const int ci = tid + i * NT;
       const int r = ci / CPR, d0 = (ci % CPR) * 8;
       if (t0 + r < p.N && d0 < p.D) {
-        qreg[S][i] = *reinterpret_cast<const Chunk16*>(qt + qoff[i]);
-        greg[S][i] = *reinterpret_cast<const Chunk16*>(gt + goff[i]);
+        qreg[S][i] = *reinterpret_cast<const Chunk16*>(qt + (int64_t)(i * (NT / CPR)) * p.qs[2] + qoff0);
+        greg[S][i] = *reinterpret_cast<const Chunk16*>(gt + (int64_t)(i * (NT / CPR)) * p.gs[2] + goff0);
       } else {
         qreg[S][i] = Chunk16{};
         greg[S][i] = Chunk16{};

@@ -19,7 +19,11 @@ DT = {"fp16": torch.float16, "bf16": torch.bfloat16}
 # D = 128; then split grids in a ragged round and causal grids in both column layouts
 SHAPES = [((2, 8, 1024, 64), False), ((8, 3, 577, 64), False), ((5, 8, 513, 64), False), ((4, 3, 1025, 64), False),
           ((9, 4, 640, 32), False), ((1, 2, 60, 128), False), ((1, 4, 1000, 128), True), ((2, 3, 129, 80), False),
-          ((2, 8, 2200, 64), False), ((3, 3, 1200, 64), True), ((2, 8, 1100, 64), True)]
+          ((2, 8, 2200, 64), False), ((3, 3, 1200, 64), True), ((2, 8, 1100, 64), True),
+          # head dims that pad to 64 (staged through registers): pairs with no partials left and with two, a causal
+          # split, one range, 8-wave work-groups
+          ((8, 3, 577, 40), False), ((4, 3, 1025, 48), False), ((1, 8, 1100, 56), False), ((1, 8, 1100, 56), True),
+          ((4, 4, 197, 40), True), ((16, 8, 600, 48), False)]
 
 
 @pytest.mark.parametrize("dt", ["fp16", "bf16"])
