@@ -261,7 +261,7 @@ void bwd_dq_half_kernel(const BwdParams p) {
   // split (the 4-wave one-tile kernel only; 1 otherwise): work-group z takes the 64-key stages z, z + split,
   // ..., so that the ranges differ by at most one stage, under a causal mask too; one without a stage
   // writes zeros.  D = 128 never splits (bwd_splits) but keeps these run-time bounds: with constant
-  // ones its register allocation spilled (20 bytes per lane, 468 biased; 16K dq 1.698 -> 1.653 ms without)
+  // ones its register allocation spilled (20 bytes per lane unbiased; 16K dq 1.698 -> 1.653 ms without)
   const int k_lo = CAN_SPLIT ? (wg.z * G + grp) * KT : 0, k_step = CAN_SPLIT ? p.split * G * KT : KT;
   // -D of this lane's row: the dP^T product starts from it and yields dP - D directly.  The
   // 16 registers per row tile of that constant would spill in the bias, D = 128 and two-tile
@@ -377,6 +377,10 @@ static_for<0, NCH>([&](auto I) {
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt) acc[rt][dt] = f32x16{};
 
+  // Biased D = 128: dP after p, which has taken the place of S, and V's fragments only then.  Together with the 16
+  // bias values they spilled 152 bytes per lane (249 VGPRs and none so): whole backward fp16 B2 H8 1K d128 0.191 ->
+  // 0.171 ms, B8 H8 N256 0.0616 -> 0.0524.  D <= 64 has the registers and is 4% slower this way (d32).
+  constexpr bool LATE_DP = HAS_BIAS && DP == 128;
   const int ntiles = k_end > k_lo ? (k_end - k_lo + k_step - 1) / k_step : 0;
   // both groups meet every barrier: the first one's stages are the most
   const int nloop = G == 1 ? ntiles : max(0, (k_end - (int)wg.z * G * KT + k_step - 1) / k_step);
@@ -392,19 +396,25 @@ static_for<0, NCH>([&](auto I) {
 #pragma unroll
         for (int kk = 0; kk < NKK; ++kk) {
           kf[kk] = *reinterpret_cast<const F*>(krow + kk * 16);
-          vf[kk] = *reinterpret_cast<const F*>(vrow + kk * 16);
+          if constexpr (!LATE_DP) vf[kk] = *reinterpret_cast<const F*>(vrow + kk * 16);
         }
         F dsp[RT][2];  // dS of the sub-tile, rounded to T: the B operand of the dQ^T product
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
           f32x16 ds;
-          f32x16 s = M::mma(kf[0], qf[rt][0], f32x16{}), dp = M::mma(vf[0], gf[rt][0], ndd[rt]);
+          f32x16 s = M::mma(kf[0], qf[rt][0], f32x16{}), dp;
+          if constexpr (LATE_DP) {
 #pragma unroll
-          for (int kk = 1; kk < NKK; ++kk) {
-            s = M::mma(kf[kk], qf[rt][kk], s);
-            dp = M::mma(vf[kk], gf[rt][kk], dp);
+            for (int kk = 1; kk < NKK; ++kk) s = M::mma(kf[kk], qf[rt][kk], s);
+          } else {
+            dp = M::mma(vf[0], gf[rt][0], ndd[rt]);
+#pragma unroll
+            for (int kk = 1; kk < NKK; ++kk) {
+              s = M::mma(kf[kk], qf[rt][kk], s);
+              dp = M::mma(vf[kk], gf[rt][kk], dp);
+            }
+            if constexpr (MFMA_D) dp = M::mma(ones_a, nd_b[rt], dp);
           }
-          if constexpr (MFMA_D) dp = M::mma(ones_a, nd_b[rt], dp);
           const int my_row = row0 + rt * 32 + c;
           const bool full = (t0 + KT <= k_end) && (!p.causal || t0 + KT - 1 <= row0 + rt * 32);
           const float nl = -lse[rt];
@@ -417,9 +427,16 @@ static_for<0, NCH>([&](auto I) {
               const int key = t0 + sub * 32 + key_of_reg(r, g);
               const bool ok = live[rt] && key < k_end && (!p.causal || key <= my_row);
               const float x = fmaf(s[r], p.scale_log2, nl);
-              const float pr = ok ? fast_exp2(fmaf(bv[r], kLog2e, x)) : 0.f;
-              ds[r] = pr * (dp[r] - dd[rt]);
+              s[r] = ok ? fast_exp2(fmaf(bv[r], kLog2e, x)) : 0.f;
             }
+            if constexpr (LATE_DP) {
+              __builtin_amdgcn_sched_barrier(0);
+              dp = ndd[rt];
+#pragma unroll
+              for (int kk = 0; kk < NKK; ++kk) dp = M::mma(*reinterpret_cast<const F*>(vrow + kk * 16), gf[rt][kk], dp);
+            }
+#pragma unroll
+            for (int r = 0; r < 16; ++r) ds[r] = s[r] * (dp[r] - dd[rt]);
           } else {
 #pragma unroll
             for (int r = 0; r < 16; ++r) ds[r] = fast_exp2(fmaf(s[r], p.scale_log2, nl));

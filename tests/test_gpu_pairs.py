@@ -75,3 +75,35 @@ def test_backward_allocates_no_partials_that_pairs_do_not_write(shape, partials)
     expect = 3 * q.numel() * 2 + 3 * rows * 4 + 3 * partials * q.numel() * 4
     assert expect <= peak <= expect + (8 << 20), (peak, expect)
     assert all(g.isfinite().all() for g in grads)
+
+
+@pytest.mark.parametrize("dt", ["fp16", "bf16"])
+@pytest.mark.parametrize("shape,bias_bh,causal", [((2, 3, 100, 128), (1, 3), False), ((1, 2, 129, 128), (1, 2), True),
+                                                  ((2, 2, 200, 72), (2, 2), False), ((2, 2, 257, 64), (1, 2), True),
+                                                  ((3, 2, 130, 40), (1, 1), False), ((1, 4, 520, 128), (1, 4), False),
+                                                  ((70, 8, 256, 64), (1, 8), False)])
+def test_biased_backward_against_fp64(dt, shape, bias_bh, causal):
+    print(f"biased {dt} {shape} {bias_bh} causal={causal}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(sum(shape))
+    q, k, v, do = (torch.randn(shape, generator=g, device="cuda").to(DT[dt]) for _ in range(4))
+    n, c = shape[2], shape[3] ** -0.5
+    bias = torch.randn((*bias_bh, n, n), generator=g, device="cuda").to(DT[dt])
+    ins = [t.requires_grad_(True) for t in (q, k, v, bias)]
+    out = elsa_amd.twopass_attention_train(q, k, v, bias=bias, is_causal=causal)
+    grads = torch.autograd.grad(out, ins, do)
+    q64, k64, v64, do64 = (t.detach().double() for t in (q, k, v, do))
+    s = torch.matmul(q64, k64.transpose(-1, -2).contiguous()) * c + bias.detach().double()
+    if causal:
+        s = s.masked_fill(torch.ones((n, n), dtype=torch.bool, device="cuda").triu(1), float("-inf"))
+    p = torch.softmax(s, -1)
+    dsum = p * (do64 * torch.matmul(p, v64)).sum(-1, keepdim=True)
+    ds = p * torch.matmul(do64, v64.transpose(-1, -2).contiguous()) - dsum
+    dst, dsumt = ds.transpose(-1, -2).contiguous(), dsum.transpose(-1, -2).contiguous()
+    want = [torch.matmul(ds, k64) * c, torch.matmul(dst, q64) * c, torch.matmul(p.transpose(-1, -2).contiguous(), do64)]
+    other = [(torch.matmul(dsum, k64) * c).norm(), (torch.matmul(dsumt, q64) * c).norm(), 0.0]
+    for dim in (0, 1):
+        if bias_bh[dim] == 1:
+            ds, dsum = ds.sum(dim, keepdim=True), dsum.sum(dim, keepdim=True)
+    for name, got, ex, ot in zip(("dq", "dk", "dv", "dbias"), grads, [*want, ds], [*other, dsum.norm()]):
+        rel = ((got.double() - ex).norm() / (ex.norm() + ot)).item()
+        assert rel <= BOUND[dt], (name, rel)
