@@ -102,11 +102,14 @@ void bwd_dkdv_d128_kernel(const BwdParams p) {
 #pragma unroll
       for (int t = 0; t < 4; ++t) s[4 * q + t] = fast_exp2(fmaf(s[4 * q + t], p.scale_log2, -l4[t]));
     }
-    if (key0 + 31 >= p.N || (p.causal && t0 < key0 + 31)) {
+    // rows past N too: their LSE2 = +inf alone leaves a NaN where the key holds an infinity, times their zeros
+    if (key0 + 31 >= p.N || t0 + TT > p.N || (p.causal && t0 < key0 + 31)) {
       asm volatile("");  // keep this a branch: boundary tiles only
 #pragma unroll
-      for (int r = 0; r < 16; ++r)
-        if (!(key_ok && (!p.causal || t0 + key_of_reg(r, g) >= my_key))) s[r] = 0.f;
+      for (int r = 0; r < 16; ++r) {
+        const int row = t0 + key_of_reg(r, g);
+        if (!(key_ok && row < p.N && (!p.causal || row >= my_key))) s[r] = 0.f;
+      }
     }
     F w[2];
     L::pack(s, w);

@@ -312,12 +312,15 @@ void bwd_dkdv_x3_kernel(const BwdParams p) {
         s[r] = fast_exp2(x);
       }
     }
-    // keys past N and, in a causal call, keys past the row (rows past N have p = 0 already)
-    if (key0 + 31 >= p.N || (p.causal && t0 < key0 + 31)) {
+    // keys and rows past N (a row's LSE2 = +inf alone leaves a NaN where the key holds an infinity, times its zeros)
+    // and, in a causal call, keys past the row
+    if (key0 + 31 >= p.N || t0 + TT > p.N || (p.causal && t0 < key0 + 31)) {
       asm volatile("");  // keep this a branch: boundary tiles only
 #pragma unroll
-      for (int r = 0; r < 16; ++r)
-        if (!(key_ok && (!p.causal || t0 + key_of_reg(r, g) >= my_key))) s[r] = 0.f;
+      for (int r = 0; r < 16; ++r) {
+        const int row = t0 + key_of_reg(r, g);
+        if (!(key_ok && row < p.N && (!p.causal || row >= my_key))) s[r] = 0.f;
+      }
     }
     Split3 w[2];
     ln.pack(s, w);

@@ -208,7 +208,8 @@ void bwd_short_kernel(const BwdParams p, int groups) {
               float y = fmaf(s[4 * q + t], p.scale_log2, -l4[t]);
               if constexpr (sizeof(T) == 4) y -= lo4[t];
               if constexpr (HAS_BIAS) y = own_ok && row < N ? fmaf(bias_s[row * BS + key], kLog2e, y) : y;
-              s[4 * q + t] = own_ok && (!p.causal || row >= key) ? fast_exp2(y) : 0.f;
+              // (rows past N: LSE2 = +inf alone leaves a NaN where the key holds an infinity, times their zeros)
+              s[4 * q + t] = own_ok && row < N && (!p.causal || row >= key) ? fast_exp2(y) : 0.f;
             }
           }
           Own w[2];
