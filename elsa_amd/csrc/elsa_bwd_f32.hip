@@ -63,19 +63,21 @@ struct X3Loader {
     });
   }
   __device__ inline void store(bf16* ta, bf16* tb, int tid, int wave) const {
-    static_for<0, NCH>([&](auto I) {
-      constexpr int i = decltype(I)::value;
-      const bool second = wave * 64 + i * NT >= TCH;
-      const int cj = (tid + i * NT) % TCH;
-      float x[8];
+    split3_all<NCH>(
+        [&](auto I, float(&x)[8]) __attribute__((always_inline)) {
+          constexpr int i = decltype(I)::value;
 #pragma unroll
-      for (int t = 0; t < 8; ++t) x[t] = reg[i][t >> 2][t & 3];
-      const Split3 s3 = split3_any(x);
-      bf16* dst = (second ? tb : ta) + S::off(cj / S::CPR, (cj % S::CPR) * 8);
-      *reinterpret_cast<bf16x8*>(dst) = s3.h;
-      *reinterpret_cast<bf16x8*>(dst + S::PLANE) = s3.m;
-      *reinterpret_cast<bf16x8*>(dst + 2 * S::PLANE) = s3.l;
-    });
+          for (int t = 0; t < 8; ++t) x[t] = reg[i][t >> 2][t & 3];
+        },
+        [&](auto I, const Split3& s3) __attribute__((always_inline)) {
+          constexpr int i = decltype(I)::value;
+          const bool second = wave * 64 + i * NT >= TCH;
+          const int cj = (tid + i * NT) % TCH;
+          bf16* dst = (second ? tb : ta) + S::off(cj / S::CPR, (cj % S::CPR) * 8);
+          *reinterpret_cast<bf16x8*>(dst) = s3.h;
+          *reinterpret_cast<bf16x8*>(dst + S::PLANE) = s3.m;
+          *reinterpret_cast<bf16x8*>(dst + 2 * S::PLANE) = s3.l;
+        });
   }
 };
 

@@ -84,34 +84,43 @@ void bwd_short_kernel(const BwdParams p, int groups) {
           if (lane < N) bias_s[r * BS + lane] = load_bias(p.bias, bi, hi, r, lane);
       }
     }
+    // q, k, v and dO into their tiles
+    auto tile_at = [&](int w, int i) __attribute__((always_inline)) -> E* {
+      const int ci = tid + i * 256, row = ci / CPR, d0 = (ci % CPR) * 8;
+      return tiles[w][row >> 5] + (row & 31) * DP + (((d0 >> 3) ^ S::swz(row & 31)) << 3);
+    };
+    if constexpr (sizeof(T) == 4) {
+      split3_all<4 * NCH>(
+          [&](auto I, float(&y)[8]) __attribute__((always_inline)) {
+            constexpr int w = decltype(I)::value / NCH, i = decltype(I)::value % NCH;
+#pragma unroll
+            for (int t = 0; t < 8; ++t) y[t] = __uint_as_float(x[w][i][t >> 2][t & 3]);
+          },
+          [&](auto I, const Split3& s3) __attribute__((always_inline)) {
+            E* dst = tile_at(decltype(I)::value / NCH, decltype(I)::value % NCH);
+            *reinterpret_cast<bf16x8*>(dst) = s3.h;
+            *reinterpret_cast<bf16x8*>(dst + S::PLANE) = s3.m;
+            *reinterpret_cast<bf16x8*>(dst + 2 * S::PLANE) = s3.l;
+          });
+    } else {
+#pragma unroll
+      for (int i = 0; i < NCH; ++i)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) *reinterpret_cast<Chunk16*>(tile_at(w, i)) = x[w][i][0];
+    }
+    // D of a row: O * dO over its CPR lanes
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
-      const int ci = tid + i * 256, row = ci / CPR, d0 = (ci % CPR) * 8;
-      const int lo = (row & 31) * DP + (((d0 >> 3) ^ S::swz(row & 31)) << 3);
+      const int ci = tid + i * 256, row = ci / CPR;
       float acc = 0.f;
+      if constexpr (sizeof(T) == 4) {
 #pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        E* dst = tiles[w][row >> 5] + lo;
-        if constexpr (sizeof(T) == 4) {
-          float y[8];
+        for (int t = 0; t < 8; ++t)
+          acc = fmaf(__uint_as_float(x[4][i][t >> 2][t & 3]), __uint_as_float(x[3][i][t >> 2][t & 3]), acc);
+      } else {
+        const F8 go = __builtin_bit_cast(F8, x[3][i][0]), oo = __builtin_bit_cast(F8, x[4][i][0]);
 #pragma unroll
-          for (int t = 0; t < 8; ++t) y[t] = __uint_as_float(x[w][i][t >> 2][t & 3]);
-          const Split3 s3 = split3_any(y);
-          *reinterpret_cast<bf16x8*>(dst) = s3.h;
-          *reinterpret_cast<bf16x8*>(dst + S::PLANE) = s3.m;
-          *reinterpret_cast<bf16x8*>(dst + 2 * S::PLANE) = s3.l;
-          if (w == 3) {
-#pragma unroll
-            for (int t = 0; t < 8; ++t) acc = fmaf(__uint_as_float(x[4][i][t >> 2][t & 3]), y[t], acc);
-          }
-        } else {
-          *reinterpret_cast<Chunk16*>(dst) = x[w][i][0];
-          if (w == 3) {
-            const F8 go = __builtin_bit_cast(F8, x[3][i][0]), oo = __builtin_bit_cast(F8, x[4][i][0]);
-#pragma unroll
-            for (int t = 0; t < 8; ++t) acc = fmaf(static_cast<float>(oo[t]), static_cast<float>(go[t]), acc);
-          }
-        }
+        for (int t = 0; t < 8; ++t) acc = fmaf(static_cast<float>(oo[t]), static_cast<float>(go[t]), acc);
       }
 #pragma unroll
       for (int w = 1; w < CPR; w <<= 1) acc += __shfl_xor(acc, w);

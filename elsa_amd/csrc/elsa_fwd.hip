@@ -411,21 +411,23 @@ void phase1_x3_kernel(const Phase1Params p) {
     });
   };
   auto sstore = [&](int buf) {
-    static_for<0, NCH>([&](auto I) {
-      constexpr int i = decltype(I)::value;
-      const int ci = tid + i * NT;
-      const bool is_v = wave * 64 + i * NT >= TCH;
-      const int cj = ci % TCH, key = cj / CPR, d0 = (cj % CPR) * 8;
-      float x[8];
+    split3_all<NCH>(
+        [&](auto I, float(&x)[8]) __attribute__((always_inline)) {
+          constexpr int i = decltype(I)::value;
 #pragma unroll
-      for (int t = 0; t < 8; ++t) x[t] = __uint_as_float(reg[i][t >> 2][t & 3]);
-      const Split3 s3 = split3_any(x);
-      bf16(*dst)[KT * KS] = is_v ? Vp[buf] : Kp[buf];
-      const int o = Tile::off(key, d0);
-      *reinterpret_cast<bf16x8*>(&dst[0][o]) = s3.h;
-      *reinterpret_cast<bf16x8*>(&dst[1][o]) = s3.m;
-      *reinterpret_cast<bf16x8*>(&dst[2][o]) = s3.l;
-    });
+          for (int t = 0; t < 8; ++t) x[t] = __uint_as_float(reg[i][t >> 2][t & 3]);
+        },
+        [&](auto I, const Split3& s3) __attribute__((always_inline)) {
+          constexpr int i = decltype(I)::value;
+          const int ci = tid + i * NT;
+          const bool is_v = wave * 64 + i * NT >= TCH;
+          const int cj = ci % TCH, key = cj / CPR, d0 = (cj % CPR) * 8;
+          bf16(*dst)[KT * KS] = is_v ? Vp[buf] : Kp[buf];
+          const int o = Tile::off(key, d0);
+          *reinterpret_cast<bf16x8*>(&dst[0][o]) = s3.h;
+          *reinterpret_cast<bf16x8*>(&dst[1][o]) = s3.m;
+          *reinterpret_cast<bf16x8*>(&dst[2][o]) = s3.l;
+        });
   };
   gload(k_begin);
 

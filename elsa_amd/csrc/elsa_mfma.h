@@ -81,6 +81,18 @@ __device__ __host__ constexpr inline int key_of_reg(int r, int g) { return 16 * 
 
 __device__ inline float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
+// Compile-time loop: f(std::integral_constant<int, I>) for I = B .. E-1.  Register
+// staging arrays indexed through it see constant indices from the start, so they are
+// split into VGPRs; indexed by a `#pragma unroll` loop variable they can instead be
+// placed in LDS or scratch before the loop is unrolled.
+template <int B, int E, typename Fn>
+__device__ inline void static_for(Fn&& f) {
+  if constexpr (B < E) {
+    f(std::integral_constant<int, B>{});
+    static_for<B + 1, E>(f);
+  }
+}
+
 // fp32 operands on the bf16 matrix cores: x = h + m + l with h, m and l bf16 (8 + 8 + 8 significant
 // bits), and a product of two such sums as the six partial products of order 2^-16 and above,
 //   x y ~ h h' + (h m' + m h') + (m m' + h l' + l h'),
@@ -112,18 +124,19 @@ __device__ inline Split3 split3_reg(const float (&x)[8]) {
   o.l = to_bf16x8(r);
   return o;
 }
-// any input: h truncated, so that no finite value becomes infinite.  An infinity or NaN goes to l, which
-// meets only the other operand's h (of its sign, 0 only for 0): as h it also met m and l, of either sign
-// or 0, and a product with infinity came out NaN.  h and m are then those of the largest finite value, whose
-// products with the other operand's l stay finite for values up to 2^16.  (Selects on a finite test
-// instead: forward B1 H8 8K 0.680 -> 0.692 ms, training step 4K 0.761 -> 0.766.)
+// any input: h truncated, so that no finite value becomes infinite.  An infinity goes to l beside h = +-1 and m = 0,
+// so that it meets only the other operand's h (of its sign, 0 below 2^-133): as h it met m and l too, of either
+// sign or 0, and a product with infinity came out NaN.  A NaN stays one in every part it reaches.  INF false: for
+// values without an infinity (the test costs two instructions a value).
+template <bool INF = true>
 __device__ inline Split3 split3_any(const float (&x)[8]) {
 #pragma clang fp contract(off)
   Split3 o;
   float r[8], h[8];
 #pragma unroll
   for (int t = 0; t < 8; ++t) {
-    const float f = __builtin_amdgcn_fmed3f(x[t], -__FLT_MAX__, __FLT_MAX__);
+    float f = x[t];
+    if constexpr (INF) f = __builtin_amdgcn_classf(f, 0x204) ? __builtin_copysignf(1.f, f) : f;
     h[t] = __uint_as_float(__float_as_uint(f) & 0xffff0000u);
     r[t] = f - h[t];
   }
@@ -133,6 +146,31 @@ __device__ inline Split3 split3_any(const float (&x)[8]) {
   for (int t = 0; t < 8; ++t) r[t] = (x[t] - h[t]) - static_cast<float>(o.m[t]);
   o.l = to_bf16x8(r);
   return o;
+}
+// put(i, split of get(i)) for i < N: one test for infinities over a wave's N groups of 8 values (half an instruction a
+// value), and split3_any's own only in a wave that holds one
+template <int N, typename Get, typename Put>
+__device__ inline void split3_all(Get&& get, Put&& put) {
+  float mx = 0.f;
+  static_for<0, N>([&](auto I) __attribute__((always_inline)) {
+    float x[8];
+    get(I, x);
+#pragma unroll
+    for (int t = 0; t < 8; t += 2) mx = fmaxf(fmaxf(mx, fabsf(x[t])), fabsf(x[t + 1]));
+  });
+  if (__any(mx == __builtin_huge_valf())) {
+    static_for<0, N>([&](auto I) __attribute__((always_inline)) {
+      float x[8];
+      get(I, x);
+      put(I, split3_any<true>(x));
+    });
+  } else {
+    static_for<0, N>([&](auto I) __attribute__((always_inline)) {
+      float x[8];
+      get(I, x);
+      put(I, split3_any<false>(x));
+    });
+  }
 }
 // acc + a b without the leading product: the five smaller partial products, least first
 __device__ inline f32x16 mma3_small(const bf16x8& ah, const bf16x8& am, const bf16x8& al, const Split3& b, f32x16 acc) {
@@ -165,18 +203,6 @@ __device__ inline typename Mfma<T>::frag pack_frag(const f32x16& v) {
 #pragma unroll
     for (int t = 0; t < 8; ++t) f[t] = static_cast<T>(v[R0 + t]);
     return f;
-  }
-}
-
-// Compile-time loop: f(std::integral_constant<int, I>) for I = B .. E-1.  Register
-// staging arrays indexed through it see constant indices from the start, so they are
-// split into VGPRs; indexed by a `#pragma unroll` loop variable they can instead be
-// placed in LDS or scratch before the loop is unrolled.
-template <int B, int E, typename Fn>
-__device__ inline void static_for(Fn&& f) {
-  if constexpr (B < E) {
-    f(std::integral_constant<int, B>{});
-    static_for<B + 1, E>(f);
   }
 }
 

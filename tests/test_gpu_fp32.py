@@ -112,6 +112,31 @@ def test_fp32_key_at_minus_infinity_drops_out():
         assert rel <= BOUND, (n, rel)
 
 
+def test_fp32_infinity_beside_a_large_partner():
+    # a product of an infinity and a value past 2^16, whose parts are large too: still the infinity
+    for n, d in ((40, 64), (64, 64), (49, 32), (300, 64), (300, 128), (600, 32)):
+        q, k, v, do = _inputs((1, 2, n, d), n)
+        q[..., 3] = (q[..., 3].abs() + 1) * 2.0 ** 18
+        k[..., 3] = k[..., 3] * 2.0 ** -18
+        k[:, :, 9, 3] = float("-inf")
+        out = elsa_amd.twopass_attention(q, k, v)
+        rest = [i for i in range(n) if i != 9]
+        ks, vs = k[:, :, rest].double(), v[:, :, rest].double()
+        want = torch.softmax(q.double() @ ks.transpose(-1, -2).contiguous() * d ** -0.5, -1) @ vs
+        assert ((out.double() - want).norm() / want.norm()).item() <= BOUND, (n, d)
+        # the gradient of v: a row of dO that is infinite in one column
+        ins = [t.detach().requires_grad_(True) for t in (q, k, v)]
+        o = elsa_amd.twopass_attention_train(*ins)
+        do = do.clone()
+        do[:, :, 5, 1] = float("inf")
+        dv = torch.autograd.grad(o, ins[2], do)[0]
+        cols = [c for c in range(d) if c != 1]
+        p = torch.softmax(q.double() @ k.double().nan_to_num(neginf=-1e300).transpose(-1, -2).contiguous() * d ** -0.5, -1)
+        want = p.transpose(-1, -2).contiguous() @ do.double()[..., cols]
+        assert ((dv[..., cols].double() - want).norm() / want.norm()).item() <= BOUND, (n, d)
+        assert (dv[:, :, rest, 1] == float("inf")).all() and not dv[:, :, 9, 1].isfinite().any()
+
+
 def test_fp32_strided_operands_match_dense_ones():
     qkv = torch.randn((2, 197, 3, 3, 64), device="cuda", generator=torch.Generator(device="cuda").manual_seed(9))
     do = torch.randn((2, 3, 197, 64), device="cuda", generator=torch.Generator(device="cuda").manual_seed(10))

@@ -17,8 +17,7 @@ def _bf16_trunc(x):
 
 
 def _split(x, truncate_h):
-    big = np.finfo(np.float32).max
-    f = np.fmin(np.fmax(x, -big), big).astype(np.float32)
+    f = np.where(np.isinf(x), np.sign(x), x).astype(np.float32)  # an infinity goes to the last part, beside +-1
     h = _bf16_trunc(f) if truncate_h else _bf16_rne(f)
     m = _bf16_rne(f - h)
     r = (x - h) - m
@@ -53,6 +52,17 @@ def test_products_with_an_infinity_are_the_fp32_ones():
             with np.errstate(over="ignore"):
                 got = al * bh + ah * bl + am * bm + am * bh + ah * bm + ah * bh
             assert np.array_equal(got, np.float32(a) * y)
+
+
+def test_products_with_an_infinity_hold_for_every_partner():
+    rng = np.random.default_rng(8)
+    y = (rng.standard_normal(4000) * 2.0 ** rng.integers(-120, 127, 4000)).astype(np.float32)
+    y = np.concatenate([y, np.array([np.inf, -np.inf, np.finfo(np.float32).max], np.float32)])
+    bh, bm, bl = _split(y, True)
+    for a in (np.inf, -np.inf):
+        ah, am, al = _split(np.full(len(y), a, np.float32), True)
+        got = al * bh + ah * bl + am * bm + am * bh + ah * bm + ah * bh
+        assert np.array_equal(got, np.float32(a) * y)
 
 
 @pytest.mark.parametrize("truncate_a,truncate_b", [(True, True), (True, False), (False, False)])
