@@ -112,6 +112,18 @@ def test_fp32_key_at_minus_infinity_drops_out():
         assert rel <= BOUND, (n, rel)
 
 
+@pytest.mark.parametrize("n,d", [(49, 64), (64, 32), (100, 64), (100, 32), (128, 128)])
+def test_fp32_values_near_the_largest_do_not_overflow(n, d):
+    # a key a little above the maximum of the stages before it must not scale the sums past the fp32 range (64 keys
+    # of equal weight, the most in a partition here, stay inside it)
+    q = torch.zeros((1, 1, n, d), device="cuda")
+    k, v = torch.zeros_like(q), torch.full_like(q, 3.0e36)
+    q[..., 0] = d ** 0.5
+    k[0, 0, n - 3, 0] = 5.0
+    out = elsa_amd.twopass_attention(q, k, v)
+    assert ((out.double() / 3.0e36 - 1).abs() <= 1e-6).all()
+
+
 def test_fp32_infinity_beside_a_large_partner():
     # a product of an infinity and a value past 2^16, whose parts are large too: still the infinity
     for n, d in ((40, 64), (64, 64), (49, 32), (300, 64), (300, 128), (600, 32)):
