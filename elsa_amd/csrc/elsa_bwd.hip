@@ -1183,11 +1183,11 @@ hipError_t launch_zero_fill(float* dst, int64_t n, hipStream_t st) {
 }
 
 // ------------------------------------------------------------------ split backward
-// Work-groups of a causal backward split into s ranges that hold work: a 128-row block's dq covers
-// the keys below k_end = min(n, 128 * (block + 1)), so its ranges from ceil(k_end / split_len) on
-// return at once (the dK/dV grid mirrors this count).
+// Line of the causal fp32 split at D <= 64 (bwd_splits): 128-row blocks times the contiguous ranges of whole 32-key
+// stages that their keys would reach.  The kernels deal the stages out in turn, so that every range of a block
+// holds its share; the count only says how far a grid is worth splitting.
 static int64_t causal_live_wgs(int64_t bh, int64_t n, int s) {
-  const int64_t len = ((n + s - 1) / s + 31) / 32 * 32;  // the fp32 split_len: whole 32-key stages
+  const int64_t len = ((n + s - 1) / s + 31) / 32 * 32;
   int64_t live = 0;
   for (int64_t b0 = 0; b0 < n; b0 += 128) live += (std::min(n, b0 + 128) + len - 1) / len;
   return bh * live;
@@ -1203,8 +1203,8 @@ static int64_t causal_live_wgs(int64_t bh, int64_t n, int s) {
 // Whole backward ms, d64: B2 H8 N4097 (528 work-groups for 512 slots) 1.90 -> 1.45 (1 -> 5 ranges); head
 // dim 128 (one 4-wave work-group per CU): B1 H8 2K 0.670 -> 0.377 (1 -> 2), B4 H2 N300 0.120 -> 0.056 (1 -> 4),
 // B1 H8 4K stays.
+constexpr int64_t kPartialBytes = int64_t(512) << 20;
 static int f32_ragged_splits(int dp, int64_t bh, int64_t n) {
-  constexpr int64_t kPartialBytes = int64_t(512) << 20;
   const int64_t w4 = bh * ((n + 127) / 128), w8 = bh * ((n + 255) / 256);
   auto cost = [&](int s) {
     const double k4 = (double)((w4 * s + 255) / 256), k8 = (double)((w8 * s + 255) / 256);
@@ -1212,6 +1212,23 @@ static int f32_ragged_splits(int dp, int64_t bh, int64_t n) {
     const double rounds = dp > 64 ? 2.33 * k4 : std::min(0.94 * k8, dq4) + 1.33 * std::min(k8, 0.645 * k4);
     const double len = (double)(((n + s - 1) / s + 31) / 32 * 32);
     return rounds * (len + 65) + (s > 1 ? 180 + 0.0032 * (double)(w4 * dp) * s : 0.0);
+  };
+  int best = 1;
+  for (int s = 2; s <= 8 && n / s >= 64 && 3 * s * bh * n * dp * 4 <= kPartialBytes; ++s)
+    if (cost(s) < cost(best)) best = s;
+  return cost(best) < 0.985 * cost(1) ? best : 1;
+}
+
+// Causal fp32 calls at D = 128 (one 4-wave work-group per CU, heaviest first): the ranges 1..8 by the larger of
+// the work of all of them over 256 CUs and the longest one, in stage rows (65 a work-group), plus the combine's
+// traffic; limits as above.  Whole backward ms by ranges 1 / 2 / 4 / 8: H8 2K 0.653 / 0.363 / 0.249 / 0.330, H24 N1025
+// 0.348 / 0.242 / 0.298 / 0.441, H16 N2049 0.664 / 0.472 / 0.560 / 0.737, H1 8K 2.53 / 1.29 / 0.676 / 0.431, H16 N4097
+// 1.48 / 1.56 / 1.74 / 2.07; the non-causal rule took 2, 1, 3, 5 and 5.
+static int f32_causal_wide_splits(int dp, int64_t bh, int64_t n) {
+  const double w4 = (double)(bh * ((n + 127) / 128));
+  auto cost = [&](int s) {
+    return std::max(w4 * ((double)n / 2 + 64 + 65 * s) / 256, (double)n / s + 65) +
+           (s > 1 ? 60 + 0.0016 * w4 * dp * s : 0.0);
   };
   int best = 1;
   for (int s = 2; s <= 8 && n / s >= 64 && 3 * s * bh * n * dp * 4 <= kPartialBytes; ++s)
@@ -1241,7 +1258,7 @@ static int half_ragged_splits(int64_t bh, int64_t n) {
 
 int bwd_splits(int dtype, int dp, int64_t bh, int64_t n, bool bias, bool causal) {
   if (bias || (dp > 64 && dtype != ELSA_F32)) return 1;
-  if (dp > 64) return f32_ragged_splits(dp, bh, n);
+  if (dp > 64) return causal ? f32_causal_wide_splits(dp, bh, n) : f32_ragged_splits(dp, bh, n);
   const int64_t wgs = bh * ((n + 127) / 128);  // the unsplit 4-wave grid
   // double while the doubled grid stays within one round of 512 work-groups (two per CU): whole
   // backward, fp16 d64, against doubling while the grid was short of 512: B8 H3 N1025 0.083 ->
@@ -1250,12 +1267,11 @@ int bwd_splits(int dtype, int dp, int64_t bh, int64_t n, bool bias, bool causal)
   // Ranges stay at least 256 keys or rows for fp16 and bf16 (128: B1 H8 N1024 0.038 -> 0.044 ms)
   // and 64 for fp32, whose stages take several times longer (against 256: B8 H3 N197 0.089 ->
   // 0.064 ms, B1 H8 N512 0.103 -> 0.061, B2 H3 N300 0.118 -> 0.064; 128 gave 0.089, 0.069, 0.082)
-  // Causal fp32 calls count only the work-groups that hold work (the others return at once): the
-  // doubling splits the longest rows' key ranges, and an fp32 stage is long enough that those set
-  // the time.  Against the count of every work-group: B1 H8 N1025 0.202 -> 0.162 ms (4 -> 8 ranges),
-  // B2 H8 N2049 0.895 -> 0.571 (1 -> 2), B1 H8 N4097 1.305 -> 1.098, N5000 1.773 -> 1.333, N3000
-  // 0.800 -> 0.723 (2 -> 4).  fp16 went both ways (B2 H8 N2049 0.103 -> 0.085 ms, but B1 H12 N2048
-  // 0.076 -> 0.083 and B1 H8 N5000 0.169 -> 0.177), so 16-bit calls count every work-group.
+  // Causal fp32 calls go further, until causal_live_wgs passes 512: their longest rows set the time.  Whole backward
+  // ms by ranges 1 / 2 / 4 / 8, the taken one marked: d64 H8 N1025 0.184 / 0.109 / 0.073 / 0.071*, H8 N3000 0.500 / 0.277
+  // / 0.231* / 0.258, H16 N2049 0.354 / 0.249* / 0.231 / 0.286, H8 N4097 0.683 / 0.456* / 0.373 / 0.420, H16 N4097 0.849* /
+  // 0.673 / 0.724 / 0.853, H100 N300 0.073 / 0.092* / 0.129 / 0.210.  16-bit calls count every work-group (fp16 B2 H8
+  // N2049 0.103 -> 0.085 ms split further, but B1 H12 N2048 0.076 -> 0.083 and B1 H8 N5000 0.169 -> 0.177).
   if (dtype == ELSA_F32 && !causal && dp == 64 && wgs > 256) return f32_ragged_splits(dp, bh, n);
   if (dtype != ELSA_F32 && !causal && dp == 64 && wgs > 256 && wgs <= 1024) return half_ragged_splits(bh, n);
   const int64_t min_range = dtype == ELSA_F32 ? 64 : 256;

@@ -128,11 +128,11 @@ struct BwdParams {
   int64_t part_stride;  // floats from the dq partials to the dK ones and from those to the dV ones
 };
 
-// Ranges the backward (fp16, bf16 and fp32) cuts its loops into when its unsplit grid (128 rows or
-// keys per work-group) leaves the chip under-filled: doubled from 1 while the doubled grid stays
-// within 512 work-groups (causal fp32: 512 that hold work) and n / (2 * split) is at least 256 (64
-// for fp32); ragged fp32 and 16-bit d64 grids without a causal mask, and fp32 at D = 128, by the rounds
-// they take.  Biased calls and 16-bit head dims above 64 keep 1.
+// Ranges the backward cuts its loops into when its unsplit grid (128 rows or keys per work-group) leaves the
+// chip under-filled.  Doubled from 1 while the doubled grid stays within 512 work-groups and n / (2 * split) is at
+// least 256 (64 for fp32); causal fp32 goes further (causal_live_wgs).  By the rounds they take: ragged fp32 and
+// 16-bit d64 grids without a causal mask, and fp32 at D = 128.  16-bit calls with a bias or a head dim above 64
+// keep 1, as do biased fp32 ones.
 int bwd_splits(int dtype, int dp, int64_t bh, int64_t n, bool bias, bool causal);
 // fp32 partials of each gradient that such a split writes (1: none): its ranges, or half of them where
 // work-groups of two wave groups take them two at a time.

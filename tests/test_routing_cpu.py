@@ -114,3 +114,18 @@ def test_wide_head_forwards_keep_one_work_group_per_cu_or_partitions_of_512_keys
                 plan = _plan(_fwd_args(_lib.ELSA_BF16, 1, h, n, d))
                 wgs = h * -(-n // plan.block_m) * plan.partitions
                 assert plan.partitions == 1 or plan.partition_len >= 512 or (wgs <= 256 and plan.partition_len >= 128)
+
+
+# causal fp32 backwards above head dim 64, ranges by their own cost (ms with the count before and after)
+@pytest.mark.parametrize("h,n,split", [
+    (8, 2048, 4),    # 0.363 with 2, 0.249
+    (24, 1025, 2),   # 0.348 with 1, 0.242
+    (16, 2049, 2),   # 0.600 with 3, 0.472
+    (16, 1024, 3),   # 0.205 with 2
+    (4, 3000, 5),
+    (1, 8192, 8),    # 0.672 with 5, 0.431
+    (16, 4097, 1),   # 1.816 with 5, 1.484
+    (100, 300, 1), (32, 2048, 1)])
+def test_causal_fp32_ranges_above_head_dim_64(h, n, split):
+    need, rows = _bwd_workspace(_lib.ELSA_F32, 1, h, n, 128, causal=True)
+    assert need == rows + (3 * -(-split * h * n * 128 * 4 // 256) * 256 if split > 1 else 0)
