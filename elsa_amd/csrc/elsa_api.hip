@@ -735,7 +735,7 @@ int elsa_bwd_dbias(const elsa_bwd_args* a, float* dbias, int32_t bias_batch, int
   float* ds = direct ? dbias
                      : reinterpret_cast<float*>(static_cast<char*>(a->workspace) + elsa_bwd_workspace_bytes(a));
   hipError_t e = hipSuccess;
-  const bool is_short = elsa::bwd_short_takes(a->dtype, a->seq_len, elsa::pad_head_dim(a->head_dim));
+  const bool is_short = elsa::bwd_short_takes(a->seq_len, elsa::pad_head_dim(a->head_dim));
   if (is_short && !direct && bias_batch == 1 && bias_heads == a->heads) {
     // dS summed over the batch inside the backward, one partial per range of it (at most batch: they fit the
     // dS buffer), then over the ranges

@@ -31,7 +31,6 @@ struct BwdCfg {
   static constexpr int RS = DP + KPAD;  // row-major tile stride [TT][RS]
   static constexpr int TS = TT + VPAD;  // transposed tile stride [DP][TS]
   static constexpr int NDT = DP / 32;
-  static constexpr int NJ = 16 / KP;
   static constexpr int CE = 16 / (int)sizeof(T);
 };
 
@@ -1356,27 +1355,23 @@ static hipError_t pre_launch(const BwdParams& p, hipStream_t st) {
 // fp16/bf16 kernels: 32 rows (dq) or 32 keys (dk/dv) per wave, 4 waves per
 // workgroup, register budget capped for 2 waves per SIMD (measured on MI355X at
 // B1 H8 N16K d64: dq 1.36 ms / dk-dv 1.68 ms versus 2.27 / 2.76 ms with 64-wide
-// wave tiles at 1 wave per SIMD).  fp32 keeps the 32-wide kernels above.
-// Single stages (elsa_bwd_stage; the whole backward is bwd_short_kernel) of
-// sequences of at most 64 rows at head dims up to 32 (Swin's 49-token windows): 2-wave
+// wave tiles at 1 wave per SIMD).
+// The dq and dk/dv stages alone (elsa_bwd_stage 1 and 2; a whole backward of these calls is bwd_short_kernel, so the
+// stages' times are not its parts) of sequences of at most 64 rows at head dims up to 32: 2-wave
 // work-groups of 64 rows or keys, so that no wave of a work-group lies wholly past N (with 4
 // waves of 32, waves 2 and 3 only staged and waited).  The split backward never applies there
-// (bwd_splits).  Wider heads keep 4 waves: at D = 64 the 2-wave fp16/bf16 dK/dV kernel spills
-// (its staging share per thread doubles) and the fp32 one drops to 1 wave per SIMD.
+// (bwd_splits).  Wider heads keep 4 waves: at D = 64 the 2-wave dK/dV kernel spills (its staging share per
+// thread doubles).
 template <typename T, int DP, bool B>
 static hipError_t bwd_launch_short(const BwdParams& p, int stage, hipStream_t st) {
   constexpr int W = 2;
   const dim3 grid((p.N + 32 * W - 1) / (32 * W), p.BH);
-  hipError_t e = hipSuccess;
-  if (stage < 0 || stage == 1) {
+  if (stage == 1) {
     hipLaunchKernelGGL((bwd_dq_half_kernel<T, DP, 1, W, B>), grid, dim3(64 * W), 0, st, p);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-  }
-  if (stage < 0 || stage == 2) {
+  } else {
     hipLaunchKernelGGL((bwd_dkdv_half_kernel<T, DP, 1, W, B>), grid, dim3(64 * W), 0, st, p);
-    e = hipGetLastError();
   }
-  return e;
+  return hipGetLastError();
 }
 
 template <typename T, int DP, bool B>
@@ -1576,7 +1571,7 @@ static hipError_t bwd_launch1(const BwdParams& p, int stage, hipStream_t st) {
 }
 
 hipError_t launch_bwd(const BwdParams& p, int dtype, int stage, hipStream_t st) {
-  if (stage < 0 && bwd_short_takes(dtype, p.N, p.dp)) return launch_bwd_short(p, dtype, p.ds_out ? 1 : 0, st);
+  if (stage < 0 && bwd_short_takes(p.N, p.dp)) return launch_bwd_short(p, dtype, p.ds_out ? 1 : 0, st);
   if (dtype == ELSA_F16) return bwd_launch1<f16>(p, stage, st);
   if (dtype == ELSA_BF16) return bwd_launch1<bf16>(p, stage, st);
   return stage == 0 ? pre_launch<float>(p, st) : launch_bwd_f32(p, stage, st);

@@ -265,7 +265,7 @@ void bwd_short_kernel(const BwdParams p, int groups) {
 }
 
 // Head dims above 64 do not fit (fp32 tiles of 64 rows at D = 128: 196 KB of LDS).
-bool bwd_short_takes(int dtype, int n, int dp) { return n <= kShortRows && dp <= 64; }
+bool bwd_short_takes(int n, int dp) { return n <= kShortRows && dp <= 64; }
 
 // Groups of windows (ds_mode 2): one round of the work-groups that run at once (by registers and LDS 3, 2,
 // 2 and 1 per CU), and no group takes more than one window more than another.

@@ -32,26 +32,16 @@ namespace elsa {
 
 int pad_head_dim(int d) { return d <= 32 ? 32 : (d <= 64 ? 64 : 128); }
 
-template <typename T, int DP>
+// Stage of the fp32 MFMA fold (phase1_kernel): 32 keys, two buffers.  K rows stay 16-byte aligned for 4-float loads;
+// V^T keeps stride KT + 1, where its transposing scalar writes are conflict-free (16-byte reads at stride KT + 4 cost
+// more in those writes than they saved: 16K Phase 1 4.68 against 4.52 ms).
+template <int DP>
 struct FwdCfg {
-  static constexpr int KP = Mfma<T>::KP;
-  static constexpr int KSTEP = 2 * KP;  // contraction length of one MFMA
-  static constexpr int NKK = DP / KSTEP;
-  static constexpr bool HALF = sizeof(T) == 2;
-  static constexpr int KT = ((HALF && DP == 128) || (!HALF && DP >= 64)) ? 32 : 64;  // keys per LDS stage
-  static constexpr int NSUB = KT / 32;
-  static constexpr int KPAD = HALF ? 8 : 4;  // fp32: K rows stay 16-byte aligned for 4-float loads
-  // fp32 V^T keeps stride KT + 1: its transposing scalar writes are conflict-free there, and
-  // 16-byte reads at stride KT + 4 cost more in those writes than they saved (16K Phase 1
-  // 4.68 against 4.52 ms)
-  static constexpr int VPAD = HALF ? 8 : 1;
-  static constexpr int KS = DP + KPAD;  // LDS row stride of K   [KT][KS]
-  static constexpr int VS = KT + VPAD;  // LDS row stride of V^T [DP][VS]
-  static constexpr int LDS_ONE = (KT * KS + DP * VS) * (int)sizeof(T);
-  static constexpr int NBUF = (2 * LDS_ONE <= 98304) ? 2 : 1;
+  static constexpr int KT = 32;
+  static constexpr int KS = DP + 4;    // LDS row stride of K   [KT][KS]
+  static constexpr int VS = KT + 1;    // LDS row stride of V^T [DP][VS]
   static constexpr int NDT = DP / 32;  // 32-wide head-dim tiles of O^T
-  static constexpr int NJ = 16 / KP;   // P^T.V^T MFMAs per 32-key sub-tile
-  static constexpr int CE = 16 / (int)sizeof(T);
+  static constexpr int CE = 4;         // elements of a 16-byte chunk
 };
 
 int phase1_key_tile(int dtype, int dp) {
@@ -113,10 +103,11 @@ __device__ inline void emit4(const Phase1Params& p, int64_t ridx, int64_t ooff, 
   *reinterpret_cast<t4*>(static_cast<T*>(p.out) + ooff + d) = o;
 }
 
-template <typename T, int DP, int WAVES, bool HAS_BIAS>
+// fp32 fold of 64-row blocks at D > 64 (others: phase1_x3_kernel)
+template <int DP, int WAVES, bool HAS_BIAS>
 __global__ __launch_bounds__(64 * WAVES) void phase1_kernel(const Phase1Params p) {
-  static_assert(sizeof(T) == 4, "fp32 fold of 64-row blocks at D > 64 (others: phase1_x3_kernel)");
-  using C = FwdCfg<T, DP>;
+  typedef float T;
+  using C = FwdCfg<DP>;
   using M = Mfma<T>;
   // The fp32 MFMA takes one operand element per lane and k-step, and the contraction order
   // over d is free: k-step kk = 4m + u of lane group g takes d = 8m + 4g + u, so one 16-byte
@@ -129,8 +120,8 @@ __global__ __launch_bounds__(64 * WAVES) void phase1_kernel(const Phase1Params p
   static_assert((C::KT * CPR) % NT == 0, "staging must divide evenly");
   constexpr int NCH = C::KT * CPR / NT;
 
-  __shared__ __attribute__((aligned(16))) T Ks[C::NBUF][C::KT * C::KS];
-  __shared__ __attribute__((aligned(16))) T Vt[C::NBUF][DP * C::VS];
+  __shared__ __attribute__((aligned(16))) T Ks[2][C::KT * C::KS];
+  __shared__ __attribute__((aligned(16))) T Vt[2][DP * C::VS];
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 31, g = lane >> 5;
@@ -202,55 +193,43 @@ __global__ __launch_bounds__(64 * WAVES) void phase1_kernel(const Phase1Params p
   __syncthreads();
 
   for (int it = 0; it < ntiles; ++it) {
-    const int buf = (C::NBUF == 2) ? (it & 1) : 0;
+    const int buf = it & 1;
     const int t0 = k_begin + it * C::KT;
     const bool has_next = it + 1 < ntiles;
-    if (C::NBUF == 2 && has_next) gload(t0 + C::KT);
+    if (has_next) gload(t0 + C::KT);
     const T* ks = Ks[buf];
     const T* vt = Vt[buf];
 
-    // S^T = K Q^T : lane (c, g) register r <-> key t0 + 32*sub + key_of_reg(r, g), row c.
-    f32x16 s[C::NSUB];
+    // S^T = K Q^T : lane (c, g) register r <-> key t0 + key_of_reg(r, g), row c.
+    f32x16 s = f32x16{};
+    const T* krow = ks + swap23(c) * C::KS + 4 * g;
 #pragma unroll
-    for (int sub = 0; sub < C::NSUB; ++sub) {
-      s[sub] = f32x16{};
-      const T* krow = ks + (sub * 32 + swap23(c)) * C::KS + 4 * g;
+    for (int m = 0; m < NM; ++m) {
+      const f32x4 ka = *reinterpret_cast<const f32x4*>(krow + 8 * m);
 #pragma unroll
-      for (int m = 0; m < NM; ++m) {
-        const f32x4 ka = *reinterpret_cast<const f32x4*>(krow + 8 * m);
-#pragma unroll
-        for (int u = 0; u < 4; ++u) s[sub] = M::mma(ka[u], qf[m][u], s[sub]);
-      }
+      for (int u = 0; u < 4; ++u) s = M::mma(ka[u], qf[m][u], s);
     }
 
     float mx = kNegInf;
     if constexpr (HAS_BIAS) {
 #pragma unroll
-      for (int sub = 0; sub < C::NSUB; ++sub)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int key = t0 + sub * 32 + key_of_reg(r, g);
-          const bool ok = row_ok && key < k_end && (!p.causal || key <= my_row);
-          const float x = ok ? fmaf(s[sub][r], cs, load_bias(p.bias, bi, hi, my_row, key) * p.bias_log2) : kNegInf;
-          s[sub][r] = x;
-          mx = fmaxf(mx, x);
-        }
+      for (int r = 0; r < 16; ++r) {
+        const int key = t0 + key_of_reg(r, g);
+        const bool ok = row_ok && key < k_end && (!p.causal || key <= my_row);
+        s[r] = ok ? fmaf(s[r], cs, load_bias(p.bias, bi, hi, my_row, key) * p.bias_log2) : kNegInf;
+        mx = fmaxf(mx, s[r]);
+      }
     } else {
       const bool need_mask = (t0 + C::KT > k_end) || (p.causal && (t0 + C::KT - 1 > row0));
       if (need_mask) {
 #pragma unroll
-        for (int sub = 0; sub < C::NSUB; ++sub)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int key = t0 + sub * 32 + key_of_reg(r, g);
-            const bool ok = key < k_end && (!p.causal || key <= my_row);
-            if (!ok) s[sub][r] = kNegInf;
-          }
+        for (int r = 0; r < 16; ++r) {
+          const int key = t0 + key_of_reg(r, g);
+          if (!(key < k_end && (!p.causal || key <= my_row))) s[r] = kNegInf;
+        }
       }
 #pragma unroll
-      for (int sub = 0; sub < C::NSUB; ++sub)
-#pragma unroll
-        for (int r = 0; r < 16; r += 2) mx = fmaxf(mx, fmaxf(s[sub][r], s[sub][r + 1]));
+      for (int r = 0; r < 16; r += 2) mx = fmaxf(mx, fmaxf(s[r], s[r + 1]));
     }
     mx = wave_max_pair(mx);
     const float m_tile = HAS_BIAS ? mx : mx * cs;
@@ -259,13 +238,10 @@ __global__ __launch_bounds__(64 * WAVES) void phase1_kernel(const Phase1Params p
     const float alpha = fast_exp2(m_run - m_use);
     float zs = 0.f;
 #pragma unroll
-    for (int sub = 0; sub < C::NSUB; ++sub)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const float pr = HAS_BIAS ? fast_exp2(s[sub][r] - m_use) : fast_exp2(fmaf(s[sub][r], cs, -m_use));
-        s[sub][r] = pr;
-        zs += pr;
-      }
+    for (int r = 0; r < 16; ++r) {
+      s[r] = HAS_BIAS ? fast_exp2(s[r] - m_use) : fast_exp2(fmaf(s[r], cs, -m_use));
+      zs += s[r];
+    }
     z_lane = fmaf(z_lane, alpha, zs);
     if (__any(alpha != 1.0f)) {
 #pragma unroll
@@ -278,29 +254,18 @@ __global__ __launch_bounds__(64 * WAVES) void phase1_kernel(const Phase1Params p
     // O^T += V^T P^T : A = V^T rows d, B = P^T straight from the S^T registers; k-step
     // 4 jb + u takes key key_of_reg(4 jb + u, g) = k0 + u.
 #pragma unroll
-    for (int sub = 0; sub < C::NSUB; ++sub)
+    for (int jb = 0; jb < 4; ++jb) {
+      const int k0 = 16 * (jb >> 1) + 8 * g + 4 * (jb & 1);  // key_of_reg(4 jb, g)
 #pragma unroll
-      for (int jb = 0; jb < 4; ++jb) {
-        const int k0 = sub * 32 + 16 * (jb >> 1) + 8 * g + 4 * (jb & 1);  // key_of_reg(4 jb, g)
+      for (int dt = 0; dt < C::NDT; ++dt) {
+        const T* vrow = vt + (dt * 32 + c) * C::VS + k0;
 #pragma unroll
-        for (int dt = 0; dt < C::NDT; ++dt) {
-          const T* vrow = vt + (dt * 32 + c) * C::VS + k0;
-#pragma unroll
-          for (int u = 0; u < 4; ++u) oacc[dt] = M::mma(vrow[u], s[sub][4 * jb + u], oacc[dt]);
-        }
-      }
-
-    if constexpr (C::NBUF == 2) {
-      if (has_next) sstore(buf ^ 1);
-      __syncthreads();
-    } else {
-      __syncthreads();
-      if (has_next) {
-        gload(t0 + C::KT);
-        sstore(0);
-        __syncthreads();
+        for (int u = 0; u < 4; ++u) oacc[dt] = M::mma(vrow[u], s[4 * jb + u], oacc[dt]);
       }
     }
+
+    if (has_next) sstore(buf ^ 1);
+    __syncthreads();
   }
 
   const float z = wave_sum_pair(z_lane);
@@ -612,7 +577,7 @@ void phase1_x3_kernel(const Phase1Params p) {
 // 2 waves per SIMD, except the 1- and 2-wave variants at D >= 64 (sequences of at most 64
 // keys): their register staging of a whole 64-key stage does not fit that budget.  The one-tile D <= 32
 // variants run as many as their registers allow (3-5): on short windows the loads' latency is the time, and
-// more of them overlap (512 windows x 3 heads, N49, fp16 bias 0.0203 -> 0.0144 ms; 3 waves, 134 VGPRs).
+// more of them overlap (512 windows x 3 heads, N49, fp16 bias 0.0203 -> 0.0144 ms; 3 waves, 153 VGPRs).
 template <typename T, int DP, int RT, int WAVES, bool HAS_BIAS, bool PRE, bool PV32 = false, bool LD = false>
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu((WAVES <= 2 && DP >= 64) ? 1 : 2, DP == 32 && RT == 1 ? 8 : 2)))
 void phase1_half_kernel(const Phase1Params p) {
@@ -1609,10 +1574,10 @@ __global__ __launch_bounds__(256) void phase2_kernel(const Phase2Params p) {
 }
 
 // ------------------------------------------------------------------ launchers
-template <typename T, int DP, int W, bool B>
+template <int DP, int W, bool B>
 static hipError_t launch1(const Phase1Params& p, hipStream_t st) {
   const dim3 grid((p.q_len + 32 * W - 1) / (32 * W), p.BH, p.P);
-  hipLaunchKernelGGL((phase1_kernel<T, DP, W, B>), grid, dim3(64 * W), 0, st, p);
+  hipLaunchKernelGGL((phase1_kernel<DP, W, B>), grid, dim3(64 * W), 0, st, p);
   return hipGetLastError();
 }
 
@@ -1826,7 +1791,7 @@ static hipError_t launch1_f32_wb(const Phase1Params& p, int block_m, hipStream_t
   const bool b = p.bias.ptr != nullptr;
   if (block_m == 64) {
     if constexpr (DP == 128) {
-      return b ? launch1<float, DP, 2, true>(p, st) : launch1<float, DP, 2, false>(p, st);
+      return b ? launch1<DP, 2, true>(p, st) : launch1<DP, 2, false>(p, st);
     } else {
       return b ? launch1x3<DP, 2, true>(p, st) : launch1x3<DP, 2, false>(p, st);
     }

@@ -147,7 +147,7 @@ hipError_t launch_row_stats(const BwdParams& p, float* row_m, float* row_z, int 
 // The whole backward of a sequence of at most 64 rows in one launch (elsa_bwd_short.hip).  ds_mode 0:
 // no dS; 1: dS of every (batch, head) to p.ds_out, [BH][N][N]; 2: dS summed over the batch, one partial
 // [H][N][N] to p.ds_out for each of bwd_short_groups ranges of it.
-bool bwd_short_takes(int dtype, int n, int dp);
+bool bwd_short_takes(int n, int dp);
 int bwd_short_groups(int dtype, int dp, int batch, int heads);
 hipError_t launch_bwd_short(const BwdParams& p, int dtype, int ds_mode, hipStream_t stream);
 // Number of ranges the dbias reduction over broadcast (b, h) pairs is cut into (1 = direct).

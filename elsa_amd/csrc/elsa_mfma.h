@@ -193,19 +193,6 @@ __device__ inline typename Mfma<T>::frag load_frag(const T* p, bool ok) {
   }
 }
 
-// Build a B-operand fragment of type T from KP consecutive fp32 registers.
-template <typename T, int R0>
-__device__ inline typename Mfma<T>::frag pack_frag(const f32x16& v) {
-  if constexpr (Mfma<T>::KP == 1) {
-    return v[R0];
-  } else {
-    typename Mfma<T>::frag f;
-#pragma unroll
-    for (int t = 0; t < 8; ++t) f[t] = static_cast<T>(v[R0 + t]);
-    return f;
-  }
-}
-
 // 16-byte raw chunk used for global->LDS staging.  A vector type, not a struct: a
 // struct copy is a memcpy, and a staging array of structs copied global -> array ->
 // LDS by memcpy is not split into registers (it ends up in LDS or scratch).
@@ -226,16 +213,6 @@ __device__ inline Chunk16 buffer_load16(__amdgpu_buffer_rsrc_t r, uint32_t voff,
 // land at lds + 16 i (lds is wave-uniform: it goes to M0); offsets past the buffer range read zeros
 __device__ inline void buffer_load16_lds(__amdgpu_buffer_rsrc_t r, void* lds, uint32_t voff) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, voff, 0, 0, 0);
-}
-
-// acc + a + b with an fp32 accumulator (v_dot2_f32_f16 / v_dot2_f32_bf16 against (1, 1)).
-__device__ inline float sum2(f16 a, f16 b, float acc) {
-  const f16x2 v = {a, b}, one = {(f16)1.0f, (f16)1.0f};
-  return __builtin_amdgcn_fdot2(v, one, acc, false);
-}
-__device__ inline float sum2(bf16 a, bf16 b, float acc) {
-  const bf16x2 v = {a, b}, one = {(bf16)1.0f, (bf16)1.0f};
-  return __builtin_amdgcn_fdot2_f32_bf16(v, one, acc, false);
 }
 
 // Unpadded LDS tiles of 64 two-byte elements per row (128 bytes) with the 16-byte chunk q of row r
