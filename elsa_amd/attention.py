@@ -11,8 +11,9 @@ exactly like the reference and otherwise ignored: the HIP kernels pick their own
 tile shapes for gfx950.  ``block_n`` is honoured as the K-partition width,
 ``q_chunk_size`` as the number of query rows per Phase1+Phase2 pass, and
 ``summary_dtype`` as the storage type of the ``s`` summaries.  ``input_precision``
-is validated; fp32 inputs always get full-fp32 products (three bf16 parts per operand
-on the bf16 matrix cores, every bit of both), at least as accurate as ``tf32x3``.
+is validated; fp32 inputs always get products of about fp32's accuracy (three bf16 parts
+per operand on the bf16 matrix cores, which hold every bit of values from 2^-110 on; a
+product within 2^-22, 2^-24 rms), more accurate than ``tf32x3``.
 """
 from __future__ import annotations
 

@@ -94,12 +94,13 @@ __device__ inline void static_for(Fn&& f) {
 }
 
 // fp32 operands on the bf16 matrix cores: x = h + m + l with h, m and l bf16 (8 + 8 + 8 significant
-// bits), and a product of two such sums as the six partial products of order 2^-16 and above,
+// bits: every bit of values from 2^-110 on; below, l is a subnormal and x off by up to 2^-134), and a product of
+// two such sums as the six partial products of order 2^-16 and above,
 //   x y ~ h h' + (h m' + m h') + (m m' + h l' + l h'),
-// each exact in the MFMA and summed in fp32.  The dropped ones (m l', l m', l l') are below 2^-23 of
-// |x y| (2^-26 on average, of either sign): less than one fp32 rounding.  Six v_mfma_f32_32x32x16_bf16
-// (8 passes each) take 48 passes where the eight v_mfma_f32_32x32x2_f32 (16 passes each) of the same
-// 16-long contraction take 128.
+// each exact in the MFMA and summed in fp32.  The dropped ones (m l', l m', l l') come to at most 2^-22 of |x y|
+// (|m| < 2^-7 and |l| <= 2^-16 of |x| where h is truncated), 2^-24 rms and of either sign.  Six
+// v_mfma_f32_32x32x16_bf16 (8 passes each) take 48 passes where the eight v_mfma_f32_32x32x2_f32 (16 passes each)
+// of the same 16-long contraction take 128.
 struct Split3 {
   bf16x8 h, m, l;
 };

@@ -32,6 +32,16 @@ def test_three_parts_hold_every_bit(truncate_h):
     assert np.array_equal(h.astype(np.float64) + m + l, x.astype(np.float64))
 
 
+@pytest.mark.parametrize("truncate_h", [True, False])
+def test_parts_of_small_values_end_at_bf16s_smallest_subnormal(truncate_h):
+    rng = np.random.default_rng(9)
+    x = (rng.standard_normal(100_000) * 2.0 ** rng.integers(-126, -90, 100_000)).astype(np.float32)
+    h, m, l = _split(x, truncate_h)
+    err = np.abs(h.astype(np.float64) + m + l - x)
+    assert err.max() <= 2.0 ** -134
+    assert err[np.abs(x) >= 2.0 ** -110].max() == 0 and err.max() > 0
+
+
 def test_infinities_stay_in_the_last_part_and_the_largest_values_finite():
     x = np.array([np.inf, -np.inf, np.finfo(np.float32).max, -np.finfo(np.float32).max, 0.0], np.float32)
     h, m, l = _split(x, True)
