@@ -8,10 +8,10 @@
 // The stage tiles are loaded through registers one stage ahead and split by the threads that load them.
 // Bound: the matrix cores (72 and 96 MFMAs of 8 passes per 32 x 32 score tile at d64; 96 and 128 of 16
 // passes on the fp32 MFMA before).  Whole backward ms, fp32 MFMA kernels -> these (B1 H8 d64 unless noted;
-// largest relative gradient error against 64 bits): 16K 16.36 -> 9.06 (2.3e-6 -> 5.6e-7), 4K 1.065 -> 0.604
-// (9.2e-7 -> 3.5e-7), 1K 0.102 -> 0.076, B8 H3 N1025 0.306 -> 0.169, B8 H3 N197 0.055 -> 0.040, causal 4K 1.068 ->
-// 0.458 and N1025 0.133 -> 0.070 (their stages dealt out in turn, in causal_bwd_order), B1 H16 2K d32 0.320
-// -> 0.194, 4K d128 2.245 -> 1.347.  The 4K backward executes 1.0 PFLOP/s of MFMA work.
+// largest relative gradient error against 64 bits): 16K 16.30 -> 9.08 (2.3e-6 -> 5.6e-7), 4K 1.065 -> 0.606
+// (9.2e-7 -> 3.5e-7), 1K 0.102 -> 0.077, B8 H3 N1025 0.307 -> 0.169, B8 H3 N197 0.054 -> 0.040, causal 4K 1.068 ->
+// 0.452 and N1025 0.133 -> 0.071 (their stages dealt out in turn, in causal_bwd_order), B1 H16 2K d32 0.318
+// -> 0.194, 4K d128 2.237 -> 1.360.  The 4K backward executes 1.0 PFLOP/s of MFMA work.
 // A pass that wrote the parts of q, k, v and dO to memory first, so that the kernels could load stages
 // straight into LDS, took 0.618 at 4K and needs 24 B per element of workspace.
 #include <algorithm>

@@ -298,9 +298,9 @@ constexpr float kLazySum = 256.0f;  // 2^kLazyTau
 // of a running sum per output element instead of N/2.
 // Bound: the matrix cores.  48 MFMAs of 8 passes per 32 x 32 score tile (d64) against the 64 of 16
 // passes of the fp32 MFMA fold (phase1_kernel).  Forward ms, phase1_kernel -> this (relative error
-// against 64 bits): B1 H8 d64 16K 4.60 -> 2.64 (1.65e-6 -> 3.8e-7; 1.25 PFLOP/s of MFMA work, above the
-// 1.14 a large bf16 library product reaches), 8K 1.175 -> 0.673 (1.2e-6 -> 2.9e-7), 1K 0.0356 -> 0.0250,
-// B8 H3 N197 0.0149 -> 0.0135, d128 4K 0.670 -> 0.343 (7.1e-7 -> 2.3e-7), causal 4K 0.196 -> 0.115.
+// against 64 bits): B1 H8 d64 16K 4.57 -> 2.80 (1.65e-6 -> 3.8e-7; 1.18 PFLOP/s of MFMA work, above the
+// 1.14 a large bf16 library product reaches), 8K 1.168 -> 0.714 (1.2e-6 -> 2.9e-7), 1K 0.0352 -> 0.0294,
+// B8 H3 N197 0.0140 -> 0.0126, d128 4K 0.661 -> 0.349 (7.1e-7 -> 2.3e-7), causal 4K 0.193 -> 0.118.
 template <int DP>
 struct X3Tile {
   static constexpr bool SWZ = DP == 64;
